@@ -26,7 +26,15 @@ namespace lee {
 namespace {
 
 constexpr int A3_TY = 4;
-constexpr int A3_ZC = 32;
+constexpr int A3_ZC = 32;      // planes per chunk of the zeta^T filter pass
+// Planes per workgroup of the adjoint stage (see STAGE_Z_CHUNK of the
+// forward stage; here a chunk's four extra planes cost a flux evaluation
+// each, so 4 planes instead of 2).  Whole reverse step (recomputed forward
+// step, adjoint step), FP32 / FP64: 48 x 40 x 32 2377 / 2832 us with 32
+// planes, 445 / 519 with 4, 308 / 354 with 2, 249 / 292 with 1;
+// 144 x 120 x 112 3856 / 5033, 2043 / 3644, 2045 / 3691, 2249 / 3907;
+// 256 x 200 x 256 11289 / 20657, 9915 / 18102, 10315 / 18939, 11055 / 20816.
+constexpr int ADJ_Z_CHUNK = 4;
 
 inline unsigned nba(size_t n) { return (unsigned)((n + TPB - 1) / TPB); }
 
@@ -120,7 +128,7 @@ struct Zone3A {
 
 template <typename T>
 struct Adj3Args {
-  int ni, nj, nk, ntx, nty, nzc;
+  int ni, nj, nk, ntx, nty, nzc, zc;
   const T *lacc, *lin, *lyin;
   T *lout, *lyout, *mu;
   double *grad;
@@ -185,7 +193,7 @@ __global__ void __launch_bounds__(TPB) k_adj_stage3d(Adj3Args<T> a) {
   if (tile >= ntl) return;
   const int tx = threadIdx.x, ty = threadIdx.y;
   const int i0 = (tile % a.ntx) * ST_TX, j0 = (tile / a.ntx) * A3_TY;
-  const int k0 = blockIdx.y * A3_ZC, k1 = min(k0 + A3_ZC, a.nk);
+  const int k0 = blockIdx.y * a.zc, k1 = min(k0 + a.zc, a.nk);
   const int ni = a.ni, nj = a.nj, nk = a.nk;
   const size_t plane = (size_t)ni * nj, n = plane * nk;
   const int gi = i0 + tx, gj = j0 + ty;
@@ -478,7 +486,8 @@ static hipError_t adj_stage3d_t(hipStream_t s, lee_handle *h, Block &b, const Ad
   a.nk = b.nk;
   a.ntx = (b.ni + ST_TX - 1) / ST_TX;
   a.nty = (b.nj + A3_TY - 1) / A3_TY;
-  a.nzc = (b.nk + A3_ZC - 1) / A3_ZC;
+  a.zc = z_chunk((a.ntx * a.nty + 7) / 8 * 8, b.nk, ADJ_Z_CHUNK, b.cus);
+  a.nzc = (b.nk + a.zc - 1) / a.zc;
   T *const *L = sizeof(T) == 8 ? (T *const *)b.A64 : (T *const *)b.A32;
   auto buf = [&](int k) -> T * { return k < 0 ? nullptr : L[k]; };
   a.lacc = buf(st.lacc);

@@ -163,6 +163,16 @@ struct StageArgs {
 // rows of vertically adjacent tiles in its own L2.
 __device__ __forceinline__ int xcd_tile(int bid, int chunk) { return (bid & 7) * chunk + (bid >> 3); }
 
+// Planes per workgroup of a 3-D kernel whose workgroups march `tiles` (i, j)
+// tiles through chunks of z: the most (at most `most`) that still gives two
+// workgroups per CU, since fewer leave the chip waiting on the chain of one
+// workgroup's planes; 1 when no chunk does.
+inline int z_chunk(int tiles, int nk, int most, int cus) {
+  for (int zc = most; zc > 1; zc--)
+    if ((long long)tiles * ((nk + zc - 1) / zc) >= 2LL * cus) return zc;
+  return 1;
+}
+
 // One RK stage on a 64 x TY tile.  Every global operand of the thread (its
 // share of the LDS tile, the FP64 metrics and Jacobian, the accumulator and
 // y_n of its R points) is requested up front, so a launch that is a single

@@ -8,8 +8,8 @@
 // and are checked against the 2-D path on z-invariant problems and by axis
 // permutations.
 //
-// Stage kernel: a 64 x 4 tile of (i, j) columns marches through a chunk of
-// z planes.  Each plane's tile plus its 2-point (i, j) halo is staged in
+// Stage kernel: a 64 x 4 tile of (i, j) columns marches through a short
+// chunk of z planes (z_chunk).  Each plane's tile plus its 2-point (i, j) halo is staged in
 // LDS for the xi and eta derivatives; the zeta derivative comes from a
 // 5-plane register window of the thread's own column.  Filter: one pass of
 // the 2-D xi-eta tile filter per plane, then a column pass in zeta with
@@ -30,6 +30,14 @@ constexpr int S3_TY = 4;      // tile rows in j
 #define LEE_Z_CHUNK 32
 #endif
 constexpr int Z_CHUNK = LEE_Z_CHUNK;  // planes per z chunk
+// Planes per workgroup of the stage.  A workgroup's planes are one serial
+// chain (loads, barrier, arithmetic, stores: about 5 us a plane), and the
+// four window planes that the next chunk reads again are in its XCD's L2,
+// so short chunks win at every size, FP32 / FP64 middle stage: 48 x 40 x 32
+// 176 / 229 us with 32 planes, 25 / 33 with 4, 15 / 19 with 2, 10 / 14 with
+// 1; 144 x 120 x 112 218 / 376, 131 / 258, 128 / 247, 131 / 259;
+// 256 x 200 x 256 857 / 1599, 723 / 1338, 717 / 1329, 728 / 1386.
+constexpr int STAGE_Z_CHUNK = 2;
 constexpr int FUSED_Z_CHUNK = 64;     // planes per chunk of the single-pass filter (4 halo planes a side)
 
 inline unsigned nb3(size_t n) { return (unsigned)((n + TPB - 1) / TPB); }
@@ -102,7 +110,7 @@ struct Zone3 {
 
 template <typename T>
 struct Stage3Args {
-  int ni, nj, nk, ntx, nty, nzc;
+  int ni, nj, nk, ntx, nty, nzc, zc;
   const T *yin, *yn;
   T *acc, *yout;
   const double *met, *jac;
@@ -118,7 +126,7 @@ struct Stage3Args {
   T h, b, a;
 };
 
-// One RK stage on a 64 x 4 column tile through a chunk of Z_CHUNK planes.
+// One RK stage on a 64 x 4 column tile through a chunk of zc planes.
 template <typename T, bool MEANF, int KIND>
 __global__ void __launch_bounds__(TPB) k_stage3d(Stage3Args<T> a) {
   constexpr int RS = ST_TX + 2 * ST_H, NR = S3_TY + 2 * ST_H;
@@ -131,7 +139,7 @@ __global__ void __launch_bounds__(TPB) k_stage3d(Stage3Args<T> a) {
   if (tile >= ntl) return;
   const int tx = threadIdx.x, ty = threadIdx.y;
   const int i0 = (tile % a.ntx) * ST_TX, j0 = (tile / a.ntx) * S3_TY;
-  const int k0 = blockIdx.y * Z_CHUNK, k1 = min(k0 + Z_CHUNK, a.nk);
+  const int k0 = blockIdx.y * a.zc, k1 = min(k0 + a.zc, a.nk);
   const int ni = a.ni, nj = a.nj, nk = a.nk;
   const size_t plane = (size_t)ni * nj, n = plane * nk;
   const int gi = i0 + tx, gj = j0 + ty;
@@ -631,7 +639,8 @@ static hipError_t stage3d_t(hipStream_t s, lee_handle *h, Block &b, int stage, c
   a.nk = b.nk;
   a.ntx = (b.ni + ST_TX - 1) / ST_TX;
   a.nty = (b.nj + S3_TY - 1) / S3_TY;
-  a.nzc = (b.nk + Z_CHUNK - 1) / Z_CHUNK;
+  a.zc = z_chunk((a.ntx * a.nty + 7) / 8 * 8, b.nk, STAGE_Z_CHUNK, b.cus);
+  a.nzc = (b.nk + a.zc - 1) / a.zc;
   const int in_idx = stage == 0 ? 0 : (stage % 2 == 1 ? 2 : 3);
   const int out_idx = stage % 2 == 0 ? 2 : 3;
   a.yin = Y[in_idx];

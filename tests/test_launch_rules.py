@@ -1,0 +1,59 @@
+"""Kernel forms that the launch rules pick by size, at the edges of the
+rules: against plain formulas, the CPU oracle, or the form they replace."""
+import numpy as np
+import pytest
+
+from camille_amd import FP32, FP64, Solver
+
+pytestmark = pytest.mark.gpu
+
+GAMMA = 1.4
+
+
+def _rel(a, b):
+    return float(np.max(np.abs(a - b)) / max(np.max(np.abs(b)), 1e-300))
+
+
+def _box3(ni, nj, nk, seed):
+    """A stretched 3-D box with a sheared, non-constant base flow and a rough state."""
+    rng = np.random.default_rng(seed)
+    k, j, i = np.meshgrid(np.arange(nk), np.arange(nj), np.arange(ni), indexing="ij")
+    x, y, z = (0.25 * a + 0.05 * np.sin(0.3 * a) for a in (i, j, k))
+    mean = np.zeros((5, nk, nj, ni))
+    mean[0] = 0.1 * np.sin(0.2 * x)
+    mean[1] = 0.3 * np.tanh(0.4 * (y - y.mean()))
+    mean[2] = 0.1 * np.cos(0.3 * z)
+    mean[3] = 0.05 * np.sin(0.25 * x + 0.2 * y)
+    mean[4] = (1.0 + 0.1 * np.cos(0.2 * z + 0.1 * x)) / GAMMA
+    return x, y, z, mean, rng.standard_normal((5, nk, nj, ni)), rng.standard_normal((5, nk, nj, ni))
+
+
+# (131, 61, 45) takes chunks of 2 planes forwards and 4 backwards, one plane
+# left over; (70, 13, 9) and (9, 9, 14) take single planes
+@pytest.mark.parametrize("dims", [(131, 61, 45), (70, 13, 9), (9, 9, 14)])
+@pytest.mark.parametrize("prec,tol", [(FP64, 1e-12), (FP32, 2e-5)])
+def test_3d_stage_chunks(dims, prec, tol):
+    """The 3-D right-hand side equals its definition, built from the FP64
+    derivative entry point, and its transpose satisfies <L y, k> = <y, L^T k>.
+    FP32: some 40 terms of size 1 to 10, each rounded at 6e-8, relative to
+    the largest value; the dot products gather random signs and stay below."""
+    x, y, z, mean, q, kap = _box3(*dims, seed=3)
+    s = Solver([dict(x=x, y=y, z=z, mean=mean)], precision=prec, mode="FIX_DT", value=0.01, num_dim=3)
+    d = [[s.take_derivative_xyz(f, i) for i in range(3)] for f in q]
+    g = [[s.take_derivative_xyz(f, i) for i in range(3)] for f in mean]
+    rhob = (GAMMA * mean[4]) ** (1 / GAMMA) * np.exp(-mean[0])
+    rho = rhob * (q[4] / (GAMMA * mean[4]) - q[0])
+    ub, up = mean[1:4], q[1:4]
+    ref = np.zeros_like(q)
+    for i in range(3):
+        ref[0] -= ub[i] * d[0][i] + up[i] * g[0][i]
+        ref[4] -= ub[i] * d[4][i] + up[i] * g[4][i] + GAMMA * (mean[4] * d[1 + i][i] + q[4] * g[1 + i][i])
+        for v in range(3):
+            ref[1 + v] -= ub[i] * d[1 + v][i] + (up[i] + rho / rhob * ub[i]) * g[1 + v][i]
+        ref[1 + i] -= d[4][i] / rhob
+    r = s.compute_rhs(q, 0.0)
+    assert max(_rel(r[v], ref[v]) for v in range(5)) <= tol
+    lk = s.compute_rhs_adjoint(kap)
+    a, b = float(np.sum(r * kap)), float(np.sum(q * lk))
+    assert abs(a - b) <= tol * np.linalg.norm(r) * np.linalg.norm(kap)
+    s.close()
