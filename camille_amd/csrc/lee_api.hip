@@ -72,8 +72,6 @@ void free_block(Block &b) {
   }
   dfree(b.dflux);
   dfree(b.dsum);
-  dfree(b.func0);
-  dfree(b.func);
   for (auto &z : b.zones) {
     dfree(z.sigma64);
     dfree(z.sigma32);
@@ -185,47 +183,36 @@ int enqueue_fused_step(lee_handle *h) {
   return LEE_OK;
 }
 
-// temporal::time_advance with one kernel per reference operator (FP64).
+// temporal::time_advance in the reference's arithmetic (FP64).
 int enqueue_plain_step(lee_handle *h) {
   const int S = h->cfg.rk_stages, last = S - 1;
   const double tn = h->time_sol, dt = h->dt;
   hipStream_t s = h->stream;
-  for (int ib = 0; ib < h->nblk; ib++) {
-    Block &b = h->b[ib];
-    const size_t bytes = sizeof(double) * nvars(h) * (size_t)b.n;
-    HIPCHK(hipMemcpyAsync(b.Y64[1], b.Y64[0], bytes, hipMemcpyDeviceToDevice, s));  // ynp1 = yn
-    HIPCHK(hipMemcpyAsync(b.Y64[2], b.Y64[0], bytes, hipMemcpyDeviceToDevice, s));  // interim = yn
-  }
   const bool harm = h->cfg.harmonic_wave == LEE_WAVE_ENTROPY;
   for (int st = 0; st < S; st++) {
-    double s1, s2;
-    source_factors(h->cfg, tn + h->c_i[st] * dt, s1, s2);
-    const double he = harm ? harmonic_entropy(h->cfg, tn + h->c_i[st] * dt) : 0.0;
+    StageScalars sc{dt, h->b_i[st], h->a_next[st], 0.0, 0.0};
+    source_factors(h->cfg, tn + h->c_i[st] * dt, sc.s1, sc.s2);
+    if (harm) sc.he = harmonic_entropy(h->cfg, tn + h->c_i[st] * dt);
     const double he_bc = harm ? harmonic_entropy(h->cfg, tn + h->c_i[std::min(st + 1, last)] * dt) : 0.0;
     for (int ib = 0; ib < h->nblk; ib++) {
       Block &b = h->b[ib];
-      HIPCHK(plain_rhs(s, h, b, b.Y64[2], b.Y64[3], s1, s2, b.rho64, he));
+      HIPCHK(plain_stage(s, h, b, st, sc, st == 0 ? b.rho64 : nullptr));
     }
-    for (int ib = 0; ib < h->nblk; ib++) {
-      Block &b = h->b[ib];
-      HIPCHK(plain_rk_update(s, b, b.Y64[3], b.Y64[1], b.Y64[2], b.Y64[0], dt, h->b_i[st], h->a_next[st],
-                             st == last, nvars(h)));
-    }
-    const int tgt = st < last ? 2 : 1;
+    const int tgt = fused_target(h, st);
     for (int ib = 0; ib < h->nblk; ib++) {
       Block &b = h->b[ib];
       if (!b.faces.empty()) HIPCHK(apply_bcs(s, h, b, b.Y64[tgt], nullptr, false, nullptr, nullptr, he_bc));
     }
     HIPCHK(overset_interpolate(s, h, false, tgt, false));
-    for (int ib = 0; ib < h->nblk; ib++) {
-      Block &b = h->b[ib];
-      HIPCHK(aux_density(s, b, h->cfg.gamma, b.Y64[tgt], b.rho64));
-    }
   }
   for (int ib = 0; ib < h->nblk; ib++) {
     Block &b = h->b[ib];
-    if (h->cfg.filter_order > 0) HIPCHK(plain_filter(s, h, b, b.Y64[1]));
-    HIPCHK(plain_iblank_reset(s, b, b.Y64[1], nvars(h)));
+    if (h->cfg.filter_order > 0) {
+      HIPCHK(plain_filter(s, h, b, b.Y64[1], b.Y64[3], b.rho64, true));
+    } else {
+      HIPCHK(aux_density(s, b, h->cfg.gamma, b.Y64[1], b.rho64));
+      HIPCHK(plain_iblank_reset(s, b, b.Y64[1], nvars(h)));
+    }
     std::swap(b.Y64[0], b.Y64[1]);
   }
   return LEE_OK;
@@ -1118,10 +1105,6 @@ int create_impl(const lee_config *cfgs, int cfg_stride, const lee_block *blocks,
         HIPCHK(dalloc(&b.rho32, (size_t)n));
         for (int k = 0; k < 4; k++) HIPCHK(dalloc(&b.Y32[k], nv * (size_t)n));
       }
-      if (is_plain(h)) {
-        HIPCHK(dalloc(&b.func0, (size_t)n));
-        HIPCHK(dalloc(&b.func, (size_t)n));
-      }
       for (int k = 0; k < 4; k++) HIPCHK(hipMemsetAsync(b.Y64[k], 0, sizeof(double) * nv * n, s));
       if (is_fp32(h))
         for (int k = 0; k < 4; k++) HIPCHK(hipMemsetAsync(b.Y32[k], 0, sizeof(float) * nv * n, s));
@@ -1671,7 +1654,7 @@ int lee_compute_rhs(lee_handle *h, int ib, const double *y, double time, double 
   const double he = h->cfg.harmonic_wave == LEE_WAVE_ENTROPY ? harmonic_entropy(h->cfg, time) : 0.0;
   HIPCHK(hipMemcpy(b.Y64[2], y, sizeof(double) * cnt, hipMemcpyHostToDevice));
   if (is_plain(h)) {
-    HIPCHK(plain_rhs(s, h, b, b.Y64[2], b.Y64[3], s1, s2, b.dsum, he));
+    HIPCHK(plain_stage(s, h, b, -1, StageScalars{1.0, 1.0, 0.0, s1, s2, he}, nullptr));
     HIPCHK(hipMemcpyAsync(rhs, b.Y64[3], sizeof(double) * cnt, hipMemcpyDeviceToHost, s));
   } else {
     StageScalars sc{1.0, 1.0, 0.0, s1, s2, he};
@@ -1699,7 +1682,7 @@ int lee_apply_filter(lee_handle *h, int ib, double *y) {
   hipStream_t s = h->stream;
   HIPCHK(hipMemcpy(b.Y64[1], y, sizeof(double) * cnt, hipMemcpyHostToDevice));
   if (is_plain(h)) {
-    HIPCHK(plain_filter(s, h, b, b.Y64[1]));
+    HIPCHK(plain_filter(s, h, b, b.Y64[1], b.Y64[3], nullptr, false));
     HIPCHK(hipMemcpyAsync(y, b.Y64[1], sizeof(double) * cnt, hipMemcpyDeviceToHost, s));
   } else if (is_fp32(h)) {
     HIPCHK(cast_state(s, b, nv, b.Y64[1], b.Y32[1], cnt));

@@ -108,9 +108,7 @@ struct Block {
   int tune_mc = 0, tune_ml = 0;  // filter column-march form (no holes): waves per stack, rows per wave; 0 off
   int cus = 0;                 // compute units of the device
   bool tuned = false;
-  // plain-path scratch (FP64): dflux, sum, rhs (5n), func0, func, interim (5n), ynp1 (5n)
-  double *dflux = nullptr, *dsum = nullptr, *rhs = nullptr, *func0 = nullptr, *func = nullptr;
-  double *interim = nullptr, *ynp1 = nullptr, *sol = nullptr;
+  double *dflux = nullptr, *dsum = nullptr;  // scratch of the derivative entry points (n each, FP64)
   // boundaries
   std::vector<SpongeZone> zones;
   std::vector<BcFace> faces;
@@ -286,7 +284,7 @@ void plan_source(const lee_config &c, Block &b, const double *xyz_host);
 // time factors (s1, s2) of the source at time t: term = (s1 * g) * s2
 void source_factors(const lee_config &c, double t, double &s1, double &s2);
 
-// ---- kernels (lee_kernels.hip) ----
+// ---- kernels (lee_kernels.hip, lee_plain.hip) ----
 struct StageScalars {
   double h;        // dt
   double b;        // b_i
@@ -294,15 +292,17 @@ struct StageScalars {
   double s1, s2;   // source time factors
   double he = 0.0; // harmonic-wave entropy factor e(t) at the stage time
 };
-hipError_t plain_apply_op(hipStream_t s, const Block &b, const OpTable &op, const int8_t *codes,
-                          const double *f, double *df, int dir);
 hipError_t plain_take_derivative_xyz(hipStream_t s, const Block &b, const OpTable &op, const double *f,
                                      int dir_xyz);
-hipError_t plain_rhs(hipStream_t s, lee_handle *h, const Block &b, const double *y, double *rhs, double s1,
-                     double s2, double *rho, double he = 0.0);
-hipError_t plain_rk_update(hipStream_t s, const Block &b, double *rhs, double *ynext, double *interim,
-                           const double *ycur, double hdt, double bi, double a, bool last, int nv);
-hipError_t plain_filter(hipStream_t s, lee_handle *h, const Block &b, double *y);
+// One plain RK stage, buffers as the fused stages' (stage < 0: the right-hand
+// side of Y64[2] into Y64[3]); rho: the carried aux density, null for that of
+// the stage input.
+hipError_t plain_stage(hipStream_t s, lee_handle *h, const Block &b, int stage, const StageScalars &sc,
+                       const double *rho);
+// In place on y (nv n values) through tmp; rho: where the aux density of the
+// unfiltered y goes (null: not wanted).
+hipError_t plain_filter(hipStream_t s, lee_handle *h, const Block &b, double *y, double *tmp, double *rho,
+                        bool reset_holes);
 hipError_t plain_iblank_reset(hipStream_t s, const Block &b, double *y, int nv);
 hipError_t aux_density(hipStream_t s, const Block &b, double gamma, const double *y, double *rho);
 // HARMONIC_WAVE entropy factor e(t) = A (1 + sin(k c0 t)), k = 2 pi / wavelength

@@ -1,16 +1,12 @@
 // HIP kernels of the LEE time advance for gfx950 (CDNA4).
 //
-// Two families:
-//  * plain_*  -- one kernel per reference operator (take_derivative_xyz, each
-//    RHS term, sponge, source, RK update, filter sweep, blend, aux), FP64 with
-//    floating-point contraction off and the reference's operation order, so
-//    the GPU result equals the CPU reference bit for bit.  This is the
-//    drop-in FP64 path and the yardstick for the fused path.
-//  * fused_*  -- one LDS-tiled kernel per RK stage (both directional
-//    derivatives of the four active variables, chain rule with FP64 metrics,
-//    LEE right-hand side, source, sponge, RK update, aux density) and one
-//    LDS-tiled kernel per step for the two filter sweeps + blend + hole
-//    reset.  Templated on the bulk type (double or float).
+// Fused path: one LDS-tiled kernel per RK stage (both directional
+// derivatives of the four active variables, chain rule with FP64 metrics,
+// LEE right-hand side, source, sponge, RK update, aux density) and one
+// kernel per step for the two filter sweeps + blend + hole reset, templated
+// on the bulk type (double or float); batched ensembles of them; and the
+// boundary conditions and overset interpolation that both paths share.  The
+// plain path is in lee_plain.hip.
 //
 // All global indices are bounds-checked against the block extents.
 #include <hip/hip_runtime.h>
@@ -23,233 +19,6 @@
 namespace lee {
 
 namespace {
-
-// ------------------------------------------------------------------ plain
-
-// One row of the reference operator at point p (coordinate c along a line of
-// length len, memory stride st), every coefficient included, left to right.
-__device__ double plain_row(const OpTable &op, const double *f, int p, int c, int len, int st, int code) {
-#pragma clang fp contract(off)
-  double acc = 0.0;
-  if (code == CODE_INTERIOR) {
-    for (int s = -op.half; s <= op.half; s++) {
-      const int q = c + s;
-      if (q >= 0 && q < len) acc += op.st[s + op.half] * f[p + s * st];
-    }
-  } else if (code == CODE_ZERO) {
-    acc = 0.0;
-  } else if (code < CODE_LEFT + op.nb) {
-    const int k = code - CODE_LEFT;
-    for (int s = 0; s < op.sb; s++) {
-      const int q = c - k + s;
-      if (q >= 0 && q < len) acc += op.bnd[k][s] * f[p + (s - k) * st];
-    }
-  } else {
-    const int k = code - CODE_LEFT - op.nb;
-    for (int s = 0; s < op.sb; s++) {
-      const int q = c + k - s;
-      if (q >= 0 && q < len) acc += op.sign_right * op.bnd[k][s] * f[p + (k - s) * st];
-    }
-  }
-  return acc;
-}
-
-__global__ void __launch_bounds__(TPB) k_plain_op_dir(const double *__restrict__ f, double *__restrict__ df,
-                                                      const int8_t *__restrict__ codes, int ni, int nj, int dir,
-                                                      OpTable op) {
-  const int p = blockIdx.x * TPB + threadIdx.x;
-  const int n = ni * nj;
-  if (p >= n) return;
-  const int i = p % ni, j = p / ni;
-  const int c = dir == 0 ? i : j, len = dir == 0 ? ni : nj, st = dir == 0 ? 1 : ni;
-  const int code = codes ? (int)codes[p] : default_code(c, len, op.nb);
-  df[p] = plain_row(op, f, p, c, len, st, code);
-}
-
-// StandardCentral::take_derivative_xyz (spatial:1802-1826):
-// out = (0 + m[xi][d] d/dxi + m[eta][d] d/deta) * J
-__global__ void __launch_bounds__(TPB) k_plain_deriv_xyz(const double *__restrict__ f, double *__restrict__ out,
-                                                         const double *__restrict__ met,
-                                                         const double *__restrict__ jac,
-                                                         const int8_t *__restrict__ codes, int ni, int nj, int dxyz,
-                                                         OpTable op) {
-#pragma clang fp contract(off)
-  const int p = blockIdx.x * TPB + threadIdx.x;
-  const int n = ni * nj;
-  if (p >= n) return;
-  const int i = p % ni, j = p / ni;
-  const int c0 = codes ? (int)codes[p] : default_code(i, ni, op.nb);
-  const int c1 = codes ? (int)codes[n + p] : default_code(j, nj, op.nb);
-  const double d0 = plain_row(op, f, p, i, ni, 1, c0);
-  const double d1 = plain_row(op, f, p, j, nj, ni, c1);
-  double sum = 0.0;
-  sum += met[(size_t)(0 + dxyz) * n + p] * d0;
-  sum += met[(size_t)(2 + dxyz) * n + p] * d1;
-  out[p] = sum * jac[p];
-}
-
-// metrics::compute_ThomasLombard_2D + compute_Jacobian (metrics.cpp:107-129,
-// 255-328).  xx = {x_xi, x_eta, y_xi, y_eta}.
-__global__ void __launch_bounds__(TPB) k_metrics2d(const double *__restrict__ xx, double *__restrict__ met,
-                                                   double *__restrict__ jac, int n) {
-#pragma clang fp contract(off)
-  const int p = blockIdx.x * TPB + threadIdx.x;
-  if (p >= n) return;
-  const double x_xi = xx[p], x_eta = xx[(size_t)n + p], y_xi = xx[(size_t)2 * n + p], y_eta = xx[(size_t)3 * n + p];
-  met[p] = y_eta;
-  met[(size_t)n + p] = -x_eta;
-  met[(size_t)2 * n + p] = -y_xi;
-  met[(size_t)3 * n + p] = x_xi;
-  const double inv = x_xi * y_eta - x_eta * y_xi;
-  jac[p] = 1.0 / inv;
-}
-
-__global__ void __launch_bounds__(TPB) k_fill(double *__restrict__ a, double v, size_t n) {
-  const size_t p = (size_t)blockIdx.x * TPB + threadIdx.x;
-  if (p < n) a[p] = v;
-}
-
-__global__ void __launch_bounds__(TPB) k_copy(const double *__restrict__ a, double *__restrict__ b, size_t n) {
-  const size_t p = (size_t)blockIdx.x * TPB + threadIdx.x;
-  if (p < n) b[p] = a[p];
-}
-
-// rhs -= a * b
-__global__ void __launch_bounds__(TPB) k_sub_ab(double *__restrict__ r, const double *__restrict__ a,
-                                                const double *__restrict__ b, int n) {
-#pragma clang fp contract(off)
-  const int p = blockIdx.x * TPB + threadIdx.x;
-  if (p < n) r[p] -= a[p] * b[p];
-}
-
-// rhs -= (g * a) * b
-__global__ void __launch_bounds__(TPB) k_sub_gab(double *__restrict__ r, double g, const double *__restrict__ a,
-                                                 const double *__restrict__ b, int n) {
-#pragma clang fp contract(off)
-  const int p = blockIdx.x * TPB + threadIdx.x;
-  if (p < n) r[p] -= g * a[p] * b[p];
-}
-
-// rhs -= a / b
-__global__ void __launch_bounds__(TPB) k_sub_div(double *__restrict__ r, const double *__restrict__ a,
-                                                 const double *__restrict__ b, int n) {
-#pragma clang fp contract(off)
-  const int p = blockIdx.x * TPB + threadIdx.x;
-  if (p < n) r[p] -= a[p] / b[p];
-}
-
-// rhs -= (u' + rho'/rho_bar * u_bar) * grad   (spatial:2089-2092)
-__global__ void __launch_bounds__(TPB) k_sub_velgrad(double *__restrict__ r, const double *__restrict__ up,
-                                                     const double *__restrict__ rho,
-                                                     const double *__restrict__ rhob,
-                                                     const double *__restrict__ ub,
-                                                     const double *__restrict__ grad, int n) {
-#pragma clang fp contract(off)
-  const int p = blockIdx.x * TPB + threadIdx.x;
-  if (p < n) r[p] -= (up[p] + rho[p] / rhob[p] * ub[p]) * grad[p];
-}
-
-// apply_physicalSource: rhs[P] += (s1 * g) * s2 over the source support
-// compute_RHS_linearized_Euler's axisymmetric term (spatial:2119-2126):
-// rhs_p -= gamma (pbar u_r' + p' ubar_r) / (r + 1e-99), with u_r = u_y and
-// r = y (the axis of symmetry is x, input.cpp:523-531).
-__global__ void __launch_bounds__(TPB) k_plain_axisym(double *__restrict__ rp, double gam,
-                                                      const double *__restrict__ pb, const double *__restrict__ ur,
-                                                      const double *__restrict__ pp, const double *__restrict__ urb,
-                                                      const double *__restrict__ r, int n) {
-#pragma clang fp contract(off)
-  const int q = blockIdx.x * TPB + threadIdx.x;
-  if (q >= n) return;
-  const double DUMMY_SMALL = 1e-99;
-  rp[q] -= gam * (pb[q] * ur[q] + pp[q] * urb[q]) / (r[q] + DUMMY_SMALL);
-}
-
-__global__ void __launch_bounds__(TPB) k_plain_source(double *__restrict__ rp, const double *__restrict__ g,
-                                                      int ni, int i0, int i1, int j0, int j1, double s1,
-                                                      double s2) {
-#pragma clang fp contract(off)
-  const int bw = i1 - i0 + 1, bh = j1 - j0 + 1;
-  const int q = blockIdx.x * TPB + threadIdx.x;
-  if (q >= bw * bh) return;
-  const int i = i0 + q % bw, j = j0 + q / bw;
-  rp[(size_t)j * ni + i] += s1 * g[q] * s2;
-}
-
-// apply_bufferZone_Freund_ambient (source.cpp:174-201), one zone, all nv
-// vars (the passive scalars too); a harmonic zone
-// (apply_bufferZone_Freund_harmonicWave, source.cpp:264-320) relaxes s' to
-// the entropy wave he * hg (hg null: he) and the other variables to 0, the
-// data of bc_dirichlet_harmonicwave for LEE.
-__global__ void __launch_bounds__(TPB) k_plain_sponge(double *__restrict__ rhs, const double *__restrict__ y,
-                                                      const double *__restrict__ sig, int ni, int n, int i0,
-                                                      int nzi, int j0, int nzj, int harm, double he,
-                                                      const double *__restrict__ hg, int nv) {
-#pragma clang fp contract(off)
-  const int q = blockIdx.x * TPB + threadIdx.x;
-  if (q >= nzi * nzj) return;
-  const int p = (j0 + q / nzi) * ni + (i0 + q % nzi);
-  const double s = sig[q];
-  for (int v = 0; v < nv; v++) {
-    const double target = harm && v == IS ? (hg ? he * hg[q] : he) : 0.0;
-    const double relax = -s * (y[(size_t)v * n + p] - target);
-    rhs[(size_t)v * n + p] += relax;
-  }
-}
-
-// RungeKutta::integrate update loop (temporal:208-230)
-__global__ void __launch_bounds__(TPB) k_plain_rk(double *__restrict__ rhs, double *__restrict__ ynext,
-                                                  double *__restrict__ interim, const double *__restrict__ ycur,
-                                                  const int8_t *__restrict__ iblank, int n, double h, double bi,
-                                                  double a, int last, int nv) {
-#pragma clang fp contract(off)
-  const int p = blockIdx.x * TPB + threadIdx.x;
-  if (p >= n) return;
-  if (!iblank || iblank[p] != BLANKED) {
-    for (int v = 0; v < nv; v++) {
-      const size_t q = (size_t)v * n + p;
-      rhs[q] *= h;
-      ynext[q] += bi * rhs[q];
-      if (!last) interim[q] = ycur[q] + a * rhs[q];
-    }
-  } else {
-    for (int v = 0; v < nv; v++) {
-      const size_t q = (size_t)v * n + p;
-      rhs[q] = 0.0;
-      ynext[q] = 0.0;
-      interim[q] = 0.0;
-    }
-  }
-}
-
-// compute_auxiliary_variables_linear_Euler (state.cpp:701-736), rho' only:
-// rho' = (p' gamma^-1 p_bar^-1 - s') rho_bar
-__global__ void __launch_bounds__(TPB) k_aux_rho(const double *__restrict__ y, const double *__restrict__ mean,
-                                                 const double *__restrict__ rhob, double *__restrict__ rho,
-                                                 double gi, int n) {
-#pragma clang fp contract(off)
-  const int p = blockIdx.x * TPB + threadIdx.x;
-  if (p >= n) return;
-  const double pbi = 1.0 / mean[(size_t)IP * n + p];
-  double r = y[(size_t)IP * n + p] * gi * pbi - y[(size_t)IS * n + p];
-  r *= rhob[p];
-  rho[p] = r;
-}
-
-// filter blend: y = (1 - blend) func0 + blend func
-__global__ void __launch_bounds__(TPB) k_blend(double *__restrict__ y, const double *__restrict__ f0,
-                                               const double *__restrict__ f, double rem, double blend, int n) {
-#pragma clang fp contract(off)
-  const int p = blockIdx.x * TPB + threadIdx.x;
-  if (p < n) y[p] = rem * f0[p] + blend * f[p];
-}
-
-// temporal::iblank_correction (temporal:380-393): holes -> sol_ref = 0
-__global__ void __launch_bounds__(TPB) k_iblank_reset(double *__restrict__ y, const int8_t *__restrict__ iblank,
-                                                      int n, int nv) {
-  const int p = blockIdx.x * TPB + threadIdx.x;
-  if (p >= n || iblank[p] != BLANKED) return;
-  for (int v = 0; v < nv; v++) y[(size_t)v * n + p] = 0.0;
-}
 
 // ------------------------------------------------------ boundary conditions
 
@@ -1162,144 +931,6 @@ inline unsigned nblocks(size_t n) { return (unsigned)((n + TPB - 1) / TPB); }
 
 // ------------------------------------------------------------- launchers
 
-hipError_t plain_apply_op(hipStream_t s, const Block &b, const OpTable &op, const int8_t *codes, const double *f,
-                          double *df, int dir) {
-  hipLaunchKernelGGL(k_plain_op_dir, dim3(nblocks(b.n)), dim3(TPB), 0, s, f, df, codes, b.ni, b.nj, dir, op);
-  return hipGetLastError();
-}
-
-hipError_t metrics2d(hipStream_t s, Block &b, const OpTable &fd) {
-  // x_xi, x_eta, y_xi, y_eta by the FD operator with no holes (metrics are
-  // computed before overset marks any, simulation.cpp:207-217)
-  double *xx = nullptr;
-  hipError_t e = hipMalloc((void **)&xx, sizeof(double) * 4 * (size_t)b.n);
-  if (e != hipSuccess) return e;
-  for (int ph = 0; ph < 2; ph++)
-    for (int cp = 0; cp < 2; cp++) {
-      hipLaunchKernelGGL(k_plain_op_dir, dim3(nblocks(b.n)), dim3(TPB), 0, s, b.xyz + (size_t)ph * b.n,
-                         xx + (size_t)(2 * ph + cp) * b.n, (const int8_t *)nullptr, b.ni, b.nj, cp, fd);
-    }
-  hipLaunchKernelGGL(k_metrics2d, dim3(nblocks(b.n)), dim3(TPB), 0, s, xx, b.met, b.jac, b.n);
-  e = hipGetLastError();
-  hipError_t e2 = hipStreamSynchronize(s);
-  (void)hipFree(xx);
-  return e != hipSuccess ? e : e2;
-}
-
-hipError_t plain_take_derivative_xyz(hipStream_t s, const Block &b, const OpTable &op, const double *f,
-                                     int dir_xyz) {
-  hipLaunchKernelGGL(k_plain_deriv_xyz, dim3(nblocks(b.n)), dim3(TPB), 0, s, f, b.dflux, b.met, b.jac,
-                     b.has_holes ? b.code_fd : nullptr, b.ni, b.nj, dir_xyz, op);
-  return hipGetLastError();
-}
-
-hipError_t aux_density(hipStream_t s, const Block &b, double gamma, const double *y, double *rho) {
-  hipLaunchKernelGGL(k_aux_rho, dim3(nblocks(b.n)), dim3(TPB), 0, s, y, b.mean, b.rhobar, rho, 1.0 / gamma, b.n);
-  return hipGetLastError();
-}
-
-// spatial::compute_RHS + compute_RHS_linearized_Euler + add_RHSSourceTerms
-// (spatial:1963-1990, 2053-2130; source.cpp:10-18), one kernel per array
-// operation of the reference.  rho: the aux density to use; anything other
-// than the block's carried array is first filled from y.
-hipError_t plain_rhs(hipStream_t s, lee_handle *h, const Block &b, const double *y, double *rhs, double s1,
-                     double s2, double *rho, double he) {
-  const int n = b.n;
-  const dim3 g(nblocks(n)), t(TPB);
-  const double gam = h->cfg.gamma;
-  auto Y = [&](int v) { return y + (size_t)v * n; };
-  auto R = [&](int v) { return rhs + (size_t)v * n; };
-  auto M = [&](int v) { return b.mean + (size_t)v * n; };
-  auto G = [&](int v, int d) { return b.mgrad + (size_t)(2 * v + d) * n; };
-  if (rho != b.rho64) {  // unit call: aux density of y itself, carried rho' untouched
-    hipError_t e = aux_density(s, b, gam, y, rho);
-    if (e != hipSuccess) return e;
-  }
-  hipError_t err = hipSuccess;  // first failure of the derivative launches
-  auto deriv = [&](const double *f, int d) {
-    const hipError_t e = plain_take_derivative_xyz(s, b, h->fd, f, d);
-    if (err == hipSuccess) err = e;
-  };
-  const int nv = nvars(h);
-  hipLaunchKernelGGL(k_fill, dim3(nblocks((size_t)nv * n)), t, 0, s, rhs, 0.0, (size_t)nv * n);
-  for (int d = 0; d < 2; d++) {
-    deriv(Y(IS), d);
-    hipLaunchKernelGGL(k_sub_ab, g, t, 0, s, R(IS), M(IUX + d), b.dflux, n);
-    hipLaunchKernelGGL(k_sub_ab, g, t, 0, s, R(IS), Y(IUX + d), G(IS, d), n);
-  }
-  for (int vel = 0; vel < 2; vel++) {
-    for (int d = 0; d < 2; d++) {
-      deriv(Y(IUX + vel), d);
-      hipLaunchKernelGGL(k_sub_ab, g, t, 0, s, R(IUX + vel), M(IUX + d), b.dflux, n);
-      hipLaunchKernelGGL(k_sub_velgrad, g, t, 0, s, R(IUX + vel), Y(IUX + d), rho, b.rhobar, M(IUX + d),
-                         G(IUX + vel, d), n);
-    }
-    deriv(Y(IP), vel);
-    hipLaunchKernelGGL(k_sub_div, g, t, 0, s, R(IUX + vel), b.dflux, b.rhobar, n);
-  }
-  for (int d = 0; d < 2; d++) {
-    deriv(Y(IP), d);
-    hipLaunchKernelGGL(k_sub_ab, g, t, 0, s, R(IP), M(IUX + d), b.dflux, n);
-    hipLaunchKernelGGL(k_sub_ab, g, t, 0, s, R(IP), Y(IUX + d), G(IP, d), n);
-    deriv(Y(IUX + d), d);
-    hipLaunchKernelGGL(k_sub_gab, g, t, 0, s, R(IP), gam, M(IP), b.dflux, n);
-    hipLaunchKernelGGL(k_sub_gab, g, t, 0, s, R(IP), gam, Y(IP), G(IUX + d, d), n);
-  }
-  if (h->cfg.axisym)
-    hipLaunchKernelGGL(k_plain_axisym, g, t, 0, s, R(IP), gam, M(IP), Y(IUY), Y(IP), M(IUY), b.xyz + n, n);
-  // passive scalars, compute_RHS_linearized_Euler_scalar (spatial:2134-2158)
-  // after the LEE terms (spatial:1977-1979)
-  for (int v = NV; v < nv; v++)
-    for (int d = 0; d < 2; d++) {
-      deriv(Y(v), d);
-      hipLaunchKernelGGL(k_sub_ab, g, t, 0, s, R(v), M(IUX + d), b.dflux, n);
-      hipLaunchKernelGGL(k_sub_ab, g, t, 0, s, R(v), Y(IUX + d), G(v, d), n);
-    }
-  if (b.src.i1 >= b.src.i0) {
-    const size_t cnt = (size_t)(b.src.i1 - b.src.i0 + 1) * (b.src.j1 - b.src.j0 + 1);
-    hipLaunchKernelGGL(k_plain_source, dim3(nblocks(cnt)), t, 0, s, R(IP), b.src.g, b.ni, b.src.i0, b.src.i1,
-                       b.src.j0, b.src.j1, s1, s2);
-  }
-  for (const auto &z : b.zones) {
-    const size_t cnt = (size_t)z.nz[0] * z.nz[1];
-    hipLaunchKernelGGL(k_plain_sponge, dim3(nblocks(cnt)), t, 0, s, rhs, y, z.sigma64, b.ni, n, z.is[0], z.nz[0],
-                       z.is[1], z.nz[1], z.harmonic ? 1 : 0, he, z.hg, nv);
-  }
-  const hipError_t last = hipGetLastError();
-  return err != hipSuccess ? err : last;
-}
-
-hipError_t plain_rk_update(hipStream_t s, const Block &b, double *rhs, double *ynext, double *interim,
-                           const double *ycur, double hdt, double bi, double a, bool last, int nv) {
-  hipLaunchKernelGGL(k_plain_rk, dim3(nblocks(b.n)), dim3(TPB), 0, s, rhs, ynext, interim, ycur,
-                     b.has_holes ? b.iblank : nullptr, b.n, hdt, bi, a, last ? 1 : 0, nv);
-  return hipGetLastError();
-}
-
-hipError_t plain_filter(hipStream_t s, lee_handle *h, const Block &b, double *y) {
-  const int n = b.n;
-  const dim3 g(nblocks(n)), t(TPB);
-  const double blend = h->cfg.filter_blend, rem = 1.0 - blend;
-  for (int v = 0; v < nvars(h); v++) {
-    double *yv = y + (size_t)v * n;
-    hipLaunchKernelGGL(k_copy, g, t, 0, s, yv, b.func0, (size_t)n);
-    hipLaunchKernelGGL(k_copy, g, t, 0, s, b.func0, b.func, (size_t)n);
-    for (int d = 0; d < 2; d++) {
-      hipLaunchKernelGGL(k_plain_op_dir, g, t, 0, s, b.func, b.dflux,
-                         b.has_holes ? b.code_flt + (size_t)d * n : nullptr, b.ni, b.nj, d, h->flt);
-      hipLaunchKernelGGL(k_copy, g, t, 0, s, b.dflux, b.func, (size_t)n);
-    }
-    hipLaunchKernelGGL(k_blend, g, t, 0, s, yv, b.func0, b.func, rem, blend, n);
-  }
-  return hipGetLastError();
-}
-
-hipError_t plain_iblank_reset(hipStream_t s, const Block &b, double *y, int nv) {
-  if (!b.has_holes) return hipSuccess;
-  hipLaunchKernelGGL(k_iblank_reset, dim3(nblocks(b.n)), dim3(TPB), 0, s, y, b.iblank, b.n, nv);
-  return hipGetLastError();
-}
-
 static BcArgs make_bc_args(const lee_handle *h, const Block &b, const BcFace &f, double he) {
   BcArgs a{};
   a.he = he;
@@ -1359,8 +990,7 @@ static hipError_t overset_t(hipStream_t s, lee_handle *h, T *const *ys, T *const
   return hipGetLastError();
 }
 
-// buf_index selects the state buffer (Y[k]) of every block; buf_index < 0
-// means the plain path's arrays (-1 interim, -2 ynp1).
+// buf_index selects the state buffer (Y[k]) of every block.
 hipError_t overset_interpolate(hipStream_t s, lee_handle *h, bool fp32, int buf_index, bool last_stage) {
   if (h->ov.nrecv == 0) return hipSuccess;
   if (fp32) {
@@ -1376,9 +1006,8 @@ hipError_t overset_interpolate(hipStream_t s, lee_handle *h, bool fp32, int buf_
   double *ys[MAX_OV_BLOCKS], *rh[MAX_OV_BLOCKS];
   bool any_rho = false;
   for (int ib = 0; ib < h->nblk; ib++) {
-    if (buf_index >= 0) ys[ib] = h->b[ib].Y64[buf_index];
-    else ys[ib] = buf_index == -1 ? h->b[ib].interim : h->b[ib].ynp1;
-    rh[ib] = (buf_index >= 0 && !h->b[ib].uniform_mean) ? h->b[ib].rho64 : nullptr;
+    ys[ib] = h->b[ib].Y64[buf_index];
+    rh[ib] = h->b[ib].uniform_mean ? nullptr : h->b[ib].rho64;
     any_rho |= rh[ib] != nullptr;
   }
   return overset_t<double>(s, h, ys, rh, last_stage && any_rho, h->ov.buf);

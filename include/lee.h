@@ -41,8 +41,8 @@ extern "C" {
 
 /* execution path */
 #define LEE_PATH_FUSED 0  /* fused stage + filter kernels (default) */
-#define LEE_PATH_PLAIN 1  /* one kernel per reference operator, FP64 only,
-                             bit-identical arithmetic order */
+#define LEE_PATH_PLAIN 1  /* the reference's arithmetic, FP64 only,
+                             bit-identical operation order */
 
 /* boundary / buffer-zone types: src/core/param.h:104-125 numbering */
 #define LEE_BC_DIRICHLET 0                   /* rejected: the reference exits for LEE (state.cpp:746-749) */

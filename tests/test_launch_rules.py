@@ -3,7 +3,7 @@ rules: against plain formulas, the CPU oracle, or the form they replace."""
 import numpy as np
 import pytest
 
-from camille_amd import FP32, FP64, Solver
+from camille_amd import FP32, FP64, PATH_PLAIN, Solver
 
 pytestmark = pytest.mark.gpu
 
@@ -56,4 +56,37 @@ def test_3d_stage_chunks(dims, prec, tol):
     lk = s.compute_rhs_adjoint(kap)
     a, b = float(np.sum(r * kap)), float(np.sum(q * lk))
     assert abs(a - b) <= tol * np.linalg.norm(r) * np.linalg.norm(kap)
+    s.close()
+
+
+# a last column tile of 1, 4 and 1 points (11-point closure rows reach 8 back
+# into the tile before) and of 62
+@pytest.mark.parametrize("shape", [(65, 11), (68, 13), (129, 12), (126, 17)])
+@pytest.mark.parametrize("order", [4, 11])
+def test_plain_stage_tile_edges(shape, order):
+    """The plain path equals the oracle bit for bit where its tiles end in
+    slivers, with a sheared mean flow, a carried w', sponges and walls."""
+    from oracle.pyoracle import Oracle
+    ni, nj = shape
+    rng = np.random.default_rng(7)
+    i, j = np.meshgrid(np.arange(ni), np.arange(nj))
+    x, y = 0.5 * i + 0.1 * np.sin(0.7 * j), 0.5 * j + 0.1 * np.sin(0.4 * i)
+    mean = np.zeros((5, nj, ni))
+    mean[0] = 0.05 * np.cos(0.3 * x)
+    mean[1] = 0.2 * np.tanh(0.5 * (y - y.mean()))
+    mean[4] = (1.0 + 0.05 * np.sin(0.2 * x + 0.3 * y)) / GAMMA
+    ic = 1e-4 * rng.standard_normal((5, nj, ni))
+    bc = [(0, "sponge_freund_ambient", "+xi", "0", "4", "0", "-0", "0", "0"),
+          (0, "sponge_freund_ambient", "-xi", "-3", "-0", "0", "-0", "0", "0"),
+          (0, "wall_slip_kinematic", "+eta", "0", "-0", "0", "0", "0", "0"),
+          (0, "neumann", "-eta", "0", "-0", "-0", "-0", "0", "0")]
+    scheme = dict(fd_order=order, filter_order=8 if order == 4 else 11, filter_blend=0.9, filter_strength=0.6, rk=4,
+                  sponge_order=2, sponge_constant=5.0)
+    o = Oracle([dict(x=x, y=y, mean=mean, ic=ic)], scheme, bc, None, "FIX_CFL", 0.4)
+    o.run(6)
+    s = Solver([dict(x=x, y=y, mean=mean)], boundaries=bc, precision=FP64, path=PATH_PLAIN, mode="FIX_CFL", value=0.4,
+               fd_order=order, filter_order=scheme["filter_order"], filter_blend=0.9, filter_strength=0.6)
+    s.set_solution(ic)
+    s.solve(6)
+    assert np.array_equal(s.solution(), o.solution(0)[:, 0])
     s.close()
