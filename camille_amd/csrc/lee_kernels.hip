@@ -13,8 +13,9 @@
 
 #include <cmath>
 
-#include "lee_internal.h"
+#include "lee_bc.h"
 #include "lee_device.h"
+#include "lee_internal.h"
 
 namespace lee {
 
@@ -22,21 +23,7 @@ namespace {
 
 // ------------------------------------------------------ boundary conditions
 
-struct BcArgs {
-  int type, dir, end;
-  int i0, i1, j0, j1;   // face box (collapsed along dir)
-  int ni, nj;
-  double neu[9];        // closure row 0 of the FD operator (sb entries)
-  int sb;
-  double he;            // dirichlet_harmonicwave: entropy factor e(t) at the BC time
-  const double *hg;     // and g per face point (null: 1)
-  int nsc;              // passive scalars (variables NV .. NV + nsc - 1)
-};
-
-// bc::apply_BC one face (boundary_condition.cpp:46-209) with bc_neumann
-// (:348-444), bc_wall_slip_kinematic (:448-494), dirichlet_allzero and the
-// Cartesian centerline conditions.  Arithmetic in FP64 for both precisions.
-// Face point q (of the face box, i fastest) of one BC face.
+// One point of a BC face in global memory.
 template <typename T>
 __device__ __forceinline__ void bc_face_point(T *__restrict__ y, const double *__restrict__ met,
                                               const double *__restrict__ jac, const int8_t *__restrict__ iblank,
@@ -48,93 +35,26 @@ __device__ __forceinline__ void bc_face_point(T *__restrict__ y, const double *_
   const int n = a.ni * a.nj;
   const int p = j * a.ni + i;
   if (iblank && iblank[p] == BLANKED) return;
+  const int c = a.dir == 0 ? i : j, len = a.dir == 0 ? a.ni : a.nj, sg = a.end == 0 ? 1 : -1;
   const int mf = a.dir == 0 ? 1 : a.ni;
-  const int c = a.dir == 0 ? i : j, len = a.dir == 0 ? a.ni : a.nj;
+  // the block point s points inward (clamped to the face point)
+  auto at = [&](int s) {
+    const int cs = c + sg * s;
+    return p + sg * mf * (cs >= 0 && cs < len ? s : 0);
+  };
   double data[NV];
-  for (int v = 0; v < NV; v++) data[v] = 1.0e9 * (double)(a.dir + 1);
-  if (a.type == LEE_BC_DIRICHLET_ALLZERO)
-    for (int v = 0; v < NV; v++) data[v] = 0.0;
-  if (a.type == LEE_BC_DIRICHLET_HARMONICWAVE) {  // WAVE_ENTROPY: s' = e(t) g, the rest 0 (bc:250-334)
-    for (int v = 0; v < NV; v++) data[v] = 0.0;
-    data[IS] = a.hg ? a.he * a.hg[q] : a.he;
-  }
-  const bool neumann = a.type == LEE_BC_NEUMANN || a.type == LEE_BC_WALL_SLIP_KINEMATIC ||
-                       (a.type >= LEE_BC_CENTERLINE_CART_NORM2X && a.type <= LEE_BC_CENTERLINE_AXISYM);
-  if (neumann) {
-    // every neighbour value is requested first (clamped addresses), then the
-    // closure row is solved in the reference's order with the skipped
-    // entries masked: one memory latency instead of one per entry
-    const int sg = a.end == 0 ? 1 : -1;
-    T nb[NV][8];
-#pragma unroll
-    for (int s = 1; s <= 8; s++) {
-      const int cs = c + sg * s;
-      const int q = p + sg * mf * (cs >= 0 && cs < len ? s : 0);
-#pragma unroll
-      for (int v = 0; v < NV; v++) nb[v][s - 1] = y[(size_t)v * n + q];
-    }
-    for (int v = 0; v < NV; v++) {
-      if (a.type == LEE_BC_WALL_SLIP_KINEMATIC && v >= IUX && v <= IUZ) continue;
-      double d = 0.0;
-#pragma unroll
-      for (int s = 1; s <= 8; s++) {
-        const int cs = c + sg * s;
-        const bool use = s < a.sb && cs >= 0 && cs < len;
-        const double t1 = a.end == 0 ? d - a.neu[s] * (double)nb[v][s - 1] : d + a.neu[s] * (double)nb[v][s - 1];
-        d = use ? t1 : d;
-      }
-      d /= a.end == 0 ? a.neu[0] : -a.neu[0];
-      data[v] = d;
-    }
-  }
-  if (a.type == LEE_BC_WALL_SLIP_KINEMATIC) {
-    const double m00 = met[p], m01 = met[(size_t)n + p], m10 = met[(size_t)2 * n + p], m11 = met[(size_t)3 * n + p];
-    const double u = (double)y[(size_t)IUX * n + p], v = (double)y[(size_t)IUY * n + p];
-    double k0 = 0.0, k1 = 0.0;
-    k0 += m00 * u;
-    k0 += m01 * v;
-    k1 += m10 * u;
-    k1 += m11 * v;
-    if (a.dir == 0) k0 = 0.0; else k1 = 0.0;
-    // metricsInverse (metrics.cpp:375-381): [X][XI] = eta_y, [X][ETA] = -xi_y,
-    // [Y][XI] = -eta_x, [Y][ETA] = xi_x
-    const double J = jac[p];
-    double ux = 0.0, uy = 0.0;
-    ux += m11 * k0;
-    ux += -m01 * k1;
-    ux *= J;
-    uy += -m10 * k0;
-    uy += m00 * k1;
-    uy *= J;
-    data[IUX] = ux;
-    data[IUY] = uy;
-    data[IUZ] = (double)y[(size_t)IUZ * n + p];
-  }
-  if (a.type >= LEE_BC_CENTERLINE_CART_NORM2X && a.type <= LEE_BC_CENTERLINE_CART_NORM2Z)
-    data[IUX + (a.type - LEE_BC_CENTERLINE_CART_NORM2X)] = 0.0;
-  if (a.type == LEE_BC_CENTERLINE_AXISYM) data[IUY] = 0.0;  // u_r on the axis (bc:498-545, IVAR_UR)
+  bc_face_data<T>(a, q, p, c, len, met, jac, [&](int v, int s) { return y[(size_t)v * n + at(s)]; }, data);
   // passive scalars: Neumann data at Neumann, wall-slip (its non-velocity
   // variables, boundary_condition.cpp:122-136) and centerline faces; 0 at
   // dirichlet_allzero and harmonic-wave faces, whose data start at 0
   for (int z = 0; z < a.nsc; z++) {
     const size_t vo = (size_t)(NV + z) * n;
     double d = 0.0;
-    if (neumann) {
-      const int sg = a.end == 0 ? 1 : -1;
+    if (bc_is_neumann(a)) {
       T nbz[8];
 #pragma unroll
-      for (int s = 1; s <= 8; s++) {
-        const int cs = c + sg * s;
-        nbz[s - 1] = y[vo + p + sg * mf * (cs >= 0 && cs < len ? s : 0)];
-      }
-#pragma unroll
-      for (int s = 1; s <= 8; s++) {
-        const int cs = c + sg * s;
-        const bool use = s < a.sb && cs >= 0 && cs < len;
-        const double t1 = a.end == 0 ? d - a.neu[s] * (double)nbz[s - 1] : d + a.neu[s] * (double)nbz[s - 1];
-        d = use ? t1 : d;
-      }
-      d /= a.end == 0 ? a.neu[0] : -a.neu[0];
+      for (int s = 1; s <= 8; s++) nbz[s - 1] = y[vo + at(s)];
+      d = bc_neumann_value<T>(a, c, len, nbz);
     }
     y[vo + p] = (T)d;
   }
@@ -147,13 +67,27 @@ __device__ __forceinline__ void bc_face_point(T *__restrict__ y, const double *_
   }
 }
 
+// Faces of one block that neither read nor write a point another one of them
+// writes, in one launch: workgroups start[k] .. start[k + 1] - 1 take face k.
+// A launch of one face is all latency (4 us for 700 points), so faces that
+// may share one do (a channel's two walls: 8 launches a step -> 4).
+constexpr int BC_BATCH = 4;
+struct BcBatch {
+  int nf;
+  int start[BC_BATCH + 1];
+  BcArgs f[BC_BATCH];
+};
+
 template <typename T>
-__global__ void __launch_bounds__(TPB) k_bc_face(T *__restrict__ y, const double *__restrict__ met,
-                                                 const double *__restrict__ jac,
-                                                 const int8_t *__restrict__ iblank, BcArgs a,
-                                                 T *__restrict__ rho, const double *__restrict__ mean,
-                                                 const double *__restrict__ rhob, double gi) {
-  const int q = blockIdx.x * TPB + threadIdx.x;
+__global__ void __launch_bounds__(TPB) k_bc_faces(T *__restrict__ y, const double *__restrict__ met,
+                                                  const double *__restrict__ jac,
+                                                  const int8_t *__restrict__ iblank, BcBatch b,
+                                                  T *__restrict__ rho, const double *__restrict__ mean,
+                                                  const double *__restrict__ rhob, double gi) {
+  int k = 0;
+  while (k + 1 < b.nf && (int)blockIdx.x >= b.start[k + 1]) k++;
+  const BcArgs &a = b.f[k];
+  const int q = ((int)blockIdx.x - b.start[k]) * TPB + threadIdx.x;
   if (q >= (a.i1 - a.i0 + 1) * (a.j1 - a.j0 + 1)) return;
   bc_face_point<T>(y, met, jac, iblank, a, rho, mean, rhob, gi, q);
 }
@@ -950,19 +884,48 @@ static BcArgs make_bc_args(const lee_handle *h, const Block &b, const BcFace &f,
   return a;
 }
 
+// The points face f writes, grown by those its rows read.
+struct BcReach {
+  int lo[2], hi[2];
+};
+static BcReach bc_reach(const BcArgs &a) {
+  BcReach r{{a.i0, a.j0}, {a.i1, a.j1}};
+  if (a.end == 0) r.hi[a.dir] += a.sb - 1;
+  else r.lo[a.dir] -= a.sb - 1;
+  return r;
+}
+
 hipError_t apply_bcs(hipStream_t s, lee_handle *h, const Block &b, double *y64, float *y32, bool fp32,
                      double *rho64, float *rho32, double he) {
+  const int8_t *ib = b.has_holes ? b.iblank : nullptr;
+  BcBatch t{};
+  auto flush = [&]() {
+    if (t.nf == 0) return;
+    const dim3 grid(t.start[t.nf]);
+    if (fp32)
+      hipLaunchKernelGGL(k_bc_faces<float>, grid, dim3(TPB), 0, s, y32, b.met, b.jac, ib, t, rho32, b.mean, b.rhobar,
+                         1.0 / h->cfg.gamma);
+    else
+      hipLaunchKernelGGL(k_bc_faces<double>, grid, dim3(TPB), 0, s, y64, b.met, b.jac, ib, t, rho64, b.mean, b.rhobar,
+                         1.0 / h->cfg.gamma);
+    t.nf = 0;
+  };
+  // in the order of the BC file; a face joins the launch before it unless
+  // their reaches meet (faces that share a corner keep their order)
   for (const auto &f : b.faces) {
     const BcArgs a = make_bc_args(h, b, f, he);
-    const size_t cnt = (size_t)(a.i1 - a.i0 + 1) * (a.j1 - a.j0 + 1);
-    const int8_t *ib = b.has_holes ? b.iblank : nullptr;
-    if (fp32)
-      hipLaunchKernelGGL(k_bc_face<float>, dim3(nblocks(cnt)), dim3(TPB), 0, s, y32, b.met, b.jac, ib, a, rho32,
-                         b.mean, b.rhobar, 1.0 / h->cfg.gamma);
-    else
-      hipLaunchKernelGGL(k_bc_face<double>, dim3(nblocks(cnt)), dim3(TPB), 0, s, y64, b.met, b.jac, ib, a, rho64,
-                         b.mean, b.rhobar, 1.0 / h->cfg.gamma);
+    const BcReach r = bc_reach(a);
+    bool apart = t.nf < BC_BATCH;
+    for (int k = 0; k < t.nf; k++) {
+      const BcReach o = bc_reach(t.f[k]);
+      apart &= r.lo[0] > o.hi[0] || o.lo[0] > r.hi[0] || r.lo[1] > o.hi[1] || o.lo[1] > r.hi[1];
+    }
+    if (!apart) flush();
+    t.f[t.nf] = a;
+    t.start[t.nf + 1] = t.start[t.nf] + (int)nblocks((size_t)(a.i1 - a.i0 + 1) * (a.j1 - a.j0 + 1));
+    t.nf++;
   }
+  flush();
   return hipGetLastError();
 }
 
