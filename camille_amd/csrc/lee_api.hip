@@ -118,23 +118,61 @@ hipError_t mark(lee_handle *h) {
   return hipEventRecord(h->evpool[h->evused++], h->stream);
 }
 
+// Scalars of RK stage st of the step from tn.
+StageScalars stage_scalars(const lee_handle *h, int st) {
+  const double t = h->time_sol + h->c_i[st] * h->dt;
+  StageScalars sc{h->dt, h->b_i[st], h->a_next[st], 0.0, 0.0};
+  source_factors(h->cfg, t, sc.s1, sc.s2);
+  if (h->cfg.harmonic_wave == LEE_WAVE_ENTROPY) sc.he = harmonic_entropy(h->cfg, t);
+  return sc;
+}
+
+// Entropy factor of the boundary data after stage st: t + c_{min(st+1, last)} h
+// (temporal:236-246).
+double stage_bc_entropy(const lee_handle *h, int st) {
+  if (h->cfg.harmonic_wave != LEE_WAVE_ENTROPY) return 0.0;
+  return harmonic_entropy(h->cfg, h->time_sol + h->c_i[std::min(st + 1, h->cfg.rk_stages - 1)] * h->dt);
+}
+
+// The RK stages of a step two a launch; the boundary update after the last
+// one is a launch of its own, the others run inside the pairs.
+int enqueue_paired_stages(lee_handle *h) {
+  const int S = h->cfg.rk_stages;
+  for (int st = 0; st < S; st += 2) {
+    PairStep p;
+    p.sc[0] = stage_scalars(h, st);
+    p.sc[1] = stage_scalars(h, st + 1);
+    p.he_in = st > 0 ? stage_bc_entropy(h, st - 1) : 0.0;
+    p.he_mid = stage_bc_entropy(h, st);
+    if (h->ktiming) HIPCHK(mark(h));
+    for (int ib = 0; ib < h->nblk; ib++) HIPCHK(fused_pair(h->stream, h, h->b[ib], st, p));
+    if (h->ktiming) {
+      HIPCHK(mark(h));
+      h->evclass.push_back(st + 2 == S ? 2 : 0);
+    }
+  }
+  bool any_bnd = false;
+  for (int ib = 0; ib < h->nblk; ib++) any_bnd |= !h->b[ib].faces.empty();
+  if (!any_bnd) return LEE_OK;
+  if (h->ktiming) HIPCHK(mark(h));
+  HIPCHK(boundary_phase_fused(h->stream, h, is_fp32(h), 1, true, stage_bc_entropy(h, S - 1)));
+  if (h->ktiming) {
+    HIPCHK(mark(h));
+    h->evclass.push_back(4);
+  }
+  return LEE_OK;
+}
+
 int enqueue_fused_step(lee_handle *h) {
   const int S = h->cfg.rk_stages, last = S - 1;
-  const double tn = h->time_sol, dt = h->dt;
   const bool f32 = is_fp32(h);
-  for (int st = 0; st < S; st++) {
-    StageScalars sc{};
-    sc.h = dt;
-    sc.b = h->b_i[st];
-    sc.a = h->a_next[st];
-    source_factors(h->cfg, tn + h->c_i[st] * dt, sc.s1, sc.s2);
-    // boundary data after the stage: t + c_{min(i+1, last)} h (temporal:236-246)
-    const double t_bc = tn + h->c_i[std::min(st + 1, last)] * dt;
-    double he_bc = 0.0;
-    if (h->cfg.harmonic_wave == LEE_WAVE_ENTROPY) {
-      sc.he = harmonic_entropy(h->cfg, tn + h->c_i[st] * dt);
-      he_bc = harmonic_entropy(h->cfg, t_bc);
-    }
+  bool paired = true;
+  for (int ib = 0; ib < h->nblk; ib++) paired &= h->b[ib].tune_pair > 0 && paired_stages_ok(h, h->b[ib]);
+  if (paired)
+    if (int rc = enqueue_paired_stages(h)) return rc;
+  for (int st = 0; st < S && !paired; st++) {
+    const StageScalars sc = stage_scalars(h, st);
+    const double he_bc = stage_bc_entropy(h, st);
     if (h->ktiming) HIPCHK(mark(h));
     if (pair_stage_ok(h))
       HIPCHK(fused_stage_pair(h->stream, h, st, sc));
@@ -185,15 +223,11 @@ int enqueue_fused_step(lee_handle *h) {
 
 // temporal::time_advance in the reference's arithmetic (FP64).
 int enqueue_plain_step(lee_handle *h) {
-  const int S = h->cfg.rk_stages, last = S - 1;
-  const double tn = h->time_sol, dt = h->dt;
+  const int S = h->cfg.rk_stages;
   hipStream_t s = h->stream;
-  const bool harm = h->cfg.harmonic_wave == LEE_WAVE_ENTROPY;
   for (int st = 0; st < S; st++) {
-    StageScalars sc{dt, h->b_i[st], h->a_next[st], 0.0, 0.0};
-    source_factors(h->cfg, tn + h->c_i[st] * dt, sc.s1, sc.s2);
-    if (harm) sc.he = harmonic_entropy(h->cfg, tn + h->c_i[st] * dt);
-    const double he_bc = harm ? harmonic_entropy(h->cfg, tn + h->c_i[std::min(st + 1, last)] * dt) : 0.0;
+    const StageScalars sc = stage_scalars(h, st);
+    const double he_bc = stage_bc_entropy(h, st);
     for (int ib = 0; ib < h->nblk; ib++) {
       Block &b = h->b[ib];
       HIPCHK(plain_stage(s, h, b, st, sc, st == 0 ? b.rho64 : nullptr));
@@ -220,15 +254,25 @@ int enqueue_plain_step(lee_handle *h) {
 
 int enqueue_step(lee_handle *h) { return is_plain(h) ? enqueue_plain_step(h) : enqueue_fused_step(h); }
 
-// One step of a batched ensemble: a persistent launch per RK stage over the
-// tiles of every solve, the boundary conditions of the solves that have
+// One step of a batched ensemble: a launch per RK stage or pair of stages over
+// the tiles of every solve, the boundary conditions of the solves that have
 // any, then the filter launch, which also advances the device step counter.
 // The launches only read operand tables and the schedule, so the sequence
 // can be captured once in a HIP graph and replayed.
 int enqueue_batch_step(lee_handle *h) {
   const int S = h->cfg.rk_stages, last = S - 1;
   const bool f32 = is_fp32(h);
-  for (int st = 0; st < S; st++) {
+  // pairs of stages, unless the caller asked for a persistent stage grid
+  const bool paired = h->bp.pair && h->bp.grid_stage == 0;
+  for (int st = 0; st < S && paired; st += 2) {
+    if (h->ktiming) HIPCHK(mark(h));
+    HIPCHK(batch_pair(h->stream, h, st));
+    if (h->ktiming) {
+      HIPCHK(mark(h));
+      h->evclass.push_back(st == 0 ? 0 : 2);
+    }
+  }
+  for (int st = 0; st < S && !paired; st++) {
     if (h->ktiming) HIPCHK(mark(h));
     HIPCHK(batch_stage(h->stream, h, st));
     if (h->ktiming) {
@@ -359,6 +403,45 @@ int batch_autotune(lee_handle *h) {
     }
     if (rc) break;
   }
+  // pairs of stages against the best one-stage form, each over a whole step
+  int bP = 0;
+  bool pairs = true;
+  for (int k = 0; k < h->nblk; k++) pairs = pairs && paired_stages_ok(h, h->b[k]);
+  if (pairs && !rc) {
+    auto time_step = [&](float &ms) -> int {
+      auto step = [&]() -> int {
+        for (int st = 0; st < 4; st += p.pair ? 2 : 1)
+          HIPCHK(p.pair ? batch_pair(h->stream, h, st) : batch_stage(h->stream, h, st));
+        return LEE_OK;
+      };
+      ms = 1e30f;
+      for (int trial = 0; trial < 3; trial++) {
+        HIPCHK(hipEventRecord(e0, h->stream));
+        for (int k = 0; k < 2; k++)
+          if (int e = step()) return e;
+        HIPCHK(hipEventRecord(e1, h->stream));
+        HIPCHK(hipEventSynchronize(e1));
+        float t = 0.f;
+        HIPCHK(hipEventElapsedTime(&t, e0, e1));
+        ms = std::min(ms, t);
+      }
+      return LEE_OK;
+    };
+    p.R = bR;
+    best = 1e30f;
+    for (int q : {0, 1, 2}) {
+      p.pair = q;
+      p.grid_stage = q ? 0 : bG;
+      HIPCHK(batch_prepare(h->stream, h));
+      float ms = 0.f;
+      if ((rc = time_step(ms))) break;
+      if (ms < best) {
+        best = ms;
+        bP = q;
+      }
+    }
+    p.pair = 0;
+  }
   best = 1e30f;
   int bS = 0;
   p.stack = 0;
@@ -402,7 +485,8 @@ int batch_autotune(lee_handle *h) {
   batch_release(h);
   if (rc) return rc;
   p.R = bR;
-  p.grid_stage = bG;
+  p.pair = bP;
+  p.grid_stage = bP ? 0 : bG;
   p.TY = bT;
   p.stack = bS;
   p.grid_filter = bF;
@@ -469,20 +553,21 @@ int batch_solve(lee_handle *h, int nsteps) {
 // or 8 workgroups per CU) is timed with HIP events on the block itself, in
 // buffers that carry no state between steps (stage: input Y2, accumulator
 // Y3, output Y1; filter: Y1 -> Y2); the fastest is kept and cached per (ni,
-// nj, nk, device, precision, mean kind, holes, filter order, carried w')
+// nj, nk, device, precision, mean kind, holes, filter order, carried w',
+// paired stages allowed and the faces they take in)
 // for the life of the process.  The cache is shared by every handle of the
 // process and guarded by a mutex, so handles on different host threads may
 // tune concurrently (two threads may both time one key; the first result
 // stored wins).
 struct TuneKey {
-  int ni, nj, nk, device, prec, meanf, holes, filter_order, carry_w;
+  int ni, nj, nk, device, prec, meanf, holes, filter_order, carry_w, pairs;
   bool operator==(const TuneKey &o) const {
     return ni == o.ni && nj == o.nj && nk == o.nk && device == o.device && prec == o.prec && meanf == o.meanf &&
-           holes == o.holes && filter_order == o.filter_order && carry_w == o.carry_w;
+           holes == o.holes && filter_order == o.filter_order && carry_w == o.carry_w && pairs == o.pairs;
   }
 };
 struct TuneVal {
-  int r, fty, fgrid, mc, ml;
+  int r, fty, fgrid, mc, ml, pair;
 };
 std::vector<std::pair<TuneKey, TuneVal>> g_tune_cache;
 std::mutex g_tune_mutex;
@@ -490,7 +575,8 @@ std::mutex g_tune_mutex;
 TuneKey tune_key(const lee_handle *h, const Block &b) {
   const bool d3 = h->cfg.num_dim == 3;
   return TuneKey{b.ni, b.nj, b.nk, h->device, h->cfg.precision, d3 ? 0 : (b.uniform_mean ? 0 : 1),
-                 d3 ? 0 : (b.has_holes ? 1 : 0), h->cfg.filter_order, b.carry_w ? 1 : 0};
+                 d3 ? 0 : (b.has_holes ? 1 : 0), h->cfg.filter_order, b.carry_w ? 1 : 0,
+                 paired_stages_ok(h, b) ? 1 + (int)b.faces.size() : 0};
 }
 
 bool tune_lookup(const TuneKey &key, Block &b) {
@@ -502,6 +588,7 @@ bool tune_lookup(const TuneKey &key, Block &b) {
       b.tune_fgrid = e.second.fgrid;
       b.tune_mc = e.second.mc;
       b.tune_ml = e.second.ml;
+      b.tune_pair = e.second.pair;
       b.tuned = true;
       return true;
     }
@@ -512,7 +599,7 @@ void tune_store(const TuneKey &key, const Block &b) {
   std::lock_guard<std::mutex> lock(g_tune_mutex);
   for (const auto &e : g_tune_cache)
     if (e.first == key) return;
-  g_tune_cache.push_back({key, {b.tune_r, b.tune_fty, b.tune_fgrid, b.tune_mc, b.tune_ml}});
+  g_tune_cache.push_back({key, {b.tune_r, b.tune_fty, b.tune_fgrid, b.tune_mc, b.tune_ml, b.tune_pair}});
 }
 
 int autotune_block(lee_handle *h, Block &b) {
@@ -602,6 +689,42 @@ int autotune_block(lee_handle *h, Block &b) {
   }
   b.tune_mc = best_mc;
   b.tune_ml = best_ml;
+  // pairs of stages against the best one-stage form: the launches of a step's
+  // four stages, with their boundary launches, on scratch buffers
+  b.tune_pair = 0;
+  if (paired_stages_ok(h, b)) {
+    best = 1e30f;
+    int best_p = 0;
+    for (int q : {0, 1, 2}) {
+      b.tune_pair = q;
+      auto step = [&]() -> int {
+        const PairStep ps{{sc, sc}, 0.0, 0.0};
+        static const int one[4] = {-2, -1, -1, -3};
+        for (int st = 0; st < (q ? 2 : 4); st++) {
+          HIPCHK(q ? fused_pair(h->stream, h, b, -2 - st, ps) : fused_stage(h->stream, h, b, one[st], sc));
+          if (!b.faces.empty() && (!q || st == 1))
+            HIPCHK(apply_bcs(h->stream, h, b, b.Y64[1], b.Y32[1], is_fp32(h), nullptr, nullptr));
+        }
+        return LEE_OK;
+      };
+      float ms = 1e30f;
+      for (int trial = 0; trial < 4; trial++) {  // the first one untimed
+        HIPCHK(hipEventRecord(e0, h->stream));
+        for (int k = 0; k < 4; k++)
+          if (int rc = step()) return rc;
+        HIPCHK(hipEventRecord(e1, h->stream));
+        HIPCHK(hipEventSynchronize(e1));
+        float t = 0.f;
+        HIPCHK(hipEventElapsedTime(&t, e0, e1));
+        if (trial) ms = std::min(ms, t);
+      }
+      if (ms < best) {
+        best = ms;
+        best_p = q;
+      }
+    }
+    b.tune_pair = best_p;
+  }
   b.tuned = true;
   (void)hipEventDestroy(e0);
   (void)hipEventDestroy(e1);
@@ -1533,6 +1656,7 @@ int lee_set_tile_shape(lee_handle *h, int ib, int stage_rows, int filter_rows) {
   if (h->batch) {  // one launch covers every solve: the shape is the batch's
     HIPCHK(hipStreamSynchronize(h->stream));
     h->bp.R = stage_rows;
+    h->bp.pair = 0;   // stage rows select the one-stage launches
     h->bp.TY = filter_rows;
     h->bp.stack = 0;  // a tile height selects the tile forms
     h->bp.tuned = true;
@@ -1540,6 +1664,7 @@ int lee_set_tile_shape(lee_handle *h, int ib, int stage_rows, int filter_rows) {
     return LEE_OK;
   }
   h->b[ib].tune_r = stage_rows;
+  h->b[ib].tune_pair = 0;  // stage rows select the one-stage launches
   h->b[ib].tune_fty = filter_rows;
   h->b[ib].tune_mc = h->b[ib].tune_ml = 0;  // a tile height selects the tile forms
   h->b[ib].tuned = true;

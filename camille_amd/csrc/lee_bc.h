@@ -26,14 +26,15 @@ __device__ __forceinline__ bool bc_is_neumann(const BcArgs &a) {
 
 // bc_neumann (boundary_condition.cpp:348-444): the face value whose closure
 // row vanishes, from the values nb[s - 1] at s points inward; c is the face
-// coordinate on a line of length len.
-template <typename T>
-__device__ __forceinline__ double bc_neumann_value(const BcArgs &a, int c, int len, const T (&nb)[8]) {
+// coordinate on a line of length len.  NS: the most entries past the first
+// that a row of the operator has (2 for OA4, 8 for FDO11P).
+template <typename T, int NS>
+__device__ __forceinline__ double bc_neumann_value(const BcArgs &a, int c, int len, const T (&nb)[NS]) {
 #pragma clang fp contract(off)
   const int sg = a.end == 0 ? 1 : -1;
   double d = 0.0;
 #pragma unroll
-  for (int s = 1; s <= 8; s++) {
+  for (int s = 1; s <= NS; s++) {
     const int cs = c + sg * s;
     const bool use = s < a.sb && cs >= 0 && cs < len;
     const double t1 = a.end == 0 ? d - a.neu[s] * (double)nb[s - 1] : d + a.neu[s] * (double)nb[s - 1];
@@ -49,7 +50,7 @@ __device__ __forceinline__ double bc_neumann_value(const BcArgs &a, int c, int l
 // Face point q of the face box (i fastest), block point p; get(v, s) is the
 // value of variable v at s points inward (s = 0: the face point; clamped to
 // the face point where that leaves the block).
-template <typename T, typename Get>
+template <typename T, int NS, typename Get>
 __device__ __forceinline__ void bc_face_data(const BcArgs &a, int q, int p, int c, int len, const double *met,
                                              const double *jac, Get get, double (&data)[NV]) {
 #pragma clang fp contract(off)
@@ -65,14 +66,14 @@ __device__ __forceinline__ void bc_face_data(const BcArgs &a, int q, int p, int 
     // every neighbour value is requested first (clamped addresses), then the
     // closure row is solved in the reference's order with the skipped
     // entries masked: one memory latency instead of one per entry
-    T nb[NV][8];
+    T nb[NV][NS];
 #pragma unroll
-    for (int s = 1; s <= 8; s++)
+    for (int s = 1; s <= NS; s++)
 #pragma unroll
       for (int v = 0; v < NV; v++) nb[v][s - 1] = get(v, s);
     for (int v = 0; v < NV; v++) {
       if (a.type == LEE_BC_WALL_SLIP_KINEMATIC && v >= IUX && v <= IUZ) continue;
-      data[v] = bc_neumann_value<T>(a, c, len, nb[v]);
+      data[v] = bc_neumann_value<T, NS>(a, c, len, nb[v]);
     }
   }
   if (a.type == LEE_BC_WALL_SLIP_KINEMATIC) {

@@ -105,6 +105,7 @@ struct Block {
   // height 4 R) and filter tile height (4, 8, 16; FP64 4); set by the autotuner
   int tune_r = 1, tune_fty = 4;
   int tune_fgrid = 0;          // filter: 0 one workgroup per tile, else persistent pipelined grid
+  int tune_pair = 0;           // two RK stages a launch: rows per wave of the first stage (1 or 2); 0 off
   int tune_mc = 0, tune_ml = 0;  // filter column-march form (no holes): waves per stack, rows per wave; 0 off
   int cus = 0;                 // compute units of the device
   bool tuned = false;
@@ -200,6 +201,9 @@ struct BatchPlan {
   int grid_stage = 0, grid_filter = 0;  // persistent grid sizes (0: one workgroup per tile)
   int res_stage = 0, res_filter = 0;    // resident workgroups of the prepared stage and filter forms
   void *stage_args = nullptr;  // device StageArgs<T>[stages][nsolve]
+  int pair = 0;                // two RK stages a launch (one workgroup per tile only): rows per wave, 0 off
+  void *pair_args = nullptr;   // device StageArgs<T>[2][nsolve] of the pairs
+  int *tile_map_pair = nullptr, total_pair = 0;
   void *filter_args = nullptr; // device FilterArgs<T>[nsolve]
   int *tile_map_stage = nullptr, *tile_map_filter = nullptr;  // (solve, tile) per list entry
   int total_stage = 0, total_filter = 0;
@@ -334,6 +338,18 @@ bool pair_stage_ok(const lee_handle *h);
 bool pair_filter_ok(const lee_handle *h);
 hipError_t fused_stage_pair(hipStream_t s, lee_handle *h, int stage, const StageScalars &sc);
 hipError_t fused_filter_pair(hipStream_t s, lee_handle *h, int src, int dst);
+// Two RK stages of a block in one launch (lee_step2.hip): whether the block
+// can run so, and stages first and first + 1 (0, 2; -2 and -3 the tuner's
+// first and second pair on scratch buffers) with their scalars and the
+// entropy factors of the boundary update on the input and between them.
+struct PairStep {
+  StageScalars sc[2];
+  double he_in = 0.0, he_mid = 0.0;
+};
+bool paired_stages_ok(const lee_handle *h, const Block &b);
+hipError_t fused_pair(hipStream_t s, lee_handle *h, Block &b, int first, const PairStep &st);
+hipError_t batch_pair(hipStream_t s, lee_handle *h, int first);
+hipError_t batch_pair_prepare(hipStream_t s, lee_handle *h);  // called by batch_prepare
 hipError_t batch_prepare(hipStream_t s, lee_handle *h);
 hipError_t batch_stage(hipStream_t s, lee_handle *h, int stage);
 hipError_t batch_filter(hipStream_t s, lee_handle *h);

@@ -13,9 +13,11 @@
 
 #include <cmath>
 
+#include "lee_args.h"
 #include "lee_bc.h"
 #include "lee_device.h"
 #include "lee_internal.h"
+#include "lee_stage.h"
 
 namespace lee {
 
@@ -43,7 +45,7 @@ __device__ __forceinline__ void bc_face_point(T *__restrict__ y, const double *_
     return p + sg * mf * (cs >= 0 && cs < len ? s : 0);
   };
   double data[NV];
-  bc_face_data<T>(a, q, p, c, len, met, jac, [&](int v, int s) { return y[(size_t)v * n + at(s)]; }, data);
+  bc_face_data<T, 8>(a, q, p, c, len, met, jac, [&](int v, int s) { return y[(size_t)v * n + at(s)]; }, data);
   // passive scalars: Neumann data at Neumann, wall-slip (its non-velocity
   // variables, boundary_condition.cpp:122-136) and centerline faces; 0 at
   // dirichlet_allzero and harmonic-wave faces, whose data start at 0
@@ -54,7 +56,7 @@ __device__ __forceinline__ void bc_face_point(T *__restrict__ y, const double *_
       T nbz[8];
 #pragma unroll
       for (int s = 1; s <= 8; s++) nbz[s - 1] = y[vo + at(s)];
-      d = bc_neumann_value<T>(a, c, len, nbz);
+      d = bc_neumann_value<T, 8>(a, c, len, nbz);
     }
     y[vo + p] = (T)d;
   }
@@ -360,100 +362,9 @@ __device__ __forceinline__ void stage_finish(const AT &a, const StepT<T> &sc, in
         dy[v] = wide_row<T>(sp, RS, cy, a.fdw);
       }
     }
-    // chain rule with FP64 metrics (spatial:1810-1820)
-    const double mxx = pm[k][0], mxy = pm[k][1], myx = pm[k][2], myy = pm[k][3];
-    const double J = pj[k];
-    T fx[4], fy[4];
-#pragma unroll
-    for (int v = 0; v < 4; v++) {
-      fx[v] = (T)(fmx(mxx, (double)dx[v], myx * (double)dy[v]) * J);
-      fy[v] = (T)(fmx(mxy, (double)dx[v], myy * (double)dy[v]) * J);
-    }
-    // LEE right-hand side (spatial:2053-2130), reference term order
-    const T sv = yc[0], uv = yc[1], vv = yc[2], pv = yc[3];
-    T rs, ru, rv, rp;
-    if (!MEANF) {
-      const T u0 = (T)a.u0, v0 = (T)a.v0, gp0 = (T)a.gp0;
-      rs = -(u0 * fx[0]);
-      rs = fmx(-v0, fy[0], rs);
-      ru = -(u0 * fx[1]);
-      ru = fmx(-v0, fy[1], ru);
-      rv = -(u0 * fx[2]);
-      rv = fmx(-v0, fy[2], rv);
-      if (sizeof(T) == 8) {
-        ru -= fx[3] / (T)a.rhob0;
-        rv -= fy[3] / (T)a.rhob0;
-      } else {
-        const T irb = (T)(1.0 / a.rhob0);
-        ru = fmx(-fx[3], irb, ru);
-        rv = fmx(-fy[3], irb, rv);
-      }
-      rp = -(u0 * fx[3]);
-      rp = fmx(-gp0, fx[1], rp);
-      rp = fmx(-v0, fy[3], rp);
-      rp = fmx(-gp0, fy[2], rp);
-    } else {
-      // per-point mean coefficients (MC_* order): u, v, gamma p, 1/rho,
-      // the eight mean gradients, rho gi / p and rho (all at the point)
-      const T *mc = a.mc;
-      const T u0 = mc[MC_U * n + p], v0 = mc[MC_V * n + p], gp = mc[MC_GP * n + p], irb = mc[MC_IRB * n + p];
-      const T gsx = mc[MC_GSX * n + p], gsy = mc[MC_GSY * n + p];
-      const T gux = mc[MC_GUX * n + p], guy = mc[MC_GUY * n + p];
-      const T gvx = mc[MC_GVX * n + p], gvy = mc[MC_GVY * n + p];
-      const T gpx = mc[MC_GPX * n + p], gpy = mc[MC_GPY * n + p];
-      T rho;
-      if (KIND == STAGE_FIRST) rho = a.rho_in[p];
-      else rho = fmx(pv, mc[MC_RP * n + p], -(sv * mc[MC_RB * n + p]));
-      const T g = (T)a.gamma;
-      const T ru_fac = rho * irb;
-      const T uf = fmx(ru_fac, u0, uv), vf = fmx(ru_fac, v0, vv), gpv = g * pv;
-      rs = -(u0 * fx[0]);
-      rs = fmx(-uv, gsx, rs);
-      rs = fmx(-v0, fy[0], rs);
-      rs = fmx(-vv, gsy, rs);
-      ru = -(u0 * fx[1]);
-      ru = fmx(-uf, gux, ru);
-      ru = fmx(-v0, fy[1], ru);
-      ru = fmx(-vf, guy, ru);
-      ru = fmx(-fx[3], irb, ru);
-      rv = -(u0 * fx[2]);
-      rv = fmx(-uf, gvx, rv);
-      rv = fmx(-v0, fy[2], rv);
-      rv = fmx(-vf, gvy, rv);
-      rv = fmx(-fy[3], irb, rv);
-      rp = -(u0 * fx[3]);
-      rp = fmx(-uv, gpx, rp);
-      rp = fmx(-gp, fx[1], rp);
-      rp = fmx(-gpv, gux, rp);
-      rp = fmx(-v0, fy[3], rp);
-      rp = fmx(-vv, gpy, rp);
-      rp = fmx(-gp, fy[2], rp);
-      rp = fmx(-gpv, gvy, rp);
-      // axisymmetry (spatial:2119-2126): -gamma (pbar v' + p' vbar) / (r + 1e-99)
-      if (a.axi) rp -= fmx(gp, vv, g * v0 * pv) / mc[MC_R * n + p];
-    }
-    // physical source (source.cpp:22-107), pressure equation
-    if (gi >= a.si0 && gi <= a.si1 && gj >= a.sj0 && gj <= a.sj1) {
-      const double gval = a.g[(gj - a.sj0) * (a.si1 - a.si0 + 1) + (gi - a.si0)];
-      rp += (T)(sc.s1 * gval * sc.s2);
-    }
-    // Freund sponges, zone by zone (source.cpp:136-201), sol_ref = 0
-#pragma unroll 1
-    for (int z = 0; z < a.nz; z++) {
-      const auto &zz = a.z[z];
-      if (gi >= zz.i0 && gi <= zz.i1 && gj >= zz.j0 && gj <= zz.j1) {
-        const int zp = (gj - zz.j0) * zz.nzi + (gi - zz.i0);
-        const T sg = zz.sig[zp];
-        // a harmonic-wave zone relaxes s' to e(t) g (source.cpp:264-320)
-        const T ds = zz.harm ? sv - (T)(zz.hg ? a.he * zz.hg[zp] : a.he) : sv;
-        rs = fmx(-sg, ds, rs);
-        ru = fmx(-sg, uv, ru);
-        rv = fmx(-sg, vv, rv);
-        rp = fmx(-sg, pv, rp);
-      }
-    }
+    T r[4];
+    stage_rhs<T, MEANF, KIND == STAGE_FIRST>(a, sc.s1, sc.s2, a.he, gi, gj, p, n, pm[k], pj[k], yc, dx, dy, r);
     // RK stage update (temporal:208-230)
-    T r[4] = {rs, ru, rv, rp};
     const bool hole = HOLES && a.iblank[p] == BLANKED;
 #pragma unroll
     for (int v = 0; v < 4; v++) {
@@ -536,16 +447,6 @@ __global__ void __launch_bounds__(TPB) k_fused_stage_pair(StageArgs<T> a0, Stage
 // contiguous eighth of the list.  Per-solve operands come from `args`, the
 // per-step scalars from `sched`, indexed by the step counter that the
 // step's last kernel advances.
-template <typename T>
-struct BatchStageArgs {
-  const StageArgs<T> *args;      // nsolve entries for this stage
-  const int *map;                // (solve, tile) per list entry
-  const BatchSched *sched;       // [step][solve][stage]
-  const int *counter;            // step index within the schedule
-  int nsolve, nstage, stage, total, chunk;
-  T b, a;
-};
-
 // The operand tables are read through the constant address space: they do
 // not change during a launch, so their loads are scalar and the pointers
 // loaded from them are known to address global memory (no flat accesses).
@@ -865,25 +766,6 @@ inline unsigned nblocks(size_t n) { return (unsigned)((n + TPB - 1) / TPB); }
 
 // ------------------------------------------------------------- launchers
 
-static BcArgs make_bc_args(const lee_handle *h, const Block &b, const BcFace &f, double he) {
-  BcArgs a{};
-  a.he = he;
-  a.hg = f.hg;
-  a.type = f.type;
-  a.dir = f.dir;
-  a.end = f.end;
-  a.i0 = f.is[0];
-  a.i1 = f.ie[0];
-  a.j0 = f.is[1];
-  a.j1 = f.ie[1];
-  a.ni = b.ni;
-  a.nj = b.nj;
-  a.sb = h->fd.sb;
-  a.nsc = h->cfg.num_scalar;
-  for (int q = 0; q < 9; q++) a.neu[q] = h->fd.bnd[0][q];
-  return a;
-}
-
 // The points face f writes, grown by those its rows read.
 struct BcReach {
   int lo[2], hi[2];
@@ -997,94 +879,6 @@ hipError_t boundary_phase_fused(hipStream_t s, lee_handle *h, bool fp32, int tgt
     if (e != hipSuccess) return e;
   }
   return overset_interpolate(s, h, fp32, tgt, last);
-}
-
-template <typename T>
-static void fill_zones(StageArgs<T> &a, const Block &b) {
-  a.nz = 0;
-  for (const auto &z : b.zones) {
-    if (a.nz >= MAX_ZONES) break;
-    ZoneT<T> &q = a.z[a.nz++];
-    q.i0 = z.is[0];
-    q.i1 = z.ie[0];
-    q.j0 = z.is[1];
-    q.j1 = z.ie[1];
-    q.nzi = z.nz[0];
-    if constexpr (sizeof(T) == 8) q.sig = (const T *)z.sigma64;
-    else q.sig = (const T *)z.sigma32;
-    q.harm = z.harmonic ? 1 : 0;
-    q.hg = z.hg;
-  }
-}
-
-// Stage kind of RK stage `stage` (stage < 0: right-hand side only).
-static int stage_kind(const lee_handle *h, int stage) {
-  const int last = h->cfg.rk_stages - 1;
-  return stage <= 0 ? (stage == 0 ? STAGE_FIRST : STAGE_MID) : (stage == last ? STAGE_LAST : STAGE_MID);
-}
-
-// Operands of one RK stage on block b with R rows per thread.
-template <typename T>
-static StageArgs<T> make_stage_args(const lee_handle *h, const Block &b, int stage, T *const *Y, T *rho, int R,
-                                    const StageScalars &sc) {
-  StageArgs<T> a{};
-  a.ni = b.ni;
-  a.nj = b.nj;
-  a.ntx = (b.ni + ST_TX - 1) / ST_TX;
-  a.nty = (b.nj + 4 * R - 1) / (4 * R);
-  a.ntiles = a.ntx * a.nty;
-  a.chunk = (a.ntiles + 7) / 8;
-  // stage 0 reads Y0 and writes Y1 (accumulator) and Y2; odd stages read
-  // Y2 and write Y3, even stages read Y3 and write Y2; y_n stays in Y0.
-  // stage < 0 (lee_compute_rhs): y in Y[2], zeroed accumulator Y[3] with
-  // h = b = 1 receives the RHS, Y[1] is scratch
-  const int in_idx = stage == 0 ? 0 : (stage % 2 == 1 ? 2 : 3);
-  const int out_idx = stage % 2 == 0 ? 2 : 3;
-  a.yin = Y[in_idx];
-  a.yn = Y[0];
-  a.acc = Y[1];
-  a.yout = Y[out_idx];
-  if (stage < 0) {
-    a.yin = Y[2];
-    a.yn = Y[2];
-    a.acc = Y[3];
-    a.yout = Y[1];
-  }
-  a.met = b.met;
-  a.jac = b.jac;
-  a.iblank = b.iblank;
-  a.code = b.code_fd;
-  a.clean = b.clean_fd;
-  a.mean = b.mean;
-  a.mgrad = b.mgrad;
-  a.rhob = b.rhobar;
-  a.mc = sizeof(T) == 8 ? (const T *)b.mc64 : (const T *)b.mc32;
-  a.rho_in = rho;
-  a.rho_out = rho;
-  a.u0 = b.umean[IUX];
-  a.v0 = b.umean[IUY];
-  a.gamma = h->cfg.gamma;
-  a.axi = h->cfg.axisym;
-  a.gi = 1.0 / h->cfg.gamma;
-  a.gp0 = h->cfg.gamma * b.umean[IP];
-  {
-    const double pbar = b.umean[IP], sbar = b.umean[IS];
-    a.rhob0 = std::pow(h->cfg.gamma * pbar, 1.0 / h->cfg.gamma) * std::exp(-sbar);
-  }
-  fill_zones(a, b);
-  a.si0 = b.src.i0;
-  a.si1 = b.src.i1;
-  a.sj0 = b.src.j0;
-  a.sj1 = b.src.j1;
-  a.g = b.src.g;
-  a.s1 = sc.s1;
-  a.s2 = sc.s2;
-  a.he = sc.he;
-  a.h = (T)sc.h;
-  a.b = (T)sc.b;
-  a.a = (T)sc.a;
-  a.fdw = h->fdw;
-  return a;
 }
 
 template <typename T>
@@ -1405,29 +1199,24 @@ hipError_t fused_filter(hipStream_t s, lee_handle *h, Block &b, int src, int dst
 
 // ------------------------------------------------------------ batched ensemble
 
-// A device table as a constant-address-space pointer (the kernels' view).
-template <typename P>
-static const LEE_CONST_AS P *CA(const P *p) {
-  return (const LEE_CONST_AS P *)p;
-}
-
 void batch_release(lee_handle *h) {
   BatchPlan &p = h->bp;
   if (p.exec) (void)hipGraphExecDestroy(p.exec);
   p.exec = nullptr;
-  for (void *q : {p.stage_args, p.filter_args, (void *)p.tile_map_stage, (void *)p.tile_map_filter})
+  for (void *q : {p.stage_args, p.filter_args, p.pair_args, (void *)p.tile_map_stage, (void *)p.tile_map_filter,
+                  (void *)p.tile_map_pair})
     if (q) (void)hipFree(q);
-  p.stage_args = p.filter_args = nullptr;
-  p.tile_map_stage = p.tile_map_filter = nullptr;
+  p.stage_args = p.filter_args = p.pair_args = nullptr;
+  p.tile_map_stage = p.tile_map_filter = p.tile_map_pair = nullptr;
   p.ready = false;
 }
 
 // Uploads the per-solve operand tables of every stage and of the filter for
 // the current tile shape, and the tile prefix sums.  The schedule and the
 // step counter are allocated by the caller.
-// With p.tuning the tables describe runs on scratch buffers only (every
-// stage: the right-hand-side form, Y2 -> Y3 and Y1; filter: Y1 -> Y2), so
-// the autotuner can time launches without touching the state in Y0.
+// With p.tuning the tables describe runs on scratch buffers only (stages: Y2
+// -> Y3 and Y1; filter: Y1 -> Y2), so the autotuner can time launches without
+// touching the state in Y0.
 template <typename T>
 static void batch_resident_t(lee_handle *h);
 
@@ -1444,7 +1233,7 @@ static hipError_t batch_prepare_t(hipStream_t s, lee_handle *h) {
     T *const *Y = sizeof(T) == 8 ? (T *const *)b.Y64 : (T *const *)b.Y32;
     T *rho = sizeof(T) == 8 ? (T *)b.rho64 : (T *)b.rho32;
     for (int st = 0; st < S; st++)
-      sa[(size_t)st * ns + k] = make_stage_args<T>(h, b, p.tuning ? -1 : st, Y, rho, p.R, zero);
+      sa[(size_t)st * ns + k] = make_stage_args<T>(h, b, p.tuning ? (st == 0 ? -2 : (st == S - 1 ? -3 : -1)) : st, Y, rho, p.R, zero);
     fa[k] = make_filter_args<T>(h, b, Y, 1, p.tuning ? 2 : 0, p.TY);
     if (p.stack) {  // stacks of four waves of p.stack rows, four variables
       fa[k].ntx = (b.ni + March::STRIDE - 1) / March::STRIDE;
@@ -1484,8 +1273,8 @@ static hipError_t batch_prepare_t(hipStream_t s, lee_handle *h) {
 
 hipError_t batch_prepare(hipStream_t s, lee_handle *h) {
   batch_release(h);
-  if (h->cfg.precision == LEE_FP32) return batch_prepare_t<float>(s, h);
-  return batch_prepare_t<double>(s, h);
+  const hipError_t e = h->cfg.precision == LEE_FP32 ? batch_prepare_t<float>(s, h) : batch_prepare_t<double>(s, h);
+  return e == hipSuccess && h->bp.pair ? batch_pair_prepare(s, h) : e;
 }
 
 // Grid of a batch launch over `total` list entries: one workgroup per entry
@@ -1584,7 +1373,7 @@ static hipError_t batch_stage_t(hipStream_t s, lee_handle *h, int stage) {
   ba.chunk = (p.total_stage + 7) / 8;
   ba.b = (T)h->b_i[stage];
   ba.a = (T)h->a_next[stage];
-  const int kind = p.tuning ? STAGE_MID : stage_kind(h, stage);
+  const int kind = stage_kind(h, stage);
   const unsigned g = batch_grid(p.total_stage, p.grid_stage, p.res_stage);
   const bool queued = g < 8u * (unsigned)ba.chunk;
   const dim3 grid(g), block(64, 4);

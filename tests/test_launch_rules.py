@@ -90,3 +90,66 @@ def test_plain_stage_tile_edges(shape, order):
     s.solve(6)
     assert np.array_equal(s.solution(), o.solution(0)[:, 0])
     s.close()
+
+
+def _pair_case(ni, nj, kind, seed):
+    """A 2-D block whose sponges overlap in the corners, with a source inside
+    one of them; kind: "sponges" (uniform mean), "sheared", "faces" (a BC on
+    every side, meeting in the corners) or "wave" (a harmonic face and zone)."""
+    rng = np.random.default_rng(seed)
+    i, j = np.meshgrid(np.arange(ni), np.arange(nj))
+    x, y = 0.5 * i + 0.1 * np.sin(0.7 * j), 0.5 * j + 0.1 * np.sin(0.4 * i)
+    mean = np.zeros((5, nj, ni))
+    mean[1], mean[2] = 0.3, -0.1
+    mean[4] = 1.0 / GAMMA
+    if kind in ("sheared", "faces"):
+        mean[0] = 0.05 * np.cos(0.3 * x)
+        mean[1] = 0.2 * np.tanh(0.5 * (y - y.mean()))
+        mean[4] = (1.0 + 0.05 * np.sin(0.2 * x + 0.3 * y)) / GAMMA
+    ic = 1e-4 * rng.standard_normal((5, nj, ni))
+    ic[3] = 0.0
+    bc = [(0, "sponge_freund_ambient", "+xi", "0", "6", "0", "-0", "0", "0"),
+          (0, "sponge_freund_ambient", "+eta", "0", "-0", "0", "5", "0", "0"),
+          (0, "sponge_freund_ambient", "-eta", "0", "-0", "-4", "-0", "0", "0")]
+    harmonic = None
+    if kind == "faces":
+        bc = [(0, "wall_slip_kinematic", "+eta", "0", "-0", "0", "0", "0", "0"),
+              (0, "neumann", "+xi", "0", "0", "0", "-0", "0", "0"),
+              (0, "dirichlet_allzero", "-xi", "-0", "-0", "2", "-3", "0", "0"),
+              (0, "wall_slip_kinematic", "-eta", "0", "-0", "-0", "-0", "0", "0")]
+    if kind == "wave":
+        bc = [(0, "dirichlet_harmonicwave", "+xi", "0", "0", "0", "-0", "0", "0"),
+              (0, "sponge_freund_harmonicwave", "+xi", "0", "6", "0", "-0", "0", "0"),
+              (0, "sponge_freund_ambient", "-eta", "0", "-0", "-4", "-0", "0", "0")]
+        harmonic = dict(wave="WAVE_ENTROPY", shape="WAVEFORM_GAUSSIAN_ROUNDJET", direction="X", amplitude=0.02,
+                        wavelength=5.0, halfwidth=1.5)
+    src = (1e-3, 0.6, float(x[2, 3]), float(y[2, 3]), 0.0, 1.0)
+    return dict(x=x, y=y, mean=mean), ic, dict(boundaries=bc, harmonic=harmonic, simulation="CASE_MONOPOLE",
+                                               source_params=src, mode="FIX_CFL", value=0.4)
+
+
+# tiles of 60 x 4 and 60 x 12 points: one point past a tile, one short of it,
+# blocks narrower than a tile's halo, and one with tiles inside the block
+@pytest.mark.parametrize("shape", [(61, 13), (60, 12), (59, 25), (9, 9), (9, 131), (181, 121), (721, 500)])
+@pytest.mark.parametrize("kind", ["sponges", "sheared", "faces", "wave"])
+@pytest.mark.parametrize("prec", [FP64, FP32])
+def test_paired_stages_bit_identical(shape, kind, prec):
+    """Two RK stages a launch, as the tuner picks them, against one stage a
+    launch (a pinned tile shape), bit for bit after 5 steps."""
+    block, ic, kw = _pair_case(*shape, kind, seed=11)
+    out = []
+    for pinned in (False, True):
+        s = Solver([block], precision=prec, **kw)
+        s.set_solution(ic)
+        if pinned:
+            s.set_tile_shape(1, 4)
+        else:
+            s.autotune()
+            s.set_kernel_timing(True)
+        s.solve(5)
+        if not pinned:
+            print(shape, kind, prec, "launches", {k: v[1] for k, v in s.kernel_timing().items()}, flush=True)
+        out.append((s.solution(), s.clock()))
+        s.close()
+    assert np.all(np.isfinite(out[0][0]))
+    assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
