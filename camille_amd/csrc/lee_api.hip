@@ -1317,6 +1317,13 @@ int create_impl(const lee_config *cfgs, int cfg_stride, const lee_block *blocks,
           mc[(size_t)MC3_RP * n + p] = rb * gi / pb;
           mc[(size_t)MC3_RB * n + p] = rb;
         }
+        if (D == 3) {
+          b.mc_varies = 0;
+          for (int f = 0; f < MC3_COUNT; f++) {
+            const double *c = mc.data() + (size_t)f * n;
+            if (std::any_of(c + 1, c + n, [c](double v) { return !(v == c[0]); })) b.mc_varies |= 1u << f;
+          }
+        }
         for (int p = 0; D == 2 && p < n; p++) {
           const double pb = in.mean[(size_t)IP * n + p];
           const double rb = std::pow(gam * pb, gi) * std::exp(-in.mean[(size_t)IS * n + p]);

@@ -124,6 +124,68 @@ __device__ __forceinline__ T fd_row(const T *s, int st, int code) {
   }
 }
 
+// An OA4 row as four products in fd_row's order: the neighbours' offsets and
+// their weights, the last one or two 0 (on a neighbour already in the sum) in
+// a closure row.  A lane near an end of its line runs the same instructions as
+// its neighbours instead of a branch per row kind, each waiting for LDS: the
+// rows of a tile on the block's edge took 5800 cycles, this way ROW_CYC.
+template <typename T>
+struct Row4 {
+  int o[4];
+  T w[4];
+};
+template <typename T>
+__device__ __forceinline__ Row4<T> row4(int code) {
+  const T c1 = (T)(8.0 / 12.0), c2 = (T)(-1.0 / 12.0);
+  Row4<T> r{{-2, -1, 1, 2}, {-c2, -c1, c1, c2}};
+  if (code == CODE_LEFT + 0) r = {{0, 1, 2, 2}, {(T)-1.5, (T)2.0, (T)-0.5, (T)0}};
+  if (code == CODE_LEFT + 1) r = {{-1, 1, 1, 1}, {(T)-0.5, (T)0.5, (T)0, (T)0}};
+  if (code == CODE_LEFT + 2) r = {{0, -1, -2, -2}, {(T)1.5, (T)-2.0, (T)0.5, (T)0}};
+  if (code == CODE_LEFT + 3) r = {{1, -1, -1, -1}, {(T)0.5, (T)-0.5, (T)0, (T)0}};
+  return r;
+}
+template <typename T>
+__device__ __forceinline__ T row4_sum(const Row4<T> &r, const T *s, int st) {
+#pragma clang fp contract(off)
+  T acc = r.w[0] * s[r.o[0] * st];
+  acc = fmx(r.w[1], s[r.o[1] * st], acc);
+  acc = fmx(r.w[2], s[r.o[2] * st], acc);
+  return fmx(r.w[3], s[r.o[3] * st], acc);
+}
+
+// Weights of the transposed OA4 rows at coordinate c of a line of length len
+// without holes: (D^T f)_c = sum_o w[o + 2] f_{c+o}, 0 for neighbours off the
+// line.  Formed once per lane and line, so that tiles at a block's edge run
+// the sums of its inside.
+template <typename T>
+struct RowT5 {
+  T w[5];
+};
+template <typename T>
+__device__ __forceinline__ RowT5<T> row_t5(int c, int len) {
+  RowT5<T> r;
+#pragma unroll
+  for (int o = -2; o <= 2; o++) {
+    const int j = c + o;
+    // the row at j puts weight row4 of its code on offset -o
+    const Row4<T> q = row4<T>(default_code(j, len, 2));
+    T w = (T)0;
+#pragma unroll
+    for (int e = 0; e < 4; e++) w += q.o[e] == -o ? q.w[e] : (T)0;
+    r.w[o + 2] = j >= 0 && j < len ? w : (T)0;
+  }
+  return r;
+}
+template <typename T>
+__device__ __forceinline__ T row_t5_sum(const RowT5<T> &r, const T *f, int st) {
+  T acc = r.w[0] * f[-2 * st];
+  acc += r.w[1] * f[-st];
+  acc += r.w[2] * f[0];
+  acc += r.w[3] * f[st];
+  acc += r.w[4] * f[2 * st];
+  return acc;
+}
+
 template <typename T>
 struct ZoneT {
   int i0, i1, j0, j1, nzi;
@@ -171,6 +233,30 @@ inline int z_chunk(int tiles, int nk, int most, int cus) {
   for (int zc = most; zc > 1; zc--)
     if ((long long)tiles * ((nk + zc - 1) / zc) >= 2LL * cus) return zc;
   return 1;
+}
+
+// Bit z set where zone z meets the box (uniform over the workgroup): the boxes
+// are read at fixed places, all at once, and the planes visit only zones that
+// can reach them.
+template <typename Z>
+__device__ __forceinline__ unsigned zones_meeting3(const Z (&z)[MAX_ZONES], int nz, int i0, int i1, int j0, int j1, int k0,
+                                                   int k1) {
+  unsigned m = 0;
+#pragma unroll
+  for (int q = 0; q < MAX_ZONES; q++)
+    m |= q < nz && z[q].i0 <= i1 && z[q].i1 >= i0 && z[q].j0 <= j1 && z[q].j1 >= j0 && z[q].k0 <= k1 && z[q].k1 >= k0
+             ? 1u << q : 0;
+  return m;
+}
+
+// Mean coefficient field f of a 3-D block at point p.  A parallel jet, the
+// usual base flow, varies in few of the 22 fields (v, w, s, p and their
+// gradients are constant): a constant field is read at its first point by
+// every lane, which costs a cache hit instead of memory traffic and gives the
+// same value.  varies: Block::mc_varies (uniform).
+template <typename T>
+__device__ __forceinline__ T mean_field3(const T *mc, unsigned varies, int f, size_t n, size_t p) {
+  return mc[(size_t)f * n + (varies >> f & 1 ? p : 0)];
 }
 
 // One RK stage on a 64 x TY tile.  Every global operand of the thread (its

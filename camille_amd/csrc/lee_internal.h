@@ -94,6 +94,7 @@ struct Block {
   // non-uniform mean: MC_COUNT coefficient fields in the bulk type
   double *mc64 = nullptr;
   float *mc32 = nullptr;
+  unsigned mc_varies = ~0u;    // 3-D: bit f set where coefficient field f is not one value throughout
   // aux density rho' carried between steps (stale after the filter)
   double *rho64 = nullptr;
   float *rho32 = nullptr;

@@ -16,6 +16,7 @@
 // the blend.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include "lee_device.h"
@@ -26,19 +27,20 @@ namespace lee {
 namespace {
 
 constexpr int S3_TY = 4;      // tile rows in j
-#ifndef LEE_Z_CHUNK
-#define LEE_Z_CHUNK 32
-#endif
-constexpr int Z_CHUNK = LEE_Z_CHUNK;  // planes per z chunk
 // Planes per workgroup of the stage.  A workgroup's planes are one serial
 // chain (loads, barrier, arithmetic, stores: about 5 us a plane), and the
 // four window planes that the next chunk reads again are in its XCD's L2,
-// so short chunks win at every size, FP32 / FP64 middle stage: 48 x 40 x 32
+// so short chunks win at every size, FP32 / FP64 middle stage as measured
+// before the mean fields' and closure rows' changes below: 48 x 40 x 32
 // 176 / 229 us with 32 planes, 25 / 33 with 4, 15 / 19 with 2, 10 / 14 with
 // 1; 144 x 120 x 112 218 / 376, 131 / 258, 128 / 247, 131 / 259;
 // 256 x 200 x 256 857 / 1599, 723 / 1338, 717 / 1329, 728 / 1386.
 constexpr int STAGE_Z_CHUNK = 2;
-constexpr int FUSED_Z_CHUNK = 64;     // planes per chunk of the single-pass filter (4 halo planes a side)
+// Most planes per chunk of the single-pass filter (4 halo planes a side) and
+// of the two-pass form's column pass; smaller blocks take fewer, at least 16
+// and 4 (z_chunk).  With 64 and 32 whatever the block, the filter of a
+// 48 x 40 x 32 block took 33 us in FP32 for 1 us of traffic, now 14; 112 x 96 x 80 48, now 37.
+constexpr int FUSED_Z_CHUNK = 64, COLUMN_Z_CHUNK = 16;
 
 inline unsigned nb3(size_t n) { return (unsigned)((n + TPB - 1) / TPB); }
 
@@ -115,6 +117,7 @@ struct Stage3Args {
   T *acc, *yout;
   const double *met, *jac;
   const T *mc;                      // non-uniform mean: MC3_COUNT fields
+  unsigned varies;                  // and which of them are not constant
   const T *rho_in;
   T *rho_out;
   double u0, v0, w0, gp0, rhob0, gamma;
@@ -127,8 +130,15 @@ struct Stage3Args {
 };
 
 // One RK stage on a 64 x 4 column tile through a chunk of zc planes.
+// What bounds it: HBM at large blocks (256 x 200 x 256 FP32, a parallel jet:
+// 208 of the 268 bytes a point left once constant mean fields are read from
+// cache, 583 us, 4.7 TB/s of the 4.9 a large copy reaches; 717 us before).
+// Closure rows without branches (Row4) and zone boxes read once: middle stage
+// at 144 x 120 x 112 FP32 128 -> 104 us, FP64 247 -> 230.
+// (FP64 is held to two waves per SIMD: left alone, the middle stage takes so
+// many registers that one fits.)
 template <typename T, bool MEANF, int KIND>
-__global__ void __launch_bounds__(TPB) k_stage3d(Stage3Args<T> a) {
+__global__ void __launch_bounds__(TPB, sizeof(T) == 8 ? 2 : 3) k_stage3d(Stage3Args<T> a) {
   constexpr int RS = ST_TX + 2 * ST_H, NR = S3_TY + 2 * ST_H;
   __shared__ T s[5][NR][RS];
   // within each z chunk, XCD x (workgroups x mod 8 of a grid row that is a
@@ -137,7 +147,7 @@ __global__ void __launch_bounds__(TPB) k_stage3d(Stage3Args<T> a) {
   const int ntl = a.ntx * a.nty;
   const int tile = xcd_tile(blockIdx.x, (ntl + 7) / 8);
   if (tile >= ntl) return;
-  const int tx = threadIdx.x, ty = threadIdx.y;
+  const int tx = threadIdx.x, ty = __builtin_amdgcn_readfirstlane((int)threadIdx.y);  // a wave is one row
   const int i0 = (tile % a.ntx) * ST_TX, j0 = (tile / a.ntx) * S3_TY;
   const int k0 = blockIdx.y * a.zc, k1 = min(k0 + a.zc, a.nk);
   const int ni = a.ni, nj = a.nj, nk = a.nk;
@@ -145,6 +155,8 @@ __global__ void __launch_bounds__(TPB) k_stage3d(Stage3Args<T> a) {
   const int gi = i0 + tx, gj = j0 + ty;
   const bool own = gi < ni && gj < nj;
   const size_t col = own ? (size_t)gj * ni + gi : 0;
+  const Row4<T> rx = row4<T>(default_code(gi, ni, 2)), ry = row4<T>(default_code(gj, nj, 2));
+  const unsigned zmask = zones_meeting3(a.z, a.nz, i0, i0 + ST_TX - 1, j0, j0 + S3_TY - 1, k0, k1 - 1);
   // register window of the own column: planes k - 2 .. k + 2
   T w[5][5];
 #pragma unroll
@@ -199,7 +211,7 @@ __global__ void __launch_bounds__(TPB) k_stage3d(Stage3Args<T> a) {
     if (MEANF) {
 #pragma unroll
       for (int f = 0; f < MC3_COUNT; f++)
-        mcv[f] = (f < MC3_RP || KIND != STAGE_FIRST) ? a.mc[(size_t)f * n + p] : (T)0;
+        mcv[f] = (f < MC3_RP || KIND != STAGE_FIRST) ? mean_field3(a.mc, a.varies, f, n, p) : (T)0;
     }
     const T rho_first = (MEANF && KIND == STAGE_FIRST) ? a.rho_in[p] : (T)0;
     T accp[5], ynp[5];
@@ -219,14 +231,14 @@ __global__ void __launch_bounds__(TPB) k_stage3d(Stage3Args<T> a) {
     }
     __syncthreads();
     if (own) {
-      const int cx = default_code(gi, ni, 2), cy = default_code(gj, nj, 2), cz = default_code(k, nk, 2);
+      const int cz = default_code(k, nk, 2);
       T d[5][3], yc[5];
 #pragma unroll
       for (int v = 0; v < 5; v++) {
         const T *sp = &s[v][ty + ST_H][tx + ST_H];
         yc[v] = w[v][2];
-        d[v][0] = fd_row<T>(sp, 1, cx);
-        d[v][1] = fd_row<T>(sp, RS, cy);
+        d[v][0] = row4_sum<T>(rx, sp, 1);
+        d[v][1] = row4_sum<T>(ry, sp, RS);
         d[v][2] = fd_row<T>(&w[v][2], 1, cz);
       }
       T f[5][3];  // f[v][x_i] = d var / d x_i
@@ -304,9 +316,8 @@ __global__ void __launch_bounds__(TPB) k_stage3d(Stage3Args<T> a) {
             a.g[((size_t)(k - a.sk0) * (a.sj1 - a.sj0 + 1) + (gj - a.sj0)) * (a.si1 - a.si0 + 1) + (gi - a.si0)];
         r[IP] += (T)(a.s1 * gval * a.s2);
       }
-#pragma unroll 1
-      for (int z = 0; z < a.nz; z++) {
-        const Zone3<T> &zz = a.z[z];
+      for (unsigned zm = zmask; zm; zm &= zm - 1) {
+        const Zone3<T> &zz = a.z[__builtin_ctz(zm)];
         if (gi >= zz.i0 && gi <= zz.i1 && gj >= zz.j0 && gj <= zz.j1 && k >= zz.k0 && k <= zz.k1) {
           const T sg = zz.sig[((size_t)(k - zz.k0) * zz.nzj + (gj - zz.j0)) * zz.nzi + (gi - zz.i0)];
 #pragma unroll
@@ -542,12 +553,13 @@ __global__ void __launch_bounds__(TPB) k_filter3d_fused(FilterArgs<T> a, int nk,
 // planes (9-plane register window), blend with y, into dst.
 template <typename T, int ORDER>
 __global__ void __launch_bounds__(TPB) k_filter3d_z(const T *__restrict__ tmp, const T *__restrict__ y,
-                                                    T *__restrict__ dst, int ni, int nj, int nk, T rem, T blend) {
+                                                    T *__restrict__ dst, int ni, int nj, int nk, int zc, T rem,
+                                                    T blend) {
   constexpr int H = FL_H, NB = ORDER / 2;
   const size_t plane = (size_t)ni * nj, n = plane * nk;
   const size_t col = (size_t)blockIdx.x * TPB + threadIdx.x;
   if (col >= plane) return;
-  const int k0 = blockIdx.y * Z_CHUNK, k1 = min(k0 + Z_CHUNK, nk);
+  const int k0 = blockIdx.y * zc, k1 = min(k0 + zc, nk);
   T w[5][2 * H + 1];
 #pragma unroll
   for (int q = 0; q < 2 * H; q++) {
@@ -656,6 +668,7 @@ static hipError_t stage3d_t(hipStream_t s, lee_handle *h, Block &b, int stage, c
   a.met = b.met;
   a.jac = b.jac;
   a.mc = sizeof(T) == 8 ? (const T *)b.mc64 : (const T *)b.mc32;
+  a.varies = b.mc_varies;
   a.rho_in = rho;
   a.rho_out = rho;
   a.u0 = b.umean[IUX];
@@ -735,7 +748,7 @@ static hipError_t filter3d_t(hipStream_t s, lee_handle *h, Block &b, T *const *Y
     a.nty = (b.nj + TY - 1) / TY;
     a.ntiles = 5 * a.ntx * a.nty;
     a.chunk = (a.ntiles + 7) / 8;
-    const int zc = FUSED_Z_CHUNK;
+    const int zc = std::max(16, z_chunk(a.chunk * 8, b.nk, FUSED_Z_CHUNK, b.cus));
     const dim3 grid(a.chunk * 8, (b.nk + zc - 1) / zc), block(64, 4);
 #define LEE_F3F(OR)                                                                                      \
   do {                                                                                                   \
@@ -768,10 +781,11 @@ static hipError_t filter3d_t(hipStream_t s, lee_handle *h, Block &b, T *const *Y
     if (o8) hipLaunchKernelGGL((k_filter3d_plane<T, 8, TYF>), grid, block, 0, s, a, plane);
     else hipLaunchKernelGGL((k_filter3d_plane<T, 4, TYF>), grid, block, 0, s, a, plane);
   }
-  const dim3 gz(nb3(plane), (b.nk + Z_CHUNK - 1) / Z_CHUNK);
+  const int zz = std::max(4, z_chunk((int)nb3(plane), b.nk, COLUMN_Z_CHUNK, b.cus));
+  const dim3 gz(nb3(plane), (b.nk + zz - 1) / zz);
   const T blend = (T)h->cfg.filter_blend, rem = (T)(1.0 - h->cfg.filter_blend);
-  if (o8) hipLaunchKernelGGL((k_filter3d_z<T, 8>), gz, dim3(TPB), 0, s, Y[tmp], Y[src], Y[dst], b.ni, b.nj, b.nk, rem, blend);
-  else hipLaunchKernelGGL((k_filter3d_z<T, 4>), gz, dim3(TPB), 0, s, Y[tmp], Y[src], Y[dst], b.ni, b.nj, b.nk, rem, blend);
+  if (o8) hipLaunchKernelGGL((k_filter3d_z<T, 8>), gz, dim3(TPB), 0, s, Y[tmp], Y[src], Y[dst], b.ni, b.nj, b.nk, zz, rem, blend);
+  else hipLaunchKernelGGL((k_filter3d_z<T, 4>), gz, dim3(TPB), 0, s, Y[tmp], Y[src], Y[dst], b.ni, b.nj, b.nk, zz, rem, blend);
   return hipGetLastError();
 }
 

@@ -114,35 +114,6 @@ __device__ __forceinline__ void st_off(U *base, unsigned off, U v) {
   *(U *)((char *)base + off) = v;
 }
 
-// An OA4 row as four products in fd_row's order: the neighbours' offsets and
-// their weights, the last one or two 0 (on a neighbour already in the sum) in
-// a closure row.  A lane near an end of its line runs the same instructions as
-// its neighbours instead of a branch per row kind, each waiting for LDS: the
-// rows of a tile on the block's edge took 5800 cycles, this way ROW_CYC.
-template <typename T>
-struct Row4 {
-  int o[4];
-  T w[4];
-};
-template <typename T>
-__device__ __forceinline__ Row4<T> row4(int code) {
-  const T c1 = (T)(8.0 / 12.0), c2 = (T)(-1.0 / 12.0);
-  Row4<T> r{{-2, -1, 1, 2}, {-c2, -c1, c1, c2}};
-  if (code == CODE_LEFT + 0) r = {{0, 1, 2, 2}, {(T)-1.5, (T)2.0, (T)-0.5, (T)0}};
-  if (code == CODE_LEFT + 1) r = {{-1, 1, 1, 1}, {(T)-0.5, (T)0.5, (T)0, (T)0}};
-  if (code == CODE_LEFT + 2) r = {{0, -1, -2, -2}, {(T)1.5, (T)-2.0, (T)0.5, (T)0}};
-  if (code == CODE_LEFT + 3) r = {{1, -1, -1, -1}, {(T)0.5, (T)-0.5, (T)0, (T)0}};
-  return r;
-}
-template <typename T>
-__device__ __forceinline__ T row4_sum(const Row4<T> &r, const T *s, int st) {
-#pragma clang fp contract(off)
-  T acc = r.w[0] * s[r.o[0] * st];
-  acc = fmx(r.w[1], s[r.o[1] * st], acc);
-  acc = fmx(r.w[2], s[r.o[2] * st], acc);
-  return fmx(r.w[3], s[r.o[3] * st], acc);
-}
-
 template <typename T, int RA>
 using PairLds = T[4][P2_WAVES * RA + 4][68];
 

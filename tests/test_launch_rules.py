@@ -14,8 +14,9 @@ def _rel(a, b):
     return float(np.max(np.abs(a - b)) / max(np.max(np.abs(b)), 1e-300))
 
 
-def _box3(ni, nj, nk, seed):
-    """A stretched 3-D box with a sheared, non-constant base flow and a rough state."""
+def _box3(ni, nj, nk, seed, flow="general"):
+    """A stretched 3-D box with a rough state and a base flow: "general" varies
+    in every field, "jet" only in u(y, z), "rotor" in u and p."""
     rng = np.random.default_rng(seed)
     k, j, i = np.meshgrid(np.arange(nk), np.arange(nj), np.arange(ni), indexing="ij")
     x, y, z = (0.25 * a + 0.05 * np.sin(0.3 * a) for a in (i, j, k))
@@ -25,19 +26,27 @@ def _box3(ni, nj, nk, seed):
     mean[2] = 0.1 * np.cos(0.3 * z)
     mean[3] = 0.05 * np.sin(0.25 * x + 0.2 * y)
     mean[4] = (1.0 + 0.1 * np.cos(0.2 * z + 0.1 * x)) / GAMMA
+    if flow != "general":
+        mean[0], mean[2], mean[3] = 0.0, 0.1, 0.0
+        mean[1] = 0.3 * np.tanh(0.4 * (y - y.mean())) * np.cos(0.2 * z)
+    if flow == "jet":
+        mean[4] = 1.0 / GAMMA
     return x, y, z, mean, rng.standard_normal((5, nk, nj, ni)), rng.standard_normal((5, nk, nj, ni))
 
 
 # (131, 61, 45) takes chunks of 2 planes forwards and 4 backwards, one plane
 # left over; (70, 13, 9) and (9, 9, 14) take single planes
 @pytest.mark.parametrize("dims", [(131, 61, 45), (70, 13, 9), (9, 9, 14)])
+@pytest.mark.parametrize("flow", ["general", "jet", "rotor"])
 @pytest.mark.parametrize("prec,tol", [(FP64, 1e-12), (FP32, 2e-5)])
-def test_3d_stage_chunks(dims, prec, tol):
+def test_3d_stage_chunks(dims, flow, prec, tol):
     """The 3-D right-hand side equals its definition, built from the FP64
     derivative entry point, and its transpose satisfies <L y, k> = <y, L^T k>.
     FP32: some 40 terms of size 1 to 10, each rounded at 6e-8, relative to
-    the largest value; the dot products gather random signs and stay below."""
-    x, y, z, mean, q, kap = _box3(*dims, seed=3)
+    the largest value; the dot products gather random signs and stay below.
+    The flows differ in which mean coefficient fields are constant and so read
+    at one point."""
+    x, y, z, mean, q, kap = _box3(*dims, seed=3, flow=flow)
     s = Solver([dict(x=x, y=y, z=z, mean=mean)], precision=prec, mode="FIX_DT", value=0.01, num_dim=3)
     d = [[s.take_derivative_xyz(f, i) for i in range(3)] for f in q]
     g = [[s.take_derivative_xyz(f, i) for i in range(3)] for f in mean]
