@@ -16,6 +16,7 @@
 // pass with the blend and R^T mu.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cmath>
 
 #include "lee_device.h"
@@ -26,7 +27,7 @@ namespace lee {
 namespace {
 
 constexpr int A3_TY = 4;
-constexpr int A3_ZC = 32;      // planes per chunk of the zeta^T filter pass
+constexpr int A3_ZC = 16;      // most planes per chunk of the zeta^T filter pass (at least 4, z_chunk)
 // Planes per workgroup of the adjoint stage (see STAGE_Z_CHUNK of the
 // forward stage; here a chunk's four extra planes cost a flux evaluation
 // each, so 4 planes instead of 2).  Whole reverse step (recomputed forward
@@ -37,46 +38,6 @@ constexpr int A3_ZC = 32;      // planes per chunk of the zeta^T filter pass
 constexpr int ADJ_Z_CHUNK = 4;
 
 inline unsigned nba(size_t n) { return (unsigned)((n + TPB - 1) / TPB); }
-
-template <typename T>
-__device__ __forceinline__ T fd_wt3(int code, int d) {
-  const T c1 = (T)(8.0 / 12.0), c2 = (T)(-1.0 / 12.0);
-  switch (code) {
-    case CODE_INTERIOR:
-      return d == -2 ? -c2 : d == -1 ? -c1 : d == 1 ? c1 : d == 2 ? c2 : (T)0;
-    case CODE_ZERO:
-      return (T)0;
-    case CODE_LEFT + 0:
-      return d == 0 ? (T)(-3.0 / 2.0) : d == 1 ? (T)(4.0 / 2.0) : d == 2 ? (T)(-1.0 / 2.0) : (T)0;
-    case CODE_LEFT + 1:
-      return d == -1 ? (T)(-1.0 / 2.0) : d == 1 ? (T)(1.0 / 2.0) : (T)0;
-    case CODE_LEFT + 2:
-      return d == 0 ? (T)(3.0 / 2.0) : d == -1 ? (T)(-4.0 / 2.0) : d == -2 ? (T)(1.0 / 2.0) : (T)0;
-    default:
-      return d == 1 ? (T)(1.0 / 2.0) : d == -1 ? (T)(-1.0 / 2.0) : (T)0;
-  }
-}
-
-// (D^T f) at coordinate c of a line of length len: rows of the neighbours.
-template <typename T>
-__device__ __forceinline__ T fd_t3(const T *f, int st, int c, int len) {
-  if (c >= 4 && c <= len - 5) {  // every neighbour row is interior: D^T = -D
-    const T c1 = (T)(8.0 / 12.0), c2 = (T)(-1.0 / 12.0);
-    T acc = c2 * f[-2 * st];
-    acc += c1 * f[-st];
-    acc += -c1 * f[st];
-    acc += -c2 * f[2 * st];
-    return acc;
-  }
-  T acc = 0;
-#pragma unroll
-  for (int o = -2; o <= 2; o++) {
-    const int j = c + o;
-    if (j < 0 || j >= len) continue;
-    acc += fd_wt3<T>(default_code(j, len, 2), -o) * f[o * st];
-  }
-  return acc;
-}
 
 template <typename T, int ORDER>
 __device__ __forceinline__ T flt_wt3(int code, int d) {
@@ -134,6 +95,7 @@ struct Adj3Args {
   double *grad;
   const double *met, *jac;
   const T *mc;               // MC3_COUNT coefficient fields (non-uniform mean)
+  unsigned varies;           // and which of them are not constant
   double u0, v0, w0, gp0, rhob0, gamma;
   int nz;
   Zone3A<T> z[MAX_ZONES];
@@ -152,37 +114,38 @@ __device__ __forceinline__ void adj_flux3(const Adj3Args<T> &a, size_t p, size_t
   }
   double ub[3] = {a.u0, a.v0, a.w0}, gp = a.gp0, irb = 1.0 / a.rhob0;
   if (MEANF) {
-    ub[0] = a.mc[MC3_U * n + p];
-    ub[1] = a.mc[MC3_V * n + p];
-    ub[2] = a.mc[MC3_W * n + p];
-    gp = a.mc[MC3_GP * n + p];
-    irb = a.mc[MC3_IRB * n + p];
+    ub[0] = mean_field3(a.mc, a.varies, MC3_U, n, p);
+    ub[1] = mean_field3(a.mc, a.varies, MC3_V, n, p);
+    ub[2] = mean_field3(a.mc, a.varies, MC3_W, n, p);
+    gp = mean_field3(a.mc, a.varies, MC3_GP, n, p);
+    irb = mean_field3(a.mc, a.varies, MC3_IRB, n, p);
   }
-  double A[3][5];
-#pragma unroll
-  for (int d = 0; d < 3; d++) {
-    A[d][IS] = -ub[d] * (double)kap[IS];
-#pragma unroll
-    for (int i = 0; i < 3; i++) A[d][IUX + i] = -ub[d] * (double)kap[IUX + i] - (i == d ? gp * (double)kap[IP] : 0.0);
-    A[d][IP] = -ub[d] * (double)kap[IP] - (double)kap[IUX + d] * irb;
-  }
+  // F_l = -J (U_l kappa + ...) with the contravariant velocity U_l = m_l . ubar
+  const double ks = kap[IS], ku[3] = {kap[IUX], kap[IUY], kap[IUZ]}, kp = kap[IP];
+  const double c = gp * kp;
   double m[3][3];
 #pragma unroll
   for (int l = 0; l < 3; l++)
 #pragma unroll
     for (int i = 0; i < 3; i++) m[l][i] = a.met[(size_t)(3 * l + i) * n + p];
-  const double J = a.jac[p];
+  const double J = -a.jac[p];
 #pragma unroll
-  for (int l = 0; l < 3; l++)
+  for (int l = 0; l < 3; l++) {
+    const double U = m[l][0] * ub[0] + m[l][1] * ub[1] + m[l][2] * ub[2];
+    F[l][IS] = (T)(U * ks * J);
 #pragma unroll
-    for (int v = 0; v < 5; v++) {
-      double f = 0.0;
-#pragma unroll
-      for (int d = 0; d < 3; d++) f += m[l][d] * A[d][v];
-      F[l][v] = (T)(f * J);
-    }
+    for (int i = 0; i < 3; i++) F[l][IUX + i] = (T)((U * ku[i] + m[l][i] * c) * J);
+    F[l][IP] = (T)((U * kp + (m[l][0] * ku[0] + m[l][1] * ku[1] + m[l][2] * ku[2]) * irb) * J);
+  }
 }
 
+// What bounds it: latency and FP64 arithmetic (a flux evaluation is some 75
+// FP64 operations, 3.1 of them a point with the halo) more than its 268 bytes
+// a point.  Fluxes through the contravariant velocity (19 operations a
+// direction instead of 29), the halo's points spread over the workgroup, the
+// point's own operands requested before the barrier and transposed closure
+// rows without branches: whole reverse step, FP32 / FP64, 112 x 96 x 80 836 /
+// 1238 -> 607 / 1106 us, 256 x 200 x 256 9632 / 16118 -> 8145 / 14972.
 template <typename T, bool MEANF, int KIND>
 __global__ void __launch_bounds__(TPB) k_adj_stage3d(Adj3Args<T> a) {
   constexpr int RS = ST_TX + 2 * ST_H, NR = A3_TY + 2 * ST_H;
@@ -191,7 +154,7 @@ __global__ void __launch_bounds__(TPB) k_adj_stage3d(Adj3Args<T> a) {
   const int ntl = a.ntx * a.nty;
   const int tile = xcd_tile(blockIdx.x, (ntl + 7) / 8);
   if (tile >= ntl) return;
-  const int tx = threadIdx.x, ty = threadIdx.y;
+  const int tx = threadIdx.x, ty = __builtin_amdgcn_readfirstlane((int)threadIdx.y);  // a wave is one row
   const int i0 = (tile % a.ntx) * ST_TX, j0 = (tile / a.ntx) * A3_TY;
   const int k0 = blockIdx.y * a.zc, k1 = min(k0 + a.zc, a.nk);
   const int ni = a.ni, nj = a.nj, nk = a.nk;
@@ -199,6 +162,8 @@ __global__ void __launch_bounds__(TPB) k_adj_stage3d(Adj3Args<T> a) {
   const int gi = i0 + tx, gj = j0 + ty;
   const bool own = gi < ni && gj < nj;
   const size_t col = own ? (size_t)gj * ni + gi : 0;
+  const RowT5<T> rx = row_t5<T>(gi, ni), ry = row_t5<T>(gj, nj);
+  const unsigned zmask = zones_meeting3(a.z, a.nz, i0, i0 + ST_TX - 1, j0, j0 + A3_TY - 1, k0, k1 - 1);
   // zeta fluxes of the own column, planes k - 2 .. k + 2
   T wz[5][5];
 #pragma unroll
@@ -223,48 +188,61 @@ __global__ void __launch_bounds__(TPB) k_adj_stage3d(Adj3Args<T> a) {
 #pragma unroll
       for (int v = 0; v < 5; v++) wz[v][4] = F[2][v];
     }
-    // xi and eta fluxes of plane k over the tile and its halo
+    // xi and eta fluxes of plane k over the tile and its halo: its points in
+    // line order over the 256 threads, two each and 32 more (a row and its
+    // halo columns at a time cost every wave two evaluations for four lanes);
+    // points outside the block evaluate the nearest one inside and store 0
+    auto ring = [&](int idx) {
+      const int r = idx / RS, c = idx - r * RS;
+      const int rj = j0 - ST_H + r, ri = i0 - ST_H + c;
+      const bool ok = rj >= 0 && rj < nj && ri >= 0 && ri < ni;
+      T kap[5], F[3][5];
+      adj_flux3<T, MEANF, KIND>(
+          a, (size_t)k * plane + (size_t)min(max(rj, 0), nj - 1) * ni + min(max(ri, 0), ni - 1), n, kap, F);
 #pragma unroll
-    for (int mm = 0; mm < 2; mm++) {
-      const int r = ty + 4 * mm;
-      const int rj = j0 - ST_H + r;
-#pragma unroll
-      for (int half = 0; half < 2; half++) {
-        const int c = half == 0 ? tx : ST_TX + tx;
-        if (half == 1 && tx >= 2 * ST_H) continue;
-        const int ri = i0 - ST_H + c;
-        const bool ok = rj >= 0 && rj < nj && ri >= 0 && ri < ni;
-        T kap[5], F[3][5];
-        if (ok) adj_flux3<T, MEANF, KIND>(a, (size_t)k * plane + (size_t)rj * ni + ri, n, kap, F);
-#pragma unroll
-        for (int v = 0; v < 5; v++) {
-          S[v][r][c] = ok ? F[0][v] : (T)0;
-          S[5 + v][r][c] = ok ? F[1][v] : (T)0;
-        }
+      for (int v = 0; v < 5; v++) {
+        S[v][r][c] = ok ? F[0][v] : (T)0;
+        S[5 + v][r][c] = ok ? F[1][v] : (T)0;
       }
+    };
+    const int tid = ty * 64 + tx;
+    static_assert(NR * RS > 2 * TPB && NR * RS <= 3 * TPB, "two full passes and a short one");
+    ring(tid);
+    ring(tid + TPB);
+    if (tid + 2 * TPB < NR * RS) ring(tid + 2 * TPB);
+    // the own point's operands, requested before the barrier
+    const size_t p = (size_t)k * plane + col;
+    T lacc[5], lin[5], lyin[5], mcv[MC3_COUNT];
+#pragma unroll
+    for (int v = 0; v < 5; v++) {
+      lacc[v] = a.lacc[v * n + p];
+      lin[v] = (KIND != STAGE_LAST && a.lin) ? a.lin[v * n + p] : (T)0;
+      lyin[v] = KIND != STAGE_LAST && a.lyin ? a.lyin[v * n + p] : (T)0;
+    }
+    if (MEANF) {
+#pragma unroll
+      for (int f = 0; f < MC3_COUNT; f++)
+        mcv[f] = f == MC3_GP || (KIND == STAGE_FIRST && f >= MC3_RP) ? (T)0 : mean_field3(a.mc, a.varies, f, n, p);
     }
     __syncthreads();
     if (own) {
-      const size_t p = (size_t)k * plane + col;
+      const RowT5<T> rz = row_t5<T>(k, nk);  // uniform
       T lam[5];
 #pragma unroll
       for (int v = 0; v < 5; v++) {
-        lam[v] = fd_t3<T>(&S[v][ty + ST_H][tx + ST_H], 1, gi, ni);
-        lam[v] += fd_t3<T>(&S[5 + v][ty + ST_H][tx + ST_H], RS, gj, nj);
-        lam[v] += fd_t3<T>(&wz[v][2], 1, k, nk);
+        lam[v] = row_t5_sum<T>(rx, &S[v][ty + ST_H][tx + ST_H], 1);
+        lam[v] += row_t5_sum<T>(ry, &S[5 + v][ty + ST_H][tx + ST_H], RS);
+        lam[v] += row_t5_sum<T>(rz, &wz[v][2], 1);
       }
-      T kap[5], lacc[5], lin[5];
+      T kap[5];
 #pragma unroll
       for (int v = 0; v < 5; v++) {
-        lacc[v] = a.lacc[v * n + p];
-        lin[v] = (KIND != STAGE_LAST && a.lin) ? a.lin[v * n + p] : (T)0;
         T kv = (T)a.hb * lacc[v];
         if (KIND != STAGE_LAST && a.lin) kv += (T)a.ha * lin[v];
         kap[v] = kv;
       }
-#pragma unroll 1
-      for (int z = 0; z < a.nz; z++) {
-        const Zone3A<T> &zz = a.z[z];
+      for (unsigned zm = zmask; zm; zm &= zm - 1) {
+        const Zone3A<T> &zz = a.z[__builtin_ctz(zm)];
         if (gi >= zz.i0 && gi <= zz.i1 && gj >= zz.j0 && gj <= zz.j1 && k >= zz.k0 && k <= zz.k1) {
           const T sg = zz.sig[((size_t)(k - zz.k0) * zz.nzj + (gj - zz.j0)) * zz.nzi + (gi - zz.i0)];
 #pragma unroll
@@ -273,10 +251,10 @@ __global__ void __launch_bounds__(TPB) k_adj_stage3d(Adj3Args<T> a) {
       }
       T mur = 0;
       if (MEANF) {
-        const T *mc = a.mc;
-        auto G = [&](int v, int d) { return mc[(MC3_G + 3 * v + d) * n + p]; };
-        const T ub[3] = {mc[MC3_U * n + p], mc[MC3_V * n + p], mc[MC3_W * n + p]};
-        const T g = (T)a.gamma, irb = mc[MC3_IRB * n + p];
+        auto mc = [&](int f) { return mcv[f]; };
+        auto G = [&](int v, int d) { return mc(MC3_G + 3 * v + d); };
+        const T ub[3] = {mc(MC3_U), mc(MC3_V), mc(MC3_W)};
+        const T g = (T)a.gamma, irb = mc(MC3_IRB);
 #pragma unroll
         for (int d = 0; d < 3; d++) {
           T acc = G(IS, d) * kap[IS];
@@ -299,8 +277,8 @@ __global__ void __launch_bounds__(TPB) k_adj_stage3d(Adj3Args<T> a) {
         }
         mur = -(mu * irb);
         if (KIND != STAGE_FIRST) {
-          lam[IS] += -(mc[MC3_RB * n + p] * mur);
-          lam[IP] += mc[MC3_RP * n + p] * mur;
+          lam[IS] += -(mc(MC3_RB) * mur);
+          lam[IP] += mc(MC3_RP) * mur;
         }
       }
       if (a.grad) a.grad[p] += a.src * (double)kap[IP];
@@ -308,7 +286,7 @@ __global__ void __launch_bounds__(TPB) k_adj_stage3d(Adj3Args<T> a) {
 #pragma unroll
         for (int v = 0; v < 5; v++) {
           T out = lam[v] + lacc[v] + lin[v];
-          if (a.lyin) out += a.lyin[v * n + p];
+          if (a.lyin) out += lyin[v];
           a.lout[v * n + p] = out;
         }
         if (MEANF) a.mu[p] = mur;
@@ -319,7 +297,7 @@ __global__ void __launch_bounds__(TPB) k_adj_stage3d(Adj3Args<T> a) {
 #pragma unroll
           for (int v = 0; v < 5; v++) {
             T y = lin[v];
-            if (a.lyin) y += a.lyin[v * n + p];
+            if (a.lyin) y += lyin[v];
             a.lyout[v * n + p] = y;
           }
         }
@@ -336,12 +314,12 @@ __global__ void __launch_bounds__(TPB) k_adj_stage3d(Adj3Args<T> a) {
 // zeta^T column pass: tmp = F_zeta^T lam.
 template <typename T, int ORDER>
 __global__ void __launch_bounds__(TPB) k_adj_filter3d_z(const T *__restrict__ lam, T *__restrict__ tmp, int ni,
-                                                        int nj, int nk) {
+                                                        int nj, int nk, int zc) {
   constexpr int H = ORDER / 2;
   const size_t plane = (size_t)ni * nj, n = plane * nk;
   const size_t col = (size_t)blockIdx.x * TPB + threadIdx.x;
   if (col >= plane) return;
-  const int k0 = blockIdx.y * A3_ZC, k1 = min(k0 + A3_ZC, nk);
+  const int k0 = blockIdx.y * zc, k1 = min(k0 + zc, nk);
   T w[5][2 * H + 1];
 #pragma unroll
   for (int q = 0; q < 2 * H; q++) {
@@ -500,6 +478,7 @@ static hipError_t adj_stage3d_t(hipStream_t s, lee_handle *h, Block &b, const Ad
   a.met = b.met;
   a.jac = b.jac;
   a.mc = sizeof(T) == 8 ? (const T *)b.mc64 : (const T *)b.mc32;
+  a.varies = b.mc_varies;
   a.u0 = b.umean[IUX];
   a.v0 = b.umean[IUY];
   a.w0 = b.umean[IUZ];
@@ -550,9 +529,10 @@ static hipError_t adj_filter3d_t(hipStream_t s, lee_handle *h, Block &b, int src
   T *const *L = sizeof(T) == 8 ? (T *const *)b.A64 : (T *const *)b.A32;
   const size_t plane = (size_t)b.ni * b.nj;
   const bool o8 = h->cfg.filter_order == 8;
-  const dim3 gz(nba(plane), (b.nk + A3_ZC - 1) / A3_ZC);
-  if (o8) hipLaunchKernelGGL((k_adj_filter3d_z<T, 8>), gz, dim3(TPB), 0, s, L[src], L[scratch], b.ni, b.nj, b.nk);
-  else hipLaunchKernelGGL((k_adj_filter3d_z<T, 4>), gz, dim3(TPB), 0, s, L[src], L[scratch], b.ni, b.nj, b.nk);
+  const int zc = std::max(4, z_chunk((int)nba(plane), b.nk, A3_ZC, b.cus));
+  const dim3 gz(nba(plane), (b.nk + zc - 1) / zc);
+  if (o8) hipLaunchKernelGGL((k_adj_filter3d_z<T, 8>), gz, dim3(TPB), 0, s, L[src], L[scratch], b.ni, b.nj, b.nk, zc);
+  else hipLaunchKernelGGL((k_adj_filter3d_z<T, 4>), gz, dim3(TPB), 0, s, L[src], L[scratch], b.ni, b.nj, b.nk, zc);
   constexpr int TY = 4;
   AdjF3Args<T> a{};
   a.ni = b.ni;
