@@ -14,6 +14,7 @@
 #include <unordered_map>
 #include <vector>
 
+#include "lee_args.h"
 #include "lee_internal.h"
 
 using namespace lee;
@@ -155,7 +156,7 @@ int enqueue_paired_stages(lee_handle *h) {
   for (int ib = 0; ib < h->nblk; ib++) any_bnd |= !h->b[ib].faces.empty();
   if (!any_bnd) return LEE_OK;
   if (h->ktiming) HIPCHK(mark(h));
-  HIPCHK(boundary_phase_fused(h->stream, h, is_fp32(h), 1, true, stage_bc_entropy(h, S - 1)));
+  HIPCHK(boundary_phase(h->stream, h, is_fp32(h), 1, true, stage_bc_entropy(h, S - 1)));
   if (h->ktiming) {
     HIPCHK(mark(h));
     h->evclass.push_back(4);
@@ -188,7 +189,7 @@ int enqueue_fused_step(lee_handle *h) {
     bool any_bnd = h->ov.nrecv > 0;
     for (int ib = 0; ib < h->nblk; ib++) any_bnd |= !h->b[ib].faces.empty();
     if (h->ktiming && any_bnd) HIPCHK(mark(h));
-    if (any_bnd) HIPCHK(boundary_phase_fused(h->stream, h, f32, tgt, st == last, he_bc));
+    if (any_bnd) HIPCHK(boundary_phase(h->stream, h, f32, tgt, st == last, he_bc));
     if (h->ktiming && any_bnd) {
       HIPCHK(mark(h));
       h->evclass.push_back(4);
@@ -233,11 +234,7 @@ int enqueue_plain_step(lee_handle *h) {
       HIPCHK(plain_stage(s, h, b, st, sc, st == 0 ? b.rho64 : nullptr));
     }
     const int tgt = fused_target(h, st);
-    for (int ib = 0; ib < h->nblk; ib++) {
-      Block &b = h->b[ib];
-      if (!b.faces.empty()) HIPCHK(apply_bcs(s, h, b, b.Y64[tgt], nullptr, false, nullptr, nullptr, he_bc));
-    }
-    HIPCHK(overset_interpolate(s, h, false, tgt, false));
+    HIPCHK(boundary_phase(s, h, false, tgt, false, he_bc));
   }
   for (int ib = 0; ib < h->nblk; ib++) {
     Block &b = h->b[ib];
@@ -294,6 +291,70 @@ int enqueue_batch_step(lee_handle *h) {
     HIPCHK(mark(h));
     h->evclass.push_back(3);
   }
+  return LEE_OK;
+}
+
+// The order in which one launch may set the receivers (k_boundary), with
+// their normalised coefficients, coefficient-major, in coef5: first the
+// nheld that some stencil or face reads or a face writes, held back until the
+// sums are formed; up to nuse those whose stencils read a receiver; up to
+// nearly the others; then those whose stencils read what a face writes,
+// summed after that.  No order (the two-phase form runs) for tables that
+// name a point twice or none of their block's.
+int plan_overset(lee_handle *h, const std::vector<double> &coef5) {
+  Overset &o = h->ov;
+  enum { FACE = 1, REACH = 2, READ = 4, RECV = 8 };
+  std::vector<std::vector<uint8_t>> mark(h->nblk);
+  for (int ib = 0; ib < h->nblk; ib++) {
+    const Block &b = h->b[ib];
+    mark[ib].assign(b.n, 0);
+    for (const auto &f : b.faces) {
+      const BcArgs a = make_bc_args(h, b, f, 0.0);
+      const BcReach r = bc_reach(a);
+      for (int j = std::max(r.lo[1], 0); j <= std::min(r.hi[1], b.nj - 1); j++)
+        for (int i = std::max(r.lo[0], 0); i <= std::min(r.hi[0], b.ni - 1); i++)
+          mark[ib][(size_t)j * b.ni + i] |=
+              REACH | (i >= a.i0 && i <= a.i1 && j >= a.j0 && j <= a.j1 ? FACE : 0);
+    }
+  }
+  for (int r = 0; r < o.nrecv; r++) {
+    const int rb = o.h_rb[r], rl = o.h_rl[r];
+    if (rb < 0 || rb >= h->nblk || rl < 0 || rl >= h->b[rb].n || (mark[rb][rl] & RECV)) return LEE_OK;
+    mark[rb][rl] |= RECV;
+    for (int q = 0; q < 25; q++) mark[o.h_db[r]][o.h_dl[r] + q % 5 + q / 5 * h->b[o.h_db[r]].ni] |= READ;
+  }
+  std::vector<int> order[4];
+  for (int r = 0; r < o.nrecv; r++) {
+    unsigned seen = 0;
+    for (int q = 0; q < 25; q++) seen |= mark[o.h_db[r]][o.h_dl[r] + q % 5 + q / 5 * h->b[o.h_db[r]].ni];
+    const bool held = (mark[o.h_rb[r]][o.h_rl[r]] & (REACH | READ)) != 0;
+    order[seen & FACE ? 3 : held ? 0 : seen & RECV ? 1 : 2].push_back(r);
+  }
+  o.nheld = (int)order[0].size();
+  o.nuse = o.nheld + (int)order[1].size();
+  o.nearly = o.nuse + (int)order[2].size();
+  std::vector<int> perm;
+  for (const auto &q : order) perm.insert(perm.end(), q.begin(), q.end());
+  std::vector<int> t(o.nrecv);
+  auto upload = [&](const std::vector<int> &from, int **to) -> int {
+    for (int k = 0; k < o.nrecv; k++) t[k] = from[perm[k]];
+    HIPCHK(dalloc(to, o.nrecv));
+    HIPCHK(hipMemcpy(*to, t.data(), sizeof(int) * o.nrecv, hipMemcpyHostToDevice));
+    return LEE_OK;
+  };
+  if (int e = upload(o.h_rb, &o.q_rb)) return e;
+  if (int e = upload(o.h_rl, &o.q_rl)) return e;
+  if (int e = upload(o.h_db, &o.q_db)) return e;
+  if (int e = upload(o.h_dl, &o.q_dl)) return e;
+  std::vector<double> c(coef5.size());
+  for (int q = 0; q < 25; q++)
+    for (int k = 0; k < o.nrecv; k++) c[(size_t)q * o.nrecv + k] = coef5[(size_t)q * o.nrecv + perm[k]];
+  HIPCHK(dalloc(&o.q_coef5, c.size()));
+  HIPCHK(hipMemcpy(o.q_coef5, c.data(), sizeof(double) * c.size(), hipMemcpyHostToDevice));
+  const unsigned zero = 0;
+  HIPCHK(dalloc(&o.done, 1));
+  HIPCHK(hipMemcpy(o.done, &zero, sizeof(zero), hipMemcpyHostToDevice));
+  o.ordered = true;
   return LEE_OK;
 }
 
@@ -1066,6 +1127,12 @@ void lee_destroy(lee_handle *h) {
   dfree(h->ov.coef);
   dfree(h->ov.coef5);
   dfree(h->ov.buf);
+  dfree(h->ov.q_rb);
+  dfree(h->ov.q_rl);
+  dfree(h->ov.q_db);
+  dfree(h->ov.q_dl);
+  dfree(h->ov.q_coef5);
+  dfree(h->ov.done);
   if (h->fdw) (void)hipFree(h->fdw);
   if (h->flw) (void)hipFree(h->flw);
   for (auto e : h->evpool) (void)hipEventDestroy(e);
@@ -1463,6 +1530,7 @@ int create_impl(const lee_config *cfgs, int cfg_stride, const lee_block *blocks,
           for (int q = 0; q < 25; q++) t[(size_t)q * o.nrecv + r] = o.h_coef[(size_t)r * o.stride + q];
         HIPCHK(dalloc(&o.coef5, t.size()));
         HIPCHK(hipMemcpy(o.coef5, t.data(), sizeof(double) * t.size(), hipMemcpyHostToDevice));
+        if (int e = plan_overset(h, t)) return e;
       }
     }
     return LEE_OK;
@@ -1850,10 +1918,7 @@ int lee_update_boundary(lee_handle *h, double *const *ys) {
   for (int ib = 0; ib < h->nblk; ib++)
     HIPCHK(hipMemcpy(h->b[ib].Y64[2], ys[ib], sizeof(double) * nvars(h) * h->b[ib].n, hipMemcpyHostToDevice));
   const double he = h->cfg.harmonic_wave == LEE_WAVE_ENTROPY ? harmonic_entropy(h->cfg, h->time_sol) : 0.0;
-  for (int ib = 0; ib < h->nblk; ib++)
-    if (!h->b[ib].faces.empty())
-      HIPCHK(apply_bcs(s, h, h->b[ib], h->b[ib].Y64[2], nullptr, false, nullptr, nullptr, he));
-  HIPCHK(overset_interpolate(s, h, false, 2, false));
+  HIPCHK(boundary_phase(s, h, false, 2, false, he));
   for (int ib = 0; ib < h->nblk; ib++)
     HIPCHK(hipMemcpyAsync(ys[ib], h->b[ib].Y64[2], sizeof(double) * nvars(h) * h->b[ib].n, hipMemcpyDeviceToHost,
                           s));

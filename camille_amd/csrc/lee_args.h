@@ -30,6 +30,20 @@ inline BcArgs make_bc_args(const lee_handle *h, const Block &b, const BcFace &f,
   return a;
 }
 
+// The points face a writes, grown by those its rows read.
+struct BcReach {
+  int lo[2], hi[2];
+};
+inline BcReach bc_reach(const BcArgs &a) {
+  BcReach r{{a.i0, a.j0}, {a.i1, a.j1}};
+  if (a.end == 0) r.hi[a.dir] += a.sb - 1;
+  else r.lo[a.dir] -= a.sb - 1;
+  return r;
+}
+inline bool bc_apart(const BcReach &r, const BcReach &o) {
+  return r.lo[0] > o.hi[0] || o.lo[0] > r.hi[0] || r.lo[1] > o.hi[1] || o.lo[1] > r.hi[1];
+}
+
 template <typename T>
 inline void fill_zones(StageArgs<T> &a, const Block &b) {
   a.nz = 0;

@@ -224,6 +224,13 @@ struct Overset {
   double *coef5 = nullptr;     // when every stencil is 5 x 5: coefficient q of receiver r at q * nrecv + r
   int stride = 0;
   double *buf = nullptr;       // device nrecv * NV
+  // the same receivers ordered for one launch of the whole boundary phase
+  // (plan_overset)
+  bool ordered = false;
+  int nheld = 0, nuse = 0, nearly = 0;
+  int *q_rb = nullptr, *q_rl = nullptr, *q_db = nullptr, *q_dl = nullptr;
+  double *q_coef5 = nullptr;
+  unsigned *done = nullptr;    // counter of the launch's workgroups
   std::vector<int> h_rb, h_rl, h_db, h_dl, h_w;
   std::vector<double> h_coef;
   double **yptr = nullptr;     // device table of per-block variable pointers (NV per block)
@@ -316,8 +323,7 @@ double harmonic_entropy(const lee_config &c, double t);
 double harmonic_gaussian(const lee_config &c, double x, double y, double z);
 hipError_t apply_bcs(hipStream_t s, lee_handle *h, const Block &b, double *y64, float *y32, bool fp32,
                      double *rho64, float *rho32, double he = 0.0);
-hipError_t overset_interpolate(hipStream_t s, lee_handle *h, bool fp32, int buf_index, bool last_stage);
-hipError_t boundary_phase_fused(hipStream_t s, lee_handle *h, bool fp32, int tgt, bool last, double he);
+hipError_t boundary_phase(hipStream_t s, lee_handle *h, bool fp32, int buf_index, bool with_rho, double he);
 // Overset interpolation of caller-owned FP64 block arrays ys[b] (device,
 // 5n each), receiver values staged in buf (nrecv * NV doubles, device).
 hipError_t overset_interpolate_arrays(hipStream_t s, lee_handle *h, double *const *ys, double *buf);

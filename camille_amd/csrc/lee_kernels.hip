@@ -4,9 +4,8 @@
 // derivatives of the four active variables, chain rule with FP64 metrics,
 // LEE right-hand side, source, sponge, RK update, aux density) and one
 // kernel per step for the two filter sweeps + blend + hole reset, templated
-// on the bulk type (double or float); batched ensembles of them; and the
-// boundary conditions and overset interpolation that both paths share.  The
-// plain path is in lee_plain.hip.
+// on the bulk type (double or float); and batched ensembles of them.  The
+// plain path is in lee_plain.hip, the boundary phase in lee_boundary.hip.
 //
 // All global indices are bounds-checked against the block extents.
 #include <hip/hip_runtime.h>
@@ -14,7 +13,6 @@
 #include <cmath>
 
 #include "lee_args.h"
-#include "lee_bc.h"
 #include "lee_device.h"
 #include "lee_internal.h"
 #include "lee_stage.h"
@@ -22,217 +20,6 @@
 namespace lee {
 
 namespace {
-
-// ------------------------------------------------------ boundary conditions
-
-// One point of a BC face in global memory.
-template <typename T>
-__device__ __forceinline__ void bc_face_point(T *__restrict__ y, const double *__restrict__ met,
-                                              const double *__restrict__ jac, const int8_t *__restrict__ iblank,
-                                              const BcArgs &a, T *__restrict__ rho, const double *__restrict__ mean,
-                                              const double *__restrict__ rhob, double gi, int q) {
-#pragma clang fp contract(off)
-  const int fw = a.i1 - a.i0 + 1;
-  const int i = a.i0 + q % fw, j = a.j0 + q / fw;
-  const int n = a.ni * a.nj;
-  const int p = j * a.ni + i;
-  if (iblank && iblank[p] == BLANKED) return;
-  const int c = a.dir == 0 ? i : j, len = a.dir == 0 ? a.ni : a.nj, sg = a.end == 0 ? 1 : -1;
-  const int mf = a.dir == 0 ? 1 : a.ni;
-  // the block point s points inward (clamped to the face point)
-  auto at = [&](int s) {
-    const int cs = c + sg * s;
-    return p + sg * mf * (cs >= 0 && cs < len ? s : 0);
-  };
-  double data[NV];
-  bc_face_data<T, 8>(a, q, p, c, len, met, jac, [&](int v, int s) { return y[(size_t)v * n + at(s)]; }, data);
-  // passive scalars: Neumann data at Neumann, wall-slip (its non-velocity
-  // variables, boundary_condition.cpp:122-136) and centerline faces; 0 at
-  // dirichlet_allzero and harmonic-wave faces, whose data start at 0
-  for (int z = 0; z < a.nsc; z++) {
-    const size_t vo = (size_t)(NV + z) * n;
-    double d = 0.0;
-    if (bc_is_neumann(a)) {
-      T nbz[8];
-#pragma unroll
-      for (int s = 1; s <= 8; s++) nbz[s - 1] = y[vo + at(s)];
-      d = bc_neumann_value<T, 8>(a, c, len, nbz);
-    }
-    y[vo + p] = (T)d;
-  }
-  for (int v = 0; v < NV; v++) y[(size_t)v * n + p] = (T)data[v];
-  if (rho) {
-    const double pbi = 1.0 / mean[(size_t)IP * n + p];
-    double r = data[IP] * gi * pbi - data[IS];
-    r *= rhob[p];
-    rho[p] = (T)r;
-  }
-}
-
-// Faces of one block that neither read nor write a point another one of them
-// writes, in one launch: workgroups start[k] .. start[k + 1] - 1 take face k.
-// A launch of one face is all latency (4 us for 700 points), so faces that
-// may share one do (a channel's two walls: 8 launches a step -> 4).
-constexpr int BC_BATCH = 4;
-struct BcBatch {
-  int nf;
-  int start[BC_BATCH + 1];
-  BcArgs f[BC_BATCH];
-};
-
-template <typename T>
-__global__ void __launch_bounds__(TPB) k_bc_faces(T *__restrict__ y, const double *__restrict__ met,
-                                                  const double *__restrict__ jac,
-                                                  const int8_t *__restrict__ iblank, BcBatch b,
-                                                  T *__restrict__ rho, const double *__restrict__ mean,
-                                                  const double *__restrict__ rhob, double gi) {
-  int k = 0;
-  while (k + 1 < b.nf && (int)blockIdx.x >= b.start[k + 1]) k++;
-  const BcArgs &a = b.f[k];
-  const int q = ((int)blockIdx.x - b.start[k]) * TPB + threadIdx.x;
-  if (q >= (a.i1 - a.i0 + 1) * (a.j1 - a.j0 + 1)) return;
-  bc_face_point<T>(y, met, jac, iblank, a, rho, mean, rhob, gi, q);
-}
-
-// ---------------------------------------------------------------- overset
-
-template <typename T>
-struct OvTables {
-  int nv;  // variables per point (NV and the passive scalars)
-  T *y[MAX_OV_BLOCKS];
-  int ni[MAX_OV_BLOCKS], nn[MAX_OV_BLOCKS];
-  T *rho[MAX_OV_BLOCKS];
-  const double *mean[MAX_OV_BLOCKS];
-  const double *rhob[MAX_OV_BLOCKS];
-};
-
-// compute_weighted_sum (overset.cpp:886-974): every receiver's weighted
-// donor sum into buf before any receiver is written.
-template <typename T>
-__global__ void __launch_bounds__(TPB) k_ov_gather(OvTables<T> t, const int *__restrict__ db,
-                                                   const int *__restrict__ dl, const int *__restrict__ w,
-                                                   const double *__restrict__ coef, int stride,
-                                                   double *__restrict__ buf, int nrecv) {
-#pragma clang fp contract(off)
-  const int r = blockIdx.x * TPB + threadIdx.x;
-  if (r >= nrecv) return;
-  const int b = db[r];
-  const T *y = t.y[b];
-  const int ni = t.ni[b], n = t.nn[b];
-  const int w1 = w[3 * b], w2 = w[3 * b + 1];
-  const double *c = coef + (size_t)r * stride;
-  if (w1 == 5 && w2 == 5 && w[3 * b + 2] == 1) {
-    // ORDER 4 in 2-D: the 25 donors of one variable are requested together
-    // (clamped addresses, skipped donors masked), then summed in the
-    // reference's order; one memory latency per variable instead of one
-    // per donor
-    const int d0 = dl[r];
-    double cc[25];
-    int li[25];
-    bool ok[25];
-#pragma unroll
-    for (int q = 0; q < 25; q++) {
-      const int l1 = d0 + (q % 5) + (q / 5) * ni;
-      ok[q] = l1 >= 0 && l1 < n;
-      li[q] = ok[q] ? l1 : 0;
-      cc[q] = c[q];
-    }
-    for (int v = 0; v < t.nv; v++) {
-      T yv[25];
-#pragma unroll
-      for (int q = 0; q < 25; q++) yv[q] = y[(size_t)v * n + li[q]];
-      double a = 0.0;
-#pragma unroll
-      for (int q = 0; q < 25; q++) {
-        const double t1 = a + cc[q] * (double)yv[q];
-        a = ok[q] ? t1 : a;
-      }
-      buf[(size_t)r * t.nv + v] = a;
-    }
-    return;
-  }
-  double acc[MAXV];
-  for (int v = 0; v < MAXV; v++) acc[v] = 0.0;
-  int s = 0;
-  for (int b2 = 0; b2 < w2; b2++)
-    for (int b1 = 0; b1 < w1; b1++) {
-      const int l1 = dl[r] + b1 + b2 * ni;
-      if (l1 >= 0 && l1 < n)
-        for (int v = 0; v < t.nv; v++) acc[v] += c[s] * (double)y[(size_t)v * n + l1];
-      s++;
-    }
-  for (int v = 0; v < t.nv; v++) buf[(size_t)r * t.nv + v] = acc[v];
-}
-
-// compute_weighted_sum for 5 x 5 stencils (overset.cpp:886-974), receiver r
-// and variable v: the 25 donor values and coefficients (receiver-minor, so
-// coalesced across receivers) are requested together, then summed in the
-// reference's order with the donors outside the block skipped.
-template <typename T>
-__device__ __forceinline__ double ov_sum5(const OvTables<T> &t, const int *__restrict__ db,
-                                          const int *__restrict__ dl, const double *__restrict__ coef5, int nrecv,
-                                          int r, int v) {
-#pragma clang fp contract(off)
-  const int b = db[r];
-  const T *y = t.y[b] + (size_t)v * t.nn[b];
-  const int ni = t.ni[b], n = t.nn[b], d0 = dl[r];
-  double cc[25];
-  T yv[25];
-  bool ok[25];
-#pragma unroll
-  for (int q = 0; q < 25; q++) {
-    const int l1 = d0 + (q % 5) + (q / 5) * ni;
-    ok[q] = l1 >= 0 && l1 < n;
-    cc[q] = coef5[(size_t)q * nrecv + r];
-    yv[q] = y[ok[q] ? l1 : 0];
-  }
-  double a = 0.0;
-#pragma unroll
-  for (int q = 0; q < 25; q++) {
-    const double t1 = a + cc[q] * (double)yv[q];
-    a = ok[q] ? t1 : a;
-  }
-  return a;
-}
-
-// The gather of the two-phase update: one thread per (receiver, variable),
-// every sum into buf before any receiver is written.
-template <typename T>
-__global__ void __launch_bounds__(TPB) k_ov_gather5(OvTables<T> t, const int *__restrict__ db,
-                                                    const int *__restrict__ dl, const double *__restrict__ coef5,
-                                                    double *__restrict__ buf, int nrecv) {
-  const int gid = blockIdx.x * TPB + threadIdx.x;
-  if (gid >= t.nv * nrecv) return;
-  const int v = gid / nrecv, r = gid - v * nrecv;
-  buf[(size_t)r * t.nv + v] = ov_sum5(t, db, dl, coef5, nrecv, r, v);
-}
-
-// update_each_grid (overset.cpp:1241-1278); optionally refreshes rho'.
-template <typename T>
-__device__ __forceinline__ void ov_scatter_one(const OvTables<T> &t, const int *__restrict__ rb,
-                                               const int *__restrict__ rl, const double *__restrict__ buf,
-                                               int with_rho, double gi, int r) {
-#pragma clang fp contract(off)
-  const int b = rb[r];
-  const int n = t.nn[b], p = rl[r];
-  if (p < 0 || p >= n) return;
-  for (int v = 0; v < t.nv; v++) t.y[b][(size_t)v * n + p] = (T)buf[(size_t)r * t.nv + v];
-  if (with_rho && t.rho[b]) {
-    const double pbi = 1.0 / t.mean[b][(size_t)IP * n + p];
-    double q = buf[(size_t)r * t.nv + IP] * gi * pbi - buf[(size_t)r * t.nv + IS];
-    q *= t.rhob[b][p];
-    t.rho[b][p] = (T)q;
-  }
-}
-
-template <typename T>
-__global__ void __launch_bounds__(TPB) k_ov_scatter(OvTables<T> t, const int *__restrict__ rb,
-                                                    const int *__restrict__ rl, const double *__restrict__ buf,
-                                                    int nrecv, int with_rho, double gi) {
-  const int r = blockIdx.x * TPB + threadIdx.x;
-  if (r >= nrecv) return;
-  ov_scatter_one<T>(t, rb, rl, buf, with_rho, gi, r);
-}
 
 // ------------------------------------------------------------------ fused
 
@@ -765,121 +552,6 @@ inline unsigned nblocks(size_t n) { return (unsigned)((n + TPB - 1) / TPB); }
 }  // namespace
 
 // ------------------------------------------------------------- launchers
-
-// The points face f writes, grown by those its rows read.
-struct BcReach {
-  int lo[2], hi[2];
-};
-static BcReach bc_reach(const BcArgs &a) {
-  BcReach r{{a.i0, a.j0}, {a.i1, a.j1}};
-  if (a.end == 0) r.hi[a.dir] += a.sb - 1;
-  else r.lo[a.dir] -= a.sb - 1;
-  return r;
-}
-
-hipError_t apply_bcs(hipStream_t s, lee_handle *h, const Block &b, double *y64, float *y32, bool fp32,
-                     double *rho64, float *rho32, double he) {
-  const int8_t *ib = b.has_holes ? b.iblank : nullptr;
-  BcBatch t{};
-  auto flush = [&]() {
-    if (t.nf == 0) return;
-    const dim3 grid(t.start[t.nf]);
-    if (fp32)
-      hipLaunchKernelGGL(k_bc_faces<float>, grid, dim3(TPB), 0, s, y32, b.met, b.jac, ib, t, rho32, b.mean, b.rhobar,
-                         1.0 / h->cfg.gamma);
-    else
-      hipLaunchKernelGGL(k_bc_faces<double>, grid, dim3(TPB), 0, s, y64, b.met, b.jac, ib, t, rho64, b.mean, b.rhobar,
-                         1.0 / h->cfg.gamma);
-    t.nf = 0;
-  };
-  // in the order of the BC file; a face joins the launch before it unless
-  // their reaches meet (faces that share a corner keep their order)
-  for (const auto &f : b.faces) {
-    const BcArgs a = make_bc_args(h, b, f, he);
-    const BcReach r = bc_reach(a);
-    bool apart = t.nf < BC_BATCH;
-    for (int k = 0; k < t.nf; k++) {
-      const BcReach o = bc_reach(t.f[k]);
-      apart &= r.lo[0] > o.hi[0] || o.lo[0] > r.hi[0] || r.lo[1] > o.hi[1] || o.lo[1] > r.hi[1];
-    }
-    if (!apart) flush();
-    t.f[t.nf] = a;
-    t.start[t.nf + 1] = t.start[t.nf] + (int)nblocks((size_t)(a.i1 - a.i0 + 1) * (a.j1 - a.j0 + 1));
-    t.nf++;
-  }
-  flush();
-  return hipGetLastError();
-}
-
-template <typename T>
-static hipError_t overset_t(hipStream_t s, lee_handle *h, T *const *ys, T *const *rhos, bool with_rho, double *buf) {
-  OvTables<T> t{};
-  t.nv = nvars(h);
-  for (int ib = 0; ib < h->nblk; ib++) {
-    t.y[ib] = ys[ib];
-    t.ni[ib] = h->b[ib].ni;
-    t.nn[ib] = h->b[ib].n;
-    t.rho[ib] = rhos ? rhos[ib] : nullptr;
-    t.mean[ib] = h->b[ib].mean;
-    t.rhob[ib] = h->b[ib].rhobar;
-  }
-  const Overset &o = h->ov;
-  if (o.coef5)
-    hipLaunchKernelGGL(k_ov_gather5<T>, dim3(nblocks((size_t)t.nv * o.nrecv)), dim3(TPB), 0, s, t, o.db, o.dl, o.coef5,
-                       buf, o.nrecv);
-  else
-    hipLaunchKernelGGL(k_ov_gather<T>, dim3(nblocks(o.nrecv)), dim3(TPB), 0, s, t, o.db, o.dl, o.w, o.coef, o.stride,
-                       buf, o.nrecv);
-  hipLaunchKernelGGL(k_ov_scatter<T>, dim3(nblocks(o.nrecv)), dim3(TPB), 0, s, t, o.rb, o.rl, buf, o.nrecv,
-                     with_rho ? 1 : 0, 1.0 / h->cfg.gamma);
-  return hipGetLastError();
-}
-
-// buf_index selects the state buffer (Y[k]) of every block.
-hipError_t overset_interpolate(hipStream_t s, lee_handle *h, bool fp32, int buf_index, bool last_stage) {
-  if (h->ov.nrecv == 0) return hipSuccess;
-  if (fp32) {
-    float *ys[MAX_OV_BLOCKS], *rh[MAX_OV_BLOCKS];
-    bool any_rho = false;
-    for (int ib = 0; ib < h->nblk; ib++) {
-      ys[ib] = h->b[ib].Y32[buf_index];
-      rh[ib] = h->b[ib].uniform_mean ? nullptr : h->b[ib].rho32;
-      any_rho |= rh[ib] != nullptr;
-    }
-    return overset_t<float>(s, h, ys, rh, last_stage && any_rho, h->ov.buf);
-  }
-  double *ys[MAX_OV_BLOCKS], *rh[MAX_OV_BLOCKS];
-  bool any_rho = false;
-  for (int ib = 0; ib < h->nblk; ib++) {
-    ys[ib] = h->b[ib].Y64[buf_index];
-    rh[ib] = h->b[ib].uniform_mean ? nullptr : h->b[ib].rho64;
-    any_rho |= rh[ib] != nullptr;
-  }
-  return overset_t<double>(s, h, ys, rh, last_stage && any_rho, h->ov.buf);
-}
-
-hipError_t overset_interpolate_arrays(hipStream_t s, lee_handle *h, double *const *ys, double *buf) {
-  if (h->ov.nrecv == 0) return hipSuccess;
-  return overset_t<double>(s, h, ys, nullptr, false, buf);
-}
-
-// The boundary phase of a fused stage on the stage's target buffers: the
-// BC faces of every block (a launch per face), then the overset
-// interpolation (gather, then scatter).  One cooperative launch with grid
-// barriers in between was measured slower (overset cylinder 1.72e10
-// against 2.18e10 FP32 updates/s over 1000 steps): the runtime's
-// cooperative launch costs more than the launches it replaces.
-hipError_t boundary_phase_fused(hipStream_t s, lee_handle *h, bool fp32, int tgt, bool last, double he) {
-  hipError_t e = hipSuccess;
-  for (int ib = 0; ib < h->nblk; ib++) {
-    Block &b = h->b[ib];
-    if (b.faces.empty()) continue;
-    const bool rho = last && !b.uniform_mean;
-    e = apply_bcs(s, h, b, b.Y64[tgt], b.Y32[tgt], fp32, rho ? b.rho64 : nullptr, rho ? b.rho32 : nullptr, he);
-    if (e != hipSuccess) return e;
-  }
-  return overset_interpolate(s, h, fp32, tgt, last);
-}
 
 template <typename T>
 static hipError_t fused_stage_t(hipStream_t s, lee_handle *h, Block &b, int stage, const StageScalars &sc, T *const *Y,

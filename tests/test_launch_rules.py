@@ -4,6 +4,7 @@ import numpy as np
 import pytest
 
 from camille_amd import FP32, FP64, PATH_PLAIN, Solver
+from test_zz_no_alloc import _noalloc
 
 pytestmark = pytest.mark.gpu
 
@@ -162,3 +163,49 @@ def test_paired_stages_bit_identical(shape, kind, prec):
         s.close()
     assert np.all(np.isfinite(out[0][0]))
     assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
+
+
+_FACES = {
+    "none": [],
+    "walls": [(0, "wall_slip_kinematic", "+eta", "0", "-0", "0", "0", "0", "0"),
+              (1, "neumann", "-xi", "-0", "-0", "0", "-0", "0", "0")],
+    "meeting": [(0, "neumann", "+xi", "0", "0", "0", "-0", "0", "0"),
+                (0, "wall_slip_kinematic", "+eta", "0", "-0", "0", "0", "0", "0"),
+                (1, "dirichlet_allzero", "-eta", "0", "-0", "-0", "-0", "0", "0")],
+}
+
+
+# receivers that other sums and faces read, that faces write, and whose
+# stencils read what faces write; "twice" names points twice, which has no order
+@pytest.mark.parametrize("nrecv", [1, 25, 26, 51, 700])
+@pytest.mark.parametrize("faces", list(_FACES))
+@pytest.mark.parametrize("twice", [False, True])
+def test_boundary_phase_in_one_launch(nrecv, faces, twice):
+    """The faces and the interpolation in one launch against the launch per
+    face, gather and scatter, bit for bit, over three applications in a row."""
+    rng = np.random.default_rng(nrecv)
+    dims = [(41, 31), (67, 23)]
+    blocks = []
+    for ni, nj in dims:
+        i, j = np.meshgrid(np.arange(ni), np.arange(nj))
+        mean = np.zeros((5, nj, ni))
+        mean[4] = 1.0 / GAMMA
+        blocks.append(dict(x=i + 0.1 * np.sin(0.5 * j), y=j + 0.1 * np.sin(0.4 * i), mean=mean))
+    pts = np.array([(b, p) for b, (ni, nj) in enumerate(dims) for p in range(ni * nj)])
+    recv = pts[rng.permutation(len(pts))[:nrecv]]
+    db = rng.integers(0, 2, nrecv)
+    dl = np.array([rng.integers(0, dims[b][1] - 4) * dims[b][0] + rng.integers(0, dims[b][0] - 4) for b in db])
+    coef = rng.uniform(0.1, 1.0, (nrecv, 25))
+    if twice:
+        recv[-1], db[-1], dl[-1], coef[-1] = recv[0], db[0], dl[0], coef[0]
+    tables = dict(recv_block=recv[:, 0], recv_l=recv[:, 1], donor_block=db, donor_l=dl,
+                  widths=np.array([[5, 5, 1], [5, 5, 1]]), coef=coef, hole_block=np.zeros(0, int),
+                  hole_l=np.zeros(0, int))
+    s = Solver(blocks, overset=tables, boundaries=_FACES[faces], precision=FP64, mode="FIX_DT", value=0.01)
+    ys = [rng.standard_normal((5, nj, ni)) for ni, nj in dims]
+    for _ in range(3):
+        want = _noalloc(s, ys)
+        ys = s.update_boundary(ys)
+        for got, ref in zip(ys, want):
+            assert np.all(np.isfinite(got)) and np.array_equal(got, ref)
+    s.close()
