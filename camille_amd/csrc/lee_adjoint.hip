@@ -51,25 +51,14 @@ __device__ __forceinline__ T fd_wt(int code, int d) {
   }
 }
 
-// Transposed FD row at coordinate c of a line of length len (no holes):
-// the rows of the neighbours c + o, o in [-2, 2], that exist.
+// Transposed FD row where every neighbour's row is interior: D^T = -D there.
 template <typename T>
-__device__ __forceinline__ T fd_row_t(const T *f, int st, int c, int len, bool inner) {
-  if (inner) {  // every neighbour row is interior: D^T = -D there
-    const T c1 = (T)(8.0 / 12.0), c2 = (T)(-1.0 / 12.0);
-    T acc = c2 * f[-2 * st];
-    acc += c1 * f[-st];
-    acc += -c1 * f[st];
-    acc += -c2 * f[2 * st];
-    return acc;
-  }
-  T acc = 0;
-#pragma unroll
-  for (int o = -2; o <= 2; o++) {
-    const int j = c + o;
-    if (j < 0 || j >= len) continue;
-    acc += fd_wt<T>(default_code(j, len, 2), -o) * f[o * st];
-  }
+__device__ __forceinline__ T fd_row_t_inner(const T *f, int st) {
+  const T c1 = (T)(8.0 / 12.0), c2 = (T)(-1.0 / 12.0);
+  T acc = c2 * f[-2 * st];
+  acc += c1 * f[-st];
+  acc += -c1 * f[st];
+  acc += -c2 * f[2 * st];
   return acc;
 }
 
@@ -118,19 +107,35 @@ __device__ __forceinline__ T flt_wt(int code, int d) {
   }
 }
 
+// Transposed filter row at coordinate c of a line of length len (no holes)
+// as weights of the neighbours c + o, o in [-H, H]: the rows there that
+// exist, chosen by selects.  Filter rows are symmetric, so row j counts with
+// its weight at distance |o|.
 template <typename T, int ORDER>
-__device__ __forceinline__ T flt_row_t(const T *f, int st, int c, int len, bool inner) {
-  constexpr int NB = ORDER / 2, H = ORDER / 2;
-  if (inner) {  // symmetric interior rows: F^T = F
-    return filter_row<T, ORDER>(f, st, CODE_INTERIOR);
-  }
-  T acc = 0;
+struct FltRowT {
+  static constexpr int H = ORDER / 2;
+  T w[2 * H + 1];
+};
+template <typename T, int ORDER>
+__device__ __forceinline__ FltRowT<T, ORDER> flt_row_t(int c, int len) {
+  constexpr int H = ORDER / 2;
+  FltRowT<T, ORDER> r;
 #pragma unroll
   for (int o = -H; o <= H; o++) {
-    const int j = c + o;
-    if (j < 0 || j >= len) continue;
-    acc += flt_wt<T, ORDER>(default_code(j, len, NB), -o) * f[o * st];
+    const int j = c + o, row = j < H ? j : min(len - 1 - j, H);  // default_code
+    T w = flt_wt<T, ORDER>(CODE_INTERIOR, o);
+#pragma unroll
+    for (int k = 0; k < H; k++) w = row == k ? flt_wt<T, ORDER>(CODE_LEFT + k, o) : w;
+    r.w[o + H] = j >= 0 && j < len ? w : (T)0;
   }
+  return r;
+}
+template <typename T, int ORDER>
+__device__ __forceinline__ T flt_row_t_sum(const FltRowT<T, ORDER> &r, const T *f, int st) {
+  constexpr int H = ORDER / 2;
+  T acc = r.w[0] * f[-H * st];
+#pragma unroll
+  for (int o = 1 - H; o <= H; o++) acc += r.w[o + H] * f[o * st];
   return acc;
 }
 
@@ -168,23 +173,29 @@ struct AdjArgs {
   const T *rad;                 // axisymmetric runs: the forward's radius field r + 1e-99 (null: none)
 };
 
-template <typename T, int R>
-using AdjLds = T[8][4 * R + 2 * ST_H][ST_TX + 2 * ST_H];
+constexpr int ADJ_TY = 4;
 
-// One reversed RK stage on a 64 x 4R tile: kappa and the flux fields on the
+// What bounds it: latency, of the fluxes' operands and of each tile's serial
+// work, more than its 296 bytes a point (FP64, general mean).  Tiles of 4
+// rows (2.1 fluxes a point, but twice the workgroups of 8 rows: reverse step
+// of 385 x 257 FP64 98 against 108 us, 1025 x 513 286 against 296, 2049 x
+// 1025 1120 against 1111), the region spread over the threads in line order,
+// the point's operands requested before the barrier, transposed closure rows
+// without branches: middle stage of 385 x 257 FP64 25 -> 12.8 us.
+// One reversed RK stage on a 64 x 4 tile: kappa and the flux fields on the
 // tile and its 2-point halo go to LDS, then the transposed stencils, the
 // point-local transposed terms and the accumulations of the running
-// adjoints for the R points of each thread.
+// adjoints.
 // Blocks with holes (HOLES): the forward stage writes 0 at BLANKED points
 // whatever its inputs, so the adjoints arriving there (lacc, lin) count as 0
 // and kappa vanishes there; the transposed rows take the per-point codes.
-template <typename T, bool MEANF, int KIND, int R, bool HOLES>
+template <typename T, bool MEANF, int KIND, bool HOLES>
 __global__ void __launch_bounds__(TPB) k_adj_stage(AdjArgs<T> a) {
-  constexpr int TY = 4 * R, NR = TY + 2 * ST_H, RS = ST_TX + 2 * ST_H;
-  __shared__ AdjLds<T, R> F;  // F[v] xi-flux, F[4 + v] eta-flux
+  constexpr int TY = ADJ_TY, NR = TY + 2 * ST_H, RS = ST_TX + 2 * ST_H;
+  __shared__ T F[8][NR][RS];  // F[v] xi-flux, F[4 + v] eta-flux
   const int tile = xcd_tile(blockIdx.x, a.chunk);
   if (tile >= a.ntiles) return;
-  const int tx = threadIdx.x, ty = threadIdx.y;
+  const int tx = threadIdx.x, ty = __builtin_amdgcn_readfirstlane((int)threadIdx.y);  // a wave is one row
   const int i0 = (tile % a.ntx) * ST_TX, j0 = (tile / a.ntx) * TY;
   const int ni = a.ni, nj = a.nj, n = ni * nj;
   const int VOFF[4] = {IS * n, IUX * n, IUY * n, IP * n};
@@ -192,148 +203,163 @@ __global__ void __launch_bounds__(TPB) k_adj_stage(AdjArgs<T> a) {
                            : (i0 >= 2 * ST_H && i0 + ST_TX + 2 * ST_H <= ni && j0 >= 2 * ST_H &&
                               j0 + TY + 2 * ST_H <= nj);
   const T hb = (T)a.hb, ha = (T)a.ha;
+  // sponge zones of the tile: the boxes are kernel arguments at fixed places,
+  // read all at once
+  unsigned zmask = 0;
+#pragma unroll
+  for (int z = 0; z < MAX_ZONES; z++)
+    zmask |= z < a.nz && a.z[z].i0 < i0 + ST_TX && a.z[z].i1 >= i0 && a.z[z].j0 < j0 + TY && a.z[z].j1 >= j0
+                 ? 1u << z : 0;
 
-  // (1) kappa and fluxes over the tile plus halo; row r = ty + 4k
-  // (k = 0..R), columns tx and, for tx < 4, 64 + tx
+  // (1) kappa and fluxes over the tile plus halo, in line order over the
+  // threads; points outside the block evaluate the nearest one inside and
+  // store 0
+  auto ring = [&](int idx) {
+    const int r = idx / RS, c = idx - r * RS;
+    const int rj = j0 - ST_H + r, ri = i0 - ST_H + c;
+    const int p = min(max(rj, 0), nj - 1) * ni + min(max(ri, 0), ni - 1);
+    const bool ok = rj >= 0 && rj < nj && ri >= 0 && ri < ni && !(HOLES && a.iblank[p] == BLANKED);
+    T kap[4];
 #pragma unroll
-  for (int k = 0; k <= R; k++) {
-    const int r = ty + 4 * k;
-    const int gj = j0 - ST_H + r;
-#pragma unroll
-    for (int half = 0; half < 2; half++) {
-      const int c = half == 0 ? tx : ST_TX + tx;
-      if (half == 1 && tx >= 2 * ST_H) continue;
-      const int gi = i0 - ST_H + c;
-      const bool ok = gj >= 0 && gj < nj && gi >= 0 && gi < ni && !(HOLES && a.iblank[gj * ni + gi] == BLANKED);
-      double fx[4] = {0.0, 0.0, 0.0, 0.0}, fy[4] = {0.0, 0.0, 0.0, 0.0};
-      if (ok) {
-        const int p = gj * ni + gi;
-        T kap[4];
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          T kv = hb * a.lacc[VOFF[v] + p];
-          if (KIND != STAGE_LAST && a.lin) kv += ha * a.lin[VOFF[v] + p];
-          kap[v] = kv;
-        }
-        double u0 = a.u0, v0 = a.v0, gp = a.gp0, irb = 1.0 / a.rhob0;
-        if (MEANF) {
-          u0 = a.mean[IUX * n + p];
-          v0 = a.mean[IUY * n + p];
-          gp = a.gamma * a.mean[IP * n + p];
-          irb = 1.0 / a.rhob[p];
-        }
-        const double ks = kap[0], ku = kap[1], kv = kap[2], kp = kap[3];
-        // coefficients of d/dx (A) and d/dy (B) of each variable
-        const double A[4] = {-u0 * ks, -u0 * ku - gp * kp, -u0 * kv, -u0 * kp - ku * irb};
-        const double B[4] = {-v0 * ks, -v0 * ku, -v0 * kv - gp * kp, -v0 * kp - kv * irb};
-        const double mxx = a.met[p], mxy = a.met[(size_t)n + p], myx = a.met[(size_t)2 * n + p],
-                     myy = a.met[(size_t)3 * n + p];
-        const double J = a.jac[p];
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          fx[v] = (mxx * A[v] + mxy * B[v]) * J;
-          fy[v] = (myx * A[v] + myy * B[v]) * J;
-        }
-      }
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        F[v][r][c] = (T)fx[v];
-        F[4 + v][r][c] = (T)fy[v];
-      }
+    for (int v = 0; v < 4; v++) {
+      T kv = hb * a.lacc[VOFF[v] + p];
+      if (KIND != STAGE_LAST && a.lin) kv += ha * a.lin[VOFF[v] + p];
+      kap[v] = kv;
     }
+    double u0 = a.u0, v0 = a.v0, gp = a.gp0, irb = 1.0 / a.rhob0;
+    if (MEANF) {
+      u0 = a.mean[IUX * n + p];
+      v0 = a.mean[IUY * n + p];
+      gp = a.gamma * a.mean[IP * n + p];
+      irb = 1.0 / a.rhob[p];
+    }
+    const double ks = kap[0], ku = kap[1], kv = kap[2], kp = kap[3], c0 = gp * kp;
+    const double m[2][2] = {{a.met[p], a.met[(size_t)n + p]}, {a.met[(size_t)2 * n + p], a.met[(size_t)3 * n + p]}};
+    const double J = -a.jac[p];
+    // F_l = -J (U_l kappa + ...) with the contravariant velocity U_l
+#pragma unroll
+    for (int l = 0; l < 2; l++) {
+      const double U = m[l][0] * u0 + m[l][1] * v0;
+      const double f[4] = {U * ks * J, (U * ku + m[l][0] * c0) * J, (U * kv + m[l][1] * c0) * J,
+                           (U * kp + (m[l][0] * ku + m[l][1] * kv) * irb) * J};
+#pragma unroll
+      for (int v = 0; v < 4; v++) F[4 * l + v][r][c] = ok ? (T)f[v] : (T)0;
+    }
+  };
+  const int tid = ty * 64 + tx;
+#pragma unroll
+  for (int q = 0; q < NR * RS / TPB; q++) ring(tid + q * TPB);
+  if (tid + NR * RS / TPB * TPB < NR * RS) ring(tid + NR * RS / TPB * TPB);
+
+  // (2) the operands of the thread's point, requested before the barrier
+  const int gi = i0 + tx, gj = j0 + ty;
+  const int p = min(gj, nj - 1) * ni + min(gi, ni - 1);
+  T lacc[4], lin[4], lyin[4], mg[8];
+  double mb[4];
+  const bool hole = HOLES && a.iblank[p] == BLANKED;
+#pragma unroll
+  for (int v = 0; v < 4; v++) {
+    lacc[v] = a.lacc[VOFF[v] + p];
+    lin[v] = KIND != STAGE_LAST && a.lin ? a.lin[VOFF[v] + p] : (T)0;
+    lyin[v] = KIND != STAGE_LAST && a.lyin ? a.lyin[VOFF[v] + p] : (T)0;
+  }
+  const double gr = a.grad ? a.grad[p] : 0.0;
+  if (MEANF) {
+    mb[0] = a.mean[IUX * n + p];
+    mb[1] = a.mean[IUY * n + p];
+    mb[2] = a.rhob[p];
+    mb[3] = a.mean[IP * n + p];
+    constexpr int GV[4] = {IS, IUX, IUY, IP};
+#pragma unroll
+    for (int v = 0; v < 4; v++)
+#pragma unroll
+      for (int d = 0; d < 2; d++) mg[2 * v + d] = (T)a.mgrad[(2 * GV[v] + d) * n + p];
   }
   __syncthreads();
 
-  // (2) the R points of the thread
-  const int gi = i0 + tx;
-#pragma unroll
-  for (int k = 0; k < R; k++) {
-    const int rr = ty + 4 * k;
-    const int gj = j0 + rr;
-    if (!inner && (gi >= ni || gj >= nj)) continue;
-    const int p = gj * ni + gi;
-    const int lj = rr + ST_H, li = tx + ST_H;
-    T lam[4];
-    if (HOLES && !inner) {
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        lam[v] = fd_row_t_codes<T>(&F[v][lj][li], 1, gi, ni, a.code, p, 1);
-        lam[v] += fd_row_t_codes<T>(&F[4 + v][lj][li], RS, gj, nj, a.code + n, p, ni);
-      }
-    } else {
-#pragma unroll
-      for (int v = 0; v < 4; v++) {
-        lam[v] = fd_row_t<T>(&F[v][lj][li], 1, gi, ni, inner);
-        lam[v] += fd_row_t<T>(&F[4 + v][lj][li], RS, gj, nj, inner);
-      }
-    }
-    const bool hole = HOLES && a.iblank[p] == BLANKED;
-    // kappa at the point (recomputed from the same operands)
-    T kap[4], lacc[4], lin[4];
+  // (3) the point of the thread
+  if (gi >= ni || gj >= nj) return;
+  const int lj = ty + ST_H, li = tx + ST_H;
+  T lam[4];
+  if (inner) {
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      lacc[v] = hole ? (T)0 : a.lacc[VOFF[v] + p];
-      lin[v] = (KIND != STAGE_LAST && a.lin && !hole) ? a.lin[VOFF[v] + p] : (T)0;
-      T kv = hb * lacc[v];
-      if (KIND != STAGE_LAST && a.lin) kv += ha * lin[v];
-      kap[v] = kv;
+      lam[v] = fd_row_t_inner<T>(&F[v][lj][li], 1);
+      lam[v] += fd_row_t_inner<T>(&F[4 + v][lj][li], RS);
     }
-    // sponges: r_v -= sigma y_v
-#pragma unroll 1
-    for (int z = 0; z < a.nz; z++) {
-      const ZoneT<T> &zz = a.z[z];
-      if (gi >= zz.i0 && gi <= zz.i1 && gj >= zz.j0 && gj <= zz.j1) {
-        const T sg = zz.sig[(gj - zz.j0) * zz.nzi + (gi - zz.i0)];
+  } else if (HOLES) {
 #pragma unroll
-        for (int v = 0; v < 4; v++) lam[v] += -sg * kap[v];
-      }
+    for (int v = 0; v < 4; v++) {
+      lam[v] = fd_row_t_codes<T>(&F[v][lj][li], 1, gi, ni, a.code, p, 1);
+      lam[v] += fd_row_t_codes<T>(&F[4 + v][lj][li], RS, gj, nj, a.code + n, p, ni);
     }
-    T mur = 0;
-    if (MEANF) {
-      const T u0 = (T)a.mean[IUX * n + p], v0 = (T)a.mean[IUY * n + p];
-      const T rb = (T)a.rhob[p];
-      const T g = (T)a.gamma;
-      const T gsx = (T)a.mgrad[(2 * IS + 0) * n + p], gsy = (T)a.mgrad[(2 * IS + 1) * n + p];
-      const T gux = (T)a.mgrad[(2 * IUX + 0) * n + p], guy = (T)a.mgrad[(2 * IUX + 1) * n + p];
-      const T gvx = (T)a.mgrad[(2 * IUY + 0) * n + p], gvy = (T)a.mgrad[(2 * IUY + 1) * n + p];
-      const T gpx = (T)a.mgrad[(2 * IP + 0) * n + p], gpy = (T)a.mgrad[(2 * IP + 1) * n + p];
-      const T ks = kap[0], ku = kap[1], kv = kap[2], kp = kap[3];
-      lam[1] += -(gsx * ks) - gux * ku - gvx * kv - gpx * kp;
-      lam[2] += -(gsy * ks) - guy * ku - gvy * kv - gpy * kp;
-      lam[3] += -(g * gux * kp) - g * gvy * kp;
-      mur = -((u0 * gux + v0 * guy) * ku + (u0 * gvx + v0 * gvy) * kv) / rb;
-      if (a.rad) {
-        // axisymmetric term r_p -= (gamma pbar v' + gamma vbar p') / r
-        // (spatial:2119-2126), with the forward's gamma pbar and r fields
-        const T rr = a.rad[p], gpb = (T)(a.gamma * a.mean[IP * n + p]);
-        lam[2] += -(gpb / rr) * kp;
-        lam[3] += -(g * v0 / rr) * kp;
-      }
-      if (KIND != STAGE_FIRST) {  // rho' of this stage's input: R(u)
-        const double pb = a.mean[IP * n + p];
-        lam[0] += -(rb * mur);
-        lam[3] += (T)((double)mur * a.rhob[p] * a.gi / pb);
-      }
+  } else {
+    const RowT5<T> rx = row_t5<T>(gi, ni), ry = row_t5<T>(gj, nj);  // ry uniform
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      lam[v] = row_t5_sum<T>(rx, &F[v][lj][li], 1);
+      lam[v] += row_t5_sum<T>(ry, &F[4 + v][lj][li], RS);
     }
-    if (a.grad) a.grad[p] += a.src * (double)kap[3];
-    if (KIND == STAGE_FIRST) {
+  }
+  // kappa at the point (recomputed from the same operands)
+  T kap[4];
+#pragma unroll
+  for (int v = 0; v < 4; v++) {
+    if (hole) lacc[v] = lin[v] = (T)0;
+    T kv = hb * lacc[v];
+    if (KIND != STAGE_LAST && a.lin) kv += ha * lin[v];
+    kap[v] = kv;
+  }
+  // sponges: r_v -= sigma y_v
+  for (unsigned zm = zmask; zm; zm &= zm - 1) {
+    const ZoneT<T> &zz = a.z[__builtin_ctz(zm)];
+    if (gi >= zz.i0 && gi <= zz.i1 && gj >= zz.j0 && gj <= zz.j1) {
+      const T sg = zz.sig[(gj - zz.j0) * zz.nzi + (gi - zz.i0)];
+#pragma unroll
+      for (int v = 0; v < 4; v++) lam[v] += -sg * kap[v];
+    }
+  }
+  T mur = 0;
+  if (MEANF) {
+    const T u0 = (T)mb[0], v0 = (T)mb[1], rb = (T)mb[2];
+    const T g = (T)a.gamma;
+    const T gsx = mg[0], gsy = mg[1], gux = mg[2], guy = mg[3];
+    const T gvx = mg[4], gvy = mg[5], gpx = mg[6], gpy = mg[7];
+    const T ks = kap[0], ku = kap[1], kv = kap[2], kp = kap[3];
+    lam[1] += -(gsx * ks) - gux * ku - gvx * kv - gpx * kp;
+    lam[2] += -(gsy * ks) - guy * ku - gvy * kv - gpy * kp;
+    lam[3] += -(g * gux * kp) - g * gvy * kp;
+    mur = -((u0 * gux + v0 * guy) * ku + (u0 * gvx + v0 * gvy) * kv) / rb;
+    if (a.rad) {
+      // axisymmetric term r_p -= (gamma pbar v' + gamma vbar p') / r
+      // (spatial:2119-2126), with the forward's gamma pbar and r fields
+      const T rr = a.rad[p], gpb = (T)(a.gamma * mb[3]);
+      lam[2] += -(gpb / rr) * kp;
+      lam[3] += -(g * v0 / rr) * kp;
+    }
+    if (KIND != STAGE_FIRST) {  // rho' of this stage's input: R(u)
+      lam[0] += -(rb * mur);
+      lam[3] += (T)((double)mur * mb[2] * a.gi / mb[3]);
+    }
+  }
+  if (a.grad) a.grad[p] = gr + a.src * (double)kap[3];
+  if (KIND == STAGE_FIRST) {
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      T out = lam[v] + lacc[v] + lin[v];
+      if (a.lyin) out += lyin[v];
+      a.lout[VOFF[v] + p] = out;
+    }
+    if (MEANF) a.mu[p] = mur;
+  } else {
+#pragma unroll
+    for (int v = 0; v < 4; v++) a.lout[VOFF[v] + p] = lam[v];
+    if (a.lyout) {
 #pragma unroll
       for (int v = 0; v < 4; v++) {
-        T out = lam[v] + lacc[v] + lin[v];
-        if (a.lyin) out += a.lyin[VOFF[v] + p];
-        a.lout[VOFF[v] + p] = out;
-      }
-      if (MEANF) a.mu[p] = mur;
-    } else {
-#pragma unroll
-      for (int v = 0; v < 4; v++) a.lout[VOFF[v] + p] = lam[v];
-      if (a.lyout) {
-#pragma unroll
-        for (int v = 0; v < 4; v++) {
-          T y = lin[v];
-          if (a.lyin) y += a.lyin[VOFF[v] + p];
-          a.lyout[VOFF[v] + p] = y;
-        }
+        T y = lin[v];
+        if (a.lyin) y += lyin[v];
+        a.lyout[VOFF[v] + p] = y;
       }
     }
   }
@@ -357,14 +383,17 @@ struct AdjFilterArgs {
 // Blocks with holes (HOLES): the forward filter is followed by the hole
 // reset, so the adjoint arriving at a BLANKED point counts as 0, and the
 // transposed rows take the per-point filter codes.
+// What bounds it: latency.  Region and middle sweep go round the threads in
+// line order, and closure rows are weights chosen once per line instead of a
+// branch per tap: 385 x 257 FP64 16.5 -> 6.5 us.
 template <typename T, int ORDER, int TY, bool HOLES>
 __global__ void __launch_bounds__(TPB) k_adj_filter(AdjFilterArgs<T> a) {
-  constexpr int NR = TY + 2 * FL_H, NC = FL_TX + 2 * FL_H, KR = NR / 4;
+  constexpr int NR = TY + 2 * FL_H, NC = FL_TX + 2 * FL_H;
   __shared__ T in[4][NR][NC];
   __shared__ T mid[4][TY][NC];
   const int tile = xcd_tile(blockIdx.x, a.chunk);
   if (tile >= a.ntiles) return;
-  const int tx = threadIdx.x, ty = threadIdx.y;
+  const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
   const int i0 = (tile % a.ntx) * FL_TX, j0 = (tile / a.ntx) * TY;
   const int ni = a.ni, nj = a.nj, n = ni * nj;
   const int VOFF[4] = {IS * n, IUX * n, IUY * n, IP * n};
@@ -374,47 +403,57 @@ __global__ void __launch_bounds__(TPB) k_adj_filter(AdjFilterArgs<T> a) {
                                                    j0 + TY + FL_H))
                            : (i0 >= 2 * FL_H && i0 + FL_TX + 2 * FL_H <= ni && j0 >= 2 * FL_H &&
                               j0 + TY + 2 * FL_H <= nj);
+  // points outside the block read the nearest one inside and store 0
+  auto load = [&](int idx) {
+    const int r = idx / NC, c = idx - r * NC;
+    const int gj = j0 - FL_H + r, gi = i0 - FL_H + c;
+    const int p = min(max(gj, 0), nj - 1) * ni + min(max(gi, 0), ni - 1);
+    const bool ok = gj >= 0 && gj < nj && gi >= 0 && gi < ni && !(HOLES && a.iblank[p] == BLANKED);
 #pragma unroll
-  for (int k = 0; k < KR; k++) {
-    const int r = ty + 4 * k;
-    const int gj = j0 - FL_H + r;
-#pragma unroll
-    for (int half = 0; half < 2; half++) {
-      const int c = half == 0 ? tx : FL_TX + tx;
-      if (half == 1 && tx >= 2 * FL_H) continue;
-      const int gi = i0 - FL_H + c;
-      const bool ok = gj >= 0 && gj < nj && gi >= 0 && gi < ni && !(HOLES && a.iblank[gj * ni + gi] == BLANKED);
-#pragma unroll
-      for (int v = 0; v < 4; v++) in[v][r][c] = ok ? a.src[VOFF[v] + gj * ni + gi] : (T)0;
+    for (int v = 0; v < 4; v++) {
+      const T x = a.src[VOFF[v] + p];
+      in[v][r][c] = ok ? x : (T)0;
     }
+  };
+#pragma unroll
+  for (int q = 0; q < NR * NC / TPB; q++) load(tid + q * TPB);
+  if (tid + NR * NC / TPB * TPB < NR * NC) load(tid + NR * NC / TPB * TPB);
+  // the operands of R^T mu, requested before the barriers
+  const int gi = i0 + tx;
+  double mu[TY / 4], mp[TY / 4], rb[TY / 4];
+#pragma unroll
+  for (int k = 0; k < TY / 4; k++) {
+    const int p = min(j0 + ty + 4 * k, nj - 1) * ni + min(gi, ni - 1);
+    mu[k] = a.mu ? (double)a.mu[p] : 0.0;
+    rb[k] = a.mu ? a.rhob[p] : 0.0;
+    mp[k] = a.mu ? a.mean[IP * n + p] : 1.0;
   }
   __syncthreads();
   // eta^T over the tile rows, every column of the region
+  auto eta = [&](int idx) {
+    const int r = idx / NC, c = idx - r * NC;
+    const int gj = j0 + r, gc = i0 - FL_H + c;
+    if (inner) {  // symmetric interior rows: F^T = F
 #pragma unroll
-  for (int k = 0; k < TY / 4; k++) {
-    const int r = ty + 4 * k;
-    const int gj = j0 + r;
+      for (int v = 0; v < 4; v++) mid[v][r][c] = filter_row<T, ORDER>(&in[v][r + FL_H][c], NC, CODE_INTERIOR);
+    } else if (HOLES) {
+      const bool ok = gj < nj && gc >= 0 && gc < ni && a.code;
 #pragma unroll
-    for (int half = 0; half < 2; half++) {
-      const int c = half == 0 ? tx : FL_TX + tx;
-      if (half == 1 && tx >= 2 * FL_H) continue;
-      const int gi = i0 - FL_H + c;
-      const bool ok = gj < nj && gi >= 0 && gi < ni;
-      if (HOLES && !inner) {
+      for (int v = 0; v < 4; v++)
+        mid[v][r][c] =
+            ok ? flt_row_t_codes<T, ORDER>(&in[v][r + FL_H][c], NC, gj, nj, a.code + n, gj * ni + gc, ni) : (T)0;
+    } else {
+      const FltRowT<T, ORDER> w = flt_row_t<T, ORDER>(gj, nj);
 #pragma unroll
-        for (int v = 0; v < 4; v++)
-          mid[v][r][c] = ok && a.code
-                             ? flt_row_t_codes<T, ORDER>(&in[v][r + FL_H][c], NC, gj, nj, a.code + n, gj * ni + gi, ni)
-                             : (T)0;
-      } else {
-#pragma unroll
-        for (int v = 0; v < 4; v++)
-          mid[v][r][c] = ok ? flt_row_t<T, ORDER>(&in[v][r + FL_H][c], NC, gj, nj, inner) : (T)0;
-      }
+      for (int v = 0; v < 4; v++) mid[v][r][c] = flt_row_t_sum<T, ORDER>(w, &in[v][r + FL_H][c], NC);
     }
-  }
+  };
+#pragma unroll
+  for (int q = 0; q < TY * NC / TPB; q++) eta(tid + q * TPB);
+  if (tid + TY * NC / TPB * TPB < TY * NC) eta(tid + TY * NC / TPB * TPB);
   __syncthreads();
-  const int gi = i0 + tx;
+  FltRowT<T, ORDER> wx{};
+  if (!HOLES && !inner) wx = flt_row_t<T, ORDER>(gi, ni);
 #pragma unroll
   for (int k = 0; k < TY / 4; k++) {
     const int r = ty + 4 * k;
@@ -424,15 +463,17 @@ __global__ void __launch_bounds__(TPB) k_adj_filter(AdjFilterArgs<T> a) {
     T out[4];
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      const T f = (HOLES && !inner) ? (a.code ? flt_row_t_codes<T, ORDER>(&mid[v][r][tx + FL_H], 1, gi, ni, a.code, p, 1)
-                                              : (T)0)
-                                    : flt_row_t<T, ORDER>(&mid[v][r][tx + FL_H], 1, gi, ni, inner);
+      const T *m = &mid[v][r][tx + FL_H];
+      T f;
+      if (inner) f = filter_row<T, ORDER>(m, 1, CODE_INTERIOR);
+      else if (HOLES) f = a.code ? flt_row_t_codes<T, ORDER>(m, 1, gi, ni, a.code, p, 1) : (T)0;
+      else f = flt_row_t_sum<T, ORDER>(wx, m, 1);
       out[v] = a.rem * in[v][r + FL_H][tx + FL_H] + a.blend * f;
     }
     if (a.mu) {
-      const double m = (double)a.mu[p] * a.rhob[p];
+      const double m = mu[k] * rb[k];
       out[0] += (T)(-m);
-      out[3] += (T)(m * a.gi / a.mean[IP * n + p]);
+      out[3] += (T)(m * a.gi / mp[k]);
     }
 #pragma unroll
     for (int v = 0; v < 4; v++) a.dst[VOFF[v] + p] = out[v];
@@ -643,11 +684,10 @@ __global__ void __launch_bounds__(TPB) k_adj_bc_face(T *__restrict__ lam, const 
 template <typename T>
 static hipError_t adj_stage_t(hipStream_t s, lee_handle *h, Block &b, const AdjStage &st) {
   AdjArgs<T> a{};
-  const int R = b.adj_r == 1 ? 1 : 2;  // 8 flux fields of (4R + 4) x 68 points stay within 64 KB of LDS
   a.ni = b.ni;
   a.nj = b.nj;
   a.ntx = (b.ni + ST_TX - 1) / ST_TX;
-  a.nty = (b.nj + 4 * R - 1) / (4 * R);
+  a.nty = (b.nj + ADJ_TY - 1) / ADJ_TY;
   a.ntiles = a.ntx * a.nty;
   a.chunk = (a.ntiles + 7) / 8;
   T *const *L = sizeof(T) == 8 ? (T *const *)b.A64 : (T *const *)b.A32;
@@ -695,8 +735,7 @@ static hipError_t adj_stage_t(hipStream_t s, lee_handle *h, Block &b, const AdjS
   const bool mf = !b.uniform_mean, ho = b.has_holes;
 #define LEE_ADJ(MF, K, HO)                                                                     \
   do {                                                                                         \
-    if (R == 1) hipLaunchKernelGGL((k_adj_stage<T, MF, K, 1, HO>), grid, block, 0, s, a);      \
-    else hipLaunchKernelGGL((k_adj_stage<T, MF, K, 2, HO>), grid, block, 0, s, a);             \
+    hipLaunchKernelGGL((k_adj_stage<T, MF, K, HO>), grid, block, 0, s, a);                     \
   } while (0)
 #define LEE_ADJK(MF, HO)                                          \
   do {                                                            \

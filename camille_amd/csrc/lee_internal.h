@@ -128,7 +128,6 @@ struct Block {
   double *amu64 = nullptr;
   float *amu32 = nullptr;
   double *agrad = nullptr;
-  int adj_r = 2;               // rows per thread of the adjoint stage kernel (1 or 2)
   // observer points of the functional (device) and their weights
   int nobs = 0;
   int *obs_l = nullptr;
