@@ -39,48 +39,6 @@ constexpr int ADJ_Z_CHUNK = 4;
 
 inline unsigned nba(size_t n) { return (unsigned)((n + TPB - 1) / TPB); }
 
-template <typename T, int ORDER>
-__device__ __forceinline__ T flt_wt3(int code, int d) {
-  const int ad = d < 0 ? -d : d;
-  if (ORDER == 8) {
-    if (code == CODE_INTERIOR) {
-      const T c[5] = {(T)(93.0 / 128.0), (T)(7.0 / 32.0), (T)(-7.0 / 64.0), (T)(1.0 / 32.0), (T)(-1.0 / 256.0)};
-      return ad <= 4 ? c[ad] : (T)0;
-    }
-    if (code == CODE_ZERO) return (T)0;
-    const int k = code - CODE_LEFT;
-    const int row = k < 4 ? k : k - 4;
-    if (row <= 1) return ad == 0 ? (T)1 : (T)0;
-    if (row == 2) {
-      const T c[3] = {(T)(5.0 / 8.0), (T)((1.0 / 2.0) / 2.0), (T)((-1.0 / 8.0) / 2.0)};
-      return ad <= 2 ? c[ad] : (T)0;
-    }
-    const T c[4] = {(T)(11.0 / 16.0), (T)((15.0 / 32.0) / 2.0), (T)((-3.0 / 16.0) / 2.0), (T)((1.0 / 32.0) / 2.0)};
-    return ad <= 3 ? c[ad] : (T)0;
-  } else {
-    if (code == CODE_INTERIOR) {
-      const T c[3] = {(T)(5.0 / 8.0), (T)((1.0 / 2.0) / 2.0), (T)((-1.0 / 8.0) / 2.0)};
-      return ad <= 2 ? c[ad] : (T)0;
-    }
-    if (code == CODE_ZERO) return (T)0;
-    return ad == 0 ? (T)1 : (T)0;
-  }
-}
-
-template <typename T, int ORDER>
-__device__ __forceinline__ T flt_t3(const T *f, int st, int c, int len) {
-  constexpr int H = ORDER / 2;
-  if (c >= 2 * H && c <= len - 1 - 2 * H) return filter_row<T, ORDER>(f, st, CODE_INTERIOR);
-  T acc = 0;
-#pragma unroll
-  for (int o = -H; o <= H; o++) {
-    const int j = c + o;
-    if (j < 0 || j >= len) continue;
-    acc += flt_wt3<T, ORDER>(default_code(j, len, H), -o) * f[o * st];
-  }
-  return acc;
-}
-
 template <typename T>
 struct Zone3A {
   int i0, i1, j0, j1, k0, k1, nzi, nzj;
@@ -333,8 +291,14 @@ __global__ void __launch_bounds__(TPB) k_adj_filter3d_z(const T *__restrict__ la
   auto plane_out = [&](int k, const T (&wn)[5]) {
 #pragma unroll
     for (int v = 0; v < 5; v++) w[v][2 * H] = wn[v];
+    if (k >= 2 * H && k <= nk - 1 - 2 * H) {  // uniform; symmetric interior rows: F^T = F
 #pragma unroll
-    for (int v = 0; v < 5; v++) tmp[v * n + (size_t)k * plane + col] = flt_t3<T, ORDER>(&w[v][H], 1, k, nk);
+      for (int v = 0; v < 5; v++) tmp[v * n + (size_t)k * plane + col] = filter_row<T, ORDER>(&w[v][H], 1, CODE_INTERIOR);
+    } else {
+      const FltRowT<T, ORDER> r = flt_row_t<T, ORDER>(k, nk);
+#pragma unroll
+      for (int v = 0; v < 5; v++) tmp[v * n + (size_t)k * plane + col] = flt_row_t_sum<T, ORDER>(r, &w[v][H], 1);
+    }
 #pragma unroll
     for (int v = 0; v < 5; v++)
 #pragma unroll
@@ -376,50 +340,68 @@ struct AdjF3Args {
   T rem, blend;
 };
 
-// eta^T then xi^T sweeps of plane blockIdx.y, blend and R^T mu.
+// eta^T then xi^T sweeps of plane blockIdx.y, blend and R^T mu; region,
+// middle sweep and closure rows as in the 2-D form (k_adj_filter).
+// 112 x 96 x 80 FP32: 66 -> 19 us.
 template <typename T, int ORDER, int TY>
 __global__ void __launch_bounds__(TPB) k_adj_filter3d_plane(AdjF3Args<T> a) {
-  constexpr int NR = TY + 2 * FL_H, NC = FL_TX + 2 * FL_H, KR = NR / 4;
+  constexpr int NR = TY + 2 * FL_H, NC = FL_TX + 2 * FL_H;
   __shared__ T in[5][NR][NC];
   __shared__ T mid[5][TY][NC];
   const int tile = xcd_tile(blockIdx.x, (a.ntiles + 7) / 8);  // XCD-banded tiles of each plane
   if (tile >= a.ntiles) return;
   const int k = blockIdx.y;
-  const int tx = threadIdx.x, ty = threadIdx.y;
+  const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * 64 + tx;
   const int i0 = (tile % a.ntx) * FL_TX, j0 = (tile / a.ntx) * TY;
   const int ni = a.ni, nj = a.nj;
   const size_t plane = (size_t)ni * nj, n = plane * a.nk, off = (size_t)k * plane;
+  const bool inx = i0 >= 2 * FL_H && i0 + FL_TX + 2 * FL_H <= ni;
+  const bool iny = j0 >= 2 * FL_H && j0 + TY + 2 * FL_H <= nj;
+  // points outside the block read the nearest one inside and store 0
+  auto load = [&](int idx) {
+    const int r = idx / NC, c = idx - r * NC;
+    const int gj = j0 - FL_H + r, gi = i0 - FL_H + c;
+    const size_t p = off + (size_t)min(max(gj, 0), nj - 1) * ni + min(max(gi, 0), ni - 1);
+    const bool ok = gj >= 0 && gj < nj && gi >= 0 && gi < ni;
 #pragma unroll
-  for (int kr = 0; kr < KR; kr++) {
-    const int r = ty + 4 * kr;
-    const int gj = j0 - FL_H + r;
-#pragma unroll
-    for (int half = 0; half < 2; half++) {
-      const int c = half == 0 ? tx : FL_TX + tx;
-      if (half == 1 && tx >= 2 * FL_H) continue;
-      const int gi = i0 - FL_H + c;
-      const bool ok = gj >= 0 && gj < nj && gi >= 0 && gi < ni;
-#pragma unroll
-      for (int v = 0; v < 5; v++) in[v][r][c] = ok ? a.tmp[v * n + off + (size_t)gj * ni + gi] : (T)0;
+    for (int v = 0; v < 5; v++) {
+      const T x = a.tmp[v * n + p];
+      in[v][r][c] = ok ? x : (T)0;
     }
-  }
-  __syncthreads();
+  };
+#pragma unroll
+  for (int q = 0; q < NR * NC / TPB; q++) load(tid + q * TPB);
+  if (tid + NR * NC / TPB * TPB < NR * NC) load(tid + NR * NC / TPB * TPB);
+  // the points' own operands, requested before the barriers
+  const int gi = i0 + tx;
+  T orig[TY / 4][5], mu[TY / 4], mrb[TY / 4], mrp[TY / 4];
 #pragma unroll
   for (int kr = 0; kr < TY / 4; kr++) {
-    const int r = ty + 4 * kr;
-    const int gj = j0 + r;
+    const size_t p = off + (size_t)min(j0 + ty + 4 * kr, nj - 1) * ni + min(gi, ni - 1);
 #pragma unroll
-    for (int half = 0; half < 2; half++) {
-      const int c = half == 0 ? tx : FL_TX + tx;
-      if (half == 1 && tx >= 2 * FL_H) continue;
-      const int gi = i0 - FL_H + c;
-      const bool ok = gj < nj && gi >= 0 && gi < ni;
-#pragma unroll
-      for (int v = 0; v < 5; v++) mid[v][r][c] = ok ? flt_t3<T, ORDER>(&in[v][r + FL_H][c], NC, gj, nj) : (T)0;
-    }
+    for (int v = 0; v < 5; v++) orig[kr][v] = a.orig[v * n + p];
+    mu[kr] = a.mu ? a.mu[p] : (T)0;
+    mrb[kr] = a.mu ? a.mc[MC3_RB * n + p] : (T)0;
+    mrp[kr] = a.mu ? a.mc[MC3_RP * n + p] : (T)0;
   }
   __syncthreads();
-  const int gi = i0 + tx;
+  auto eta = [&](int idx) {
+    const int r = idx / NC, c = idx - r * NC;
+    if (iny) {
+#pragma unroll
+      for (int v = 0; v < 5; v++) mid[v][r][c] = filter_row<T, ORDER>(&in[v][r + FL_H][c], NC, CODE_INTERIOR);
+    } else {
+      const FltRowT<T, ORDER> w = flt_row_t<T, ORDER>(j0 + r, nj);
+#pragma unroll
+      for (int v = 0; v < 5; v++) mid[v][r][c] = flt_row_t_sum<T, ORDER>(w, &in[v][r + FL_H][c], NC);
+    }
+  };
+#pragma unroll
+  for (int q = 0; q < TY * NC / TPB; q++) eta(tid + q * TPB);
+  if (tid + TY * NC / TPB * TPB < TY * NC) eta(tid + TY * NC / TPB * TPB);
+  __syncthreads();
+  FltRowT<T, ORDER> wx{};
+  if (!inx) wx = flt_row_t<T, ORDER>(gi, ni);
 #pragma unroll
   for (int kr = 0; kr < TY / 4; kr++) {
     const int r = ty + 4 * kr;
@@ -429,13 +411,13 @@ __global__ void __launch_bounds__(TPB) k_adj_filter3d_plane(AdjF3Args<T> a) {
     T out[5];
 #pragma unroll
     for (int v = 0; v < 5; v++) {
-      const T f = flt_t3<T, ORDER>(&mid[v][r][tx + FL_H], 1, gi, ni);
-      out[v] = a.rem * a.orig[v * n + p] + a.blend * f;
+      const T *m = &mid[v][r][tx + FL_H];
+      const T f = inx ? filter_row<T, ORDER>(m, 1, CODE_INTERIOR) : flt_row_t_sum<T, ORDER>(wx, m, 1);
+      out[v] = a.rem * orig[kr][v] + a.blend * f;
     }
     if (a.mu) {
-      const T m = a.mu[p];
-      out[IS] += -(a.mc[MC3_RB * n + p] * m);
-      out[IP] += a.mc[MC3_RP * n + p] * m;
+      out[IS] += -(mrb[kr] * mu[kr]);
+      out[IP] += mrp[kr] * mu[kr];
     }
 #pragma unroll
     for (int v = 0; v < 5; v++) a.dst[v * n + p] = out[v];

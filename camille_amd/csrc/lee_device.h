@@ -186,6 +186,68 @@ __device__ __forceinline__ T row_t5_sum(const RowT5<T> &r, const T *f, int st) {
   return acc;
 }
 
+// Weight of the filter row with code `code` on offset d (rows are centred
+// and symmetric; filter_row in lee_device.h).
+template <typename T, int ORDER>
+__device__ __forceinline__ T flt_wt(int code, int d) {
+  const int ad = d < 0 ? -d : d;
+  if (ORDER == 8) {
+    if (code == CODE_INTERIOR) {
+      const T c[5] = {(T)(93.0 / 128.0), (T)(7.0 / 32.0), (T)(-7.0 / 64.0), (T)(1.0 / 32.0), (T)(-1.0 / 256.0)};
+      return ad <= 4 ? c[ad] : (T)0;
+    }
+    if (code == CODE_ZERO) return (T)0;
+    const int k = code - CODE_LEFT;
+    const int row = k < 4 ? k : k - 4;
+    if (row <= 1) return ad == 0 ? (T)1 : (T)0;
+    if (row == 2) {
+      const T c[3] = {(T)(5.0 / 8.0), (T)((1.0 / 2.0) / 2.0), (T)((-1.0 / 8.0) / 2.0)};
+      return ad <= 2 ? c[ad] : (T)0;
+    }
+    const T c[4] = {(T)(11.0 / 16.0), (T)((15.0 / 32.0) / 2.0), (T)((-3.0 / 16.0) / 2.0), (T)((1.0 / 32.0) / 2.0)};
+    return ad <= 3 ? c[ad] : (T)0;
+  } else {
+    if (code == CODE_INTERIOR) {
+      const T c[3] = {(T)(5.0 / 8.0), (T)((1.0 / 2.0) / 2.0), (T)((-1.0 / 8.0) / 2.0)};
+      return ad <= 2 ? c[ad] : (T)0;
+    }
+    if (code == CODE_ZERO) return (T)0;
+    return ad == 0 ? (T)1 : (T)0;
+  }
+}
+
+// Transposed filter row at coordinate c of a line of length len (no holes)
+// as weights of the neighbours c + o, o in [-H, H]: the rows there that
+// exist, chosen by selects.  Filter rows are symmetric, so row j counts with
+// its weight at distance |o|.
+template <typename T, int ORDER>
+struct FltRowT {
+  static constexpr int H = ORDER / 2;
+  T w[2 * H + 1];
+};
+template <typename T, int ORDER>
+__device__ __forceinline__ FltRowT<T, ORDER> flt_row_t(int c, int len) {
+  constexpr int H = ORDER / 2;
+  FltRowT<T, ORDER> r;
+#pragma unroll
+  for (int o = -H; o <= H; o++) {
+    const int j = c + o, row = j < H ? j : min(len - 1 - j, H);  // default_code
+    T w = flt_wt<T, ORDER>(CODE_INTERIOR, o);
+#pragma unroll
+    for (int k = 0; k < H; k++) w = row == k ? flt_wt<T, ORDER>(CODE_LEFT + k, o) : w;
+    r.w[o + H] = j >= 0 && j < len ? w : (T)0;
+  }
+  return r;
+}
+template <typename T, int ORDER>
+__device__ __forceinline__ T flt_row_t_sum(const FltRowT<T, ORDER> &r, const T *f, int st) {
+  constexpr int H = ORDER / 2;
+  T acc = r.w[0] * f[-H * st];
+#pragma unroll
+  for (int o = 1 - H; o <= H; o++) acc += r.w[o + H] * f[o * st];
+  return acc;
+}
+
 template <typename T>
 struct ZoneT {
   int i0, i1, j0, j1, nzi;
