@@ -26,16 +26,28 @@ namespace lee {
 
 namespace {
 
-constexpr int A3_TY = 4;
+constexpr int A3_TX = 32, A3_TY = 8;  // points of a stage tile
 constexpr int A3_ZC = 16;      // most planes per chunk of the zeta^T filter pass (at least 4, z_chunk)
-// Planes per workgroup of the adjoint stage (see STAGE_Z_CHUNK of the
-// forward stage; here a chunk's four extra planes cost a flux evaluation
-// each, so 4 planes instead of 2).  Whole reverse step (recomputed forward
-// step, adjoint step), FP32 / FP64: 48 x 40 x 32 2377 / 2832 us with 32
-// planes, 445 / 519 with 4, 308 / 354 with 2, 249 / 292 with 1;
-// 144 x 120 x 112 3856 / 5033, 2043 / 3644, 2045 / 3691, 2249 / 3907;
-// 256 x 200 x 256 11289 / 20657, 9915 / 18102, 10315 / 18939, 11055 / 20816.
-constexpr int ADJ_Z_CHUNK = 4;
+// Planes per workgroup of the adjoint stage when `slots` workgroups are
+// resident: the fewest rounds of workgroups times planes each marches, with
+// two more for the start of its column; up to 10, past which little is
+// shared.  Whole reverse step with 4 planes whatever the block and with this
+// rule, FP32 / FP64: 112 x 96 x 80 640 / 960 -> 516 / 906 us (5 and 8
+// planes), 144 x 120 x 112 1389 / 2515 -> 1332 / 2376 (6 and 6), 256 x 200 x
+// 256 7770 / 13339 -> 7402 / 12877; 48 x 40 x 32 208 / 275 -> 147 / 185 (1).
+inline int adj_z_chunk(int tiles, int nk, int slots) {
+  int best = 1;
+  long long cost = -1;
+  for (int zc = 1; zc <= 10 && zc <= nk; zc++) {
+    const long long groups = (long long)tiles * ((nk + zc - 1) / zc);
+    const long long c = (groups + slots - 1) / slots * (zc + 2);
+    if (cost < 0 || c < cost) {
+      cost = c;
+      best = zc;
+    }
+  }
+  return best;
+}
 
 inline unsigned nba(size_t n) { return (unsigned)((n + TPB - 1) / TPB); }
 
@@ -60,60 +72,69 @@ struct Adj3Args {
   double hb, ha, src;
 };
 
-// kappa and the three flux vectors (5 variables) at point p of plane k.
+// kappa and the mean flow at a point, and from them the flux vector of one
+// direction with its metrics m: F_l = -J (U_l kappa + ...) with the
+// contravariant velocity U_l = m . ubar.
+struct AdjPoint3 {
+  double kap[5], ub[3], c, irb, J;  // c = gamma p kappa_p; J the negative Jacobian
+};
+
 template <typename T, bool MEANF, int KIND>
-__device__ __forceinline__ void adj_flux3(const Adj3Args<T> &a, size_t p, size_t n, T kap[5], T F[3][5]) {
+__device__ __forceinline__ AdjPoint3 adj_point3(const Adj3Args<T> &a, size_t p, size_t n) {
+  AdjPoint3 q;
   const T hb = (T)a.hb, ha = (T)a.ha;
 #pragma unroll
   for (int v = 0; v < 5; v++) {
     T kv = hb * a.lacc[v * n + p];
     if (KIND != STAGE_LAST && a.lin) kv += ha * a.lin[v * n + p];
-    kap[v] = kv;
+    q.kap[v] = kv;
   }
-  double ub[3] = {a.u0, a.v0, a.w0}, gp = a.gp0, irb = 1.0 / a.rhob0;
+  double gp = a.gp0;
+  q.ub[0] = a.u0;
+  q.ub[1] = a.v0;
+  q.ub[2] = a.w0;
   if (MEANF) {
-    ub[0] = mean_field3(a.mc, a.varies, MC3_U, n, p);
-    ub[1] = mean_field3(a.mc, a.varies, MC3_V, n, p);
-    ub[2] = mean_field3(a.mc, a.varies, MC3_W, n, p);
+    q.ub[0] = mean_field3(a.mc, a.varies, MC3_U, n, p);
+    q.ub[1] = mean_field3(a.mc, a.varies, MC3_V, n, p);
+    q.ub[2] = mean_field3(a.mc, a.varies, MC3_W, n, p);
     gp = mean_field3(a.mc, a.varies, MC3_GP, n, p);
-    irb = mean_field3(a.mc, a.varies, MC3_IRB, n, p);
+    q.irb = mean_field3(a.mc, a.varies, MC3_IRB, n, p);
+  } else {
+    q.irb = 1.0 / a.rhob0;
   }
-  // F_l = -J (U_l kappa + ...) with the contravariant velocity U_l = m_l . ubar
-  const double ks = kap[IS], ku[3] = {kap[IUX], kap[IUY], kap[IUZ]}, kp = kap[IP];
-  const double c = gp * kp;
-  double m[3][3];
-#pragma unroll
-  for (int l = 0; l < 3; l++)
-#pragma unroll
-    for (int i = 0; i < 3; i++) m[l][i] = a.met[(size_t)(3 * l + i) * n + p];
-  const double J = -a.jac[p];
-#pragma unroll
-  for (int l = 0; l < 3; l++) {
-    const double U = m[l][0] * ub[0] + m[l][1] * ub[1] + m[l][2] * ub[2];
-    F[l][IS] = (T)(U * ks * J);
-#pragma unroll
-    for (int i = 0; i < 3; i++) F[l][IUX + i] = (T)((U * ku[i] + m[l][i] * c) * J);
-    F[l][IP] = (T)((U * kp + (m[l][0] * ku[0] + m[l][1] * ku[1] + m[l][2] * ku[2]) * irb) * J);
-  }
+  q.c = gp * q.kap[IP];
+  q.J = -a.jac[p];
+  return q;
 }
 
-// What bounds it: latency and FP64 arithmetic (a flux evaluation is some 75
-// FP64 operations, 3.1 of them a point with the halo) more than its 268 bytes
-// a point.  Fluxes through the contravariant velocity (19 operations a
-// direction instead of 29), the halo's points spread over the workgroup, the
-// point's own operands requested before the barrier and transposed closure
-// rows without branches: whole reverse step, FP32 / FP64, 112 x 96 x 80 836 /
-// 1238 -> 607 / 1106 us, 256 x 200 x 256 9632 / 16118 -> 8145 / 14972.
+template <typename T>
+__device__ __forceinline__ void adj_dir3(const AdjPoint3 &q, double m0, double m1, double m2, T (&F)[5]) {
+  const double U = m0 * q.ub[0] + m1 * q.ub[1] + m2 * q.ub[2], m[3] = {m0, m1, m2};
+  F[IS] = (T)(U * q.kap[IS] * q.J);
+#pragma unroll
+  for (int i = 0; i < 3; i++) F[IUX + i] = (T)((U * q.kap[IUX + i] + m[i] * q.c) * q.J);
+  F[IP] = (T)((U * q.kap[IP] + (m0 * q.kap[IUX] + m1 * q.kap[IUY] + m2 * q.kap[IUZ]) * q.irb) * q.J);
+}
+
+// What bounds it: the wait for its operands (four fifths of a wave's time);
+// a flux evaluation is some 75 FP64 operations.  Tiles of 32 x 8 points hold
+// their own fluxes in registers from the plane that first needs them, so a
+// point is evaluated once and its halo lanes (160 beside 256 points, one
+// direction each) once: 1.2 evaluations a point.  A 64 x 4 tile that
+// evaluated plane k with its whole halo again took 3.1.  Whole reverse step
+// before, FP32 / FP64: 112 x 96 x 80 537 / 1039 -> 504 / 863 us, 144 x 120 x
+// 112 1567 / 2935 -> 1284 / 2263, 256 x 200 x 256 7816 / 14353 -> 7102 / 12198.
 template <typename T, bool MEANF, int KIND>
 __global__ void __launch_bounds__(TPB) k_adj_stage3d(Adj3Args<T> a) {
-  constexpr int RS = ST_TX + 2 * ST_H, NR = A3_TY + 2 * ST_H;
-  __shared__ T S[10][NR][RS];  // xi fluxes then eta fluxes of the 5 variables
+  constexpr int H = ST_H;
+  __shared__ T SX[5][A3_TY][A3_TX + 2 * H];  // xi fluxes of plane k with their halo columns
+  __shared__ T SE[5][A3_TY + 2 * H][A3_TX];  // eta fluxes with their halo rows
   // XCD-banded tiles within each z chunk, as the forward stage
   const int ntl = a.ntx * a.nty;
   const int tile = xcd_tile(blockIdx.x, (ntl + 7) / 8);
   if (tile >= ntl) return;
-  const int tx = threadIdx.x, ty = __builtin_amdgcn_readfirstlane((int)threadIdx.y);  // a wave is one row
-  const int i0 = (tile % a.ntx) * ST_TX, j0 = (tile / a.ntx) * A3_TY;
+  const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * A3_TX + tx;
+  const int i0 = (tile % a.ntx) * A3_TX, j0 = (tile / a.ntx) * A3_TY;
   const int k0 = blockIdx.y * a.zc, k1 = min(k0 + a.zc, a.nk);
   const int ni = a.ni, nj = a.nj, nk = a.nk;
   const size_t plane = (size_t)ni * nj, n = plane * nk;
@@ -121,53 +142,60 @@ __global__ void __launch_bounds__(TPB) k_adj_stage3d(Adj3Args<T> a) {
   const bool own = gi < ni && gj < nj;
   const size_t col = own ? (size_t)gj * ni + gi : 0;
   const RowT5<T> rx = row_t5<T>(gi, ni), ry = row_t5<T>(gj, nj);
-  const unsigned zmask = zones_meeting3(a.z, a.nz, i0, i0 + ST_TX - 1, j0, j0 + A3_TY - 1, k0, k1 - 1);
-  // zeta fluxes of the own column, planes k - 2 .. k + 2
-  T wz[5][5];
+  const unsigned zmask = zones_meeting3(a.z, a.nz, i0, i0 + A3_TX - 1, j0, j0 + A3_TY - 1, k0, k1 - 1);
+  // fluxes of the own column: zeta of planes k - 2 .. k + 2, xi and eta of
+  // k .. k + 2 (each point of the tile is evaluated once per chunk)
+  T wz[5][5], wx[5][3], we[5][3];
+  auto column = [&](int kk, int q) {
+    T f[3][5];
+    if (kk >= 0 && kk < nk) {  // uniform
+      const size_t p = (size_t)kk * plane + col;
+      const AdjPoint3 pt = adj_point3<T, MEANF, KIND>(a, p, n);
 #pragma unroll
-  for (int q = 0; q < 4; q++) {
-    const int kk = k0 - 2 + q;
-    T kap[5], F[3][5];
-    if (own && kk >= 0 && kk < nk) adj_flux3<T, MEANF, KIND>(a, (size_t)kk * plane + col, n, kap, F);
-    else
-#pragma unroll
-      for (int v = 0; v < 5; v++) F[2][v] = (T)0;
-#pragma unroll
-    for (int v = 0; v < 5; v++) wz[v][q] = F[2][v];
-  }
-  for (int k = k0; k < k1; k++) {
-    {
-      const int kk = k + 2;
-      T kap[5], F[3][5];
-      if (own && kk < nk) adj_flux3<T, MEANF, KIND>(a, (size_t)kk * plane + col, n, kap, F);
-      else
-#pragma unroll
-        for (int v = 0; v < 5; v++) F[2][v] = (T)0;
-#pragma unroll
-      for (int v = 0; v < 5; v++) wz[v][4] = F[2][v];
+      for (int l = 0; l < 3; l++)
+        adj_dir3<T>(pt, a.met[(size_t)(3 * l) * n + p], a.met[(size_t)(3 * l + 1) * n + p],
+                    a.met[(size_t)(3 * l + 2) * n + p], f[l]);
     }
-    // xi and eta fluxes of plane k over the tile and its halo: its points in
-    // line order over the 256 threads, two each and 32 more (a row and its
-    // halo columns at a time cost every wave two evaluations for four lanes);
-    // points outside the block evaluate the nearest one inside and store 0
-    auto ring = [&](int idx) {
-      const int r = idx / RS, c = idx - r * RS;
-      const int rj = j0 - ST_H + r, ri = i0 - ST_H + c;
-      const bool ok = rj >= 0 && rj < nj && ri >= 0 && ri < ni;
-      T kap[5], F[3][5];
-      adj_flux3<T, MEANF, KIND>(
-          a, (size_t)k * plane + (size_t)min(max(rj, 0), nj - 1) * ni + min(max(ri, 0), ni - 1), n, kap, F);
+    const bool ok = own && kk >= 0 && kk < nk;
+#pragma unroll
+    for (int v = 0; v < 5; v++) {
+      wz[v][q] = ok ? f[2][v] : (T)0;
+      if (q >= 2) {
+        wx[v][q - 2] = ok ? f[0][v] : (T)0;
+        we[v][q - 2] = ok ? f[1][v] : (T)0;
+      }
+    }
+  };
+#pragma unroll
+  for (int q = 0; q < 4; q++) column(k0 - 2 + q, q);
+  // the halo of a plane, a point and direction per lane: four rows beside the
+  // tile (eta fluxes, waves 0 and 1) and four columns (xi, half of wave 2)
+  static_assert(A3_TX == 32 && A3_TY == 8 && TPB == 256, "halo lanes");
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), hs = (tid >> 2) & 7, hq = wave < 2 ? tid >> 5 : tid & 3;
+  const int hr = wave < 2 ? (hq < 2 ? hq : hq + A3_TY) : hs;       // row of SE or SX
+  const int hc = wave < 2 ? tx : (hq < 2 ? hq : hq + A3_TX);       // and column
+  const int hj = wave < 2 ? j0 - H + hr : j0 + hr, hi = wave < 2 ? i0 + hc : i0 - H + hc;
+  const bool hon = tid < 160, hok = hj >= 0 && hj < nj && hi >= 0 && hi < ni;
+  const size_t hp = (size_t)min(max(hj, 0), nj - 1) * ni + min(max(hi, 0), ni - 1);
+  const double *hm = a.met + (wave < 2 ? (size_t)3 * n : 0);
+  for (int k = k0; k < k1; k++) {
+    column(k + 2, 4);
+    if (hon) {
+      const size_t p = (size_t)k * plane + hp;
+      const AdjPoint3 pt = adj_point3<T, MEANF, KIND>(a, p, n);
+      T f[5];
+      adj_dir3<T>(pt, hm[p], hm[n + p], hm[2 * n + p], f);
 #pragma unroll
       for (int v = 0; v < 5; v++) {
-        S[v][r][c] = ok ? F[0][v] : (T)0;
-        S[5 + v][r][c] = ok ? F[1][v] : (T)0;
+        T *to = wave < 2 ? &SE[v][hr][hc] : &SX[v][hr][hc];
+        *to = hok ? f[v] : (T)0;
       }
-    };
-    const int tid = ty * 64 + tx;
-    static_assert(NR * RS > 2 * TPB && NR * RS <= 3 * TPB, "two full passes and a short one");
-    ring(tid);
-    ring(tid + TPB);
-    if (tid + 2 * TPB < NR * RS) ring(tid + 2 * TPB);
+    }
+#pragma unroll
+    for (int v = 0; v < 5; v++) {
+      SX[v][ty][tx + H] = wx[v][0];
+      SE[v][ty + H][tx] = we[v][0];
+    }
     // the own point's operands, requested before the barrier
     const size_t p = (size_t)k * plane + col;
     T lacc[5], lin[5], lyin[5], mcv[MC3_COUNT];
@@ -188,8 +216,8 @@ __global__ void __launch_bounds__(TPB) k_adj_stage3d(Adj3Args<T> a) {
       T lam[5];
 #pragma unroll
       for (int v = 0; v < 5; v++) {
-        lam[v] = row_t5_sum<T>(rx, &S[v][ty + ST_H][tx + ST_H], 1);
-        lam[v] += row_t5_sum<T>(ry, &S[5 + v][ty + ST_H][tx + ST_H], RS);
+        lam[v] = row_t5_sum<T>(rx, &SX[v][ty][tx + H], 1);
+        lam[v] += row_t5_sum<T>(ry, &SE[v][ty + H][tx], A3_TX);
         lam[v] += row_t5_sum<T>(rz, &wz[v][2], 1);
       }
       T kap[5];
@@ -263,9 +291,15 @@ __global__ void __launch_bounds__(TPB) k_adj_stage3d(Adj3Args<T> a) {
     }
     __syncthreads();
 #pragma unroll
-    for (int v = 0; v < 5; v++)
+    for (int v = 0; v < 5; v++) {
 #pragma unroll
       for (int q = 0; q < 4; q++) wz[v][q] = wz[v][q + 1];
+#pragma unroll
+      for (int q = 0; q < 2; q++) {
+        wx[v][q] = wx[v][q + 1];
+        we[v][q] = we[v][q + 1];
+      }
+    }
   }
 }
 
@@ -444,9 +478,9 @@ static hipError_t adj_stage3d_t(hipStream_t s, lee_handle *h, Block &b, const Ad
   a.ni = b.ni;
   a.nj = b.nj;
   a.nk = b.nk;
-  a.ntx = (b.ni + ST_TX - 1) / ST_TX;
+  a.ntx = (b.ni + A3_TX - 1) / A3_TX;
   a.nty = (b.nj + A3_TY - 1) / A3_TY;
-  a.zc = z_chunk((a.ntx * a.nty + 7) / 8 * 8, b.nk, ADJ_Z_CHUNK, b.cus);
+  a.zc = adj_z_chunk((a.ntx * a.nty + 7) / 8 * 8, b.nk, b.cus * (sizeof(T) == 8 ? 2 : b.uniform_mean ? 4 : 3));
   a.nzc = (b.nk + a.zc - 1) / a.zc;
   T *const *L = sizeof(T) == 8 ? (T *const *)b.A64 : (T *const *)b.A32;
   auto buf = [&](int k) -> T * { return k < 0 ? nullptr : L[k]; };
@@ -484,7 +518,7 @@ static hipError_t adj_stage3d_t(hipStream_t s, lee_handle *h, Block &b, const Ad
   a.hb = st.hb;
   a.ha = st.ha;
   a.src = st.src;
-  const dim3 grid((a.ntx * a.nty + 7) / 8 * 8, a.nzc), block(ST_TX, A3_TY);
+  const dim3 grid((a.ntx * a.nty + 7) / 8 * 8, a.nzc), block(A3_TX, A3_TY);
   const bool mf = !b.uniform_mean;
 #define LEE_A3(MF)                                                                                            \
   do {                                                                                                        \
