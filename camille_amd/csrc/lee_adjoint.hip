@@ -111,87 +111,116 @@ struct AdjArgs {
   const T *rad;                 // axisymmetric runs: the forward's radius field r + 1e-99 (null: none)
 };
 
-constexpr int ADJ_TY = 4;
+constexpr int ADJ_TX = 32, ADJ_TY = 8;  // points of a tile
 
 // What bounds it: latency, of the fluxes' operands and of each tile's serial
-// work, more than its 296 bytes a point (FP64, general mean).  Tiles of 4
-// rows (2.1 fluxes a point, but twice the workgroups of 8 rows: reverse step
-// of 385 x 257 FP64 98 against 108 us, 1025 x 513 286 against 296, 2049 x
-// 1025 1120 against 1111), the region spread over the threads in line order,
-// the point's operands requested before the barrier, transposed closure rows
-// without branches: middle stage of 385 x 257 FP64 25 -> 12.8 us.
-// One reversed RK stage on a 64 x 4 tile: kappa and the flux fields on the
-// tile and its 2-point halo go to LDS, then the transposed stencils, the
-// point-local transposed terms and the accumulations of the running
-// adjoints.
+// work, more than its 296 bytes a point (FP64, general mean).  Tiles of 32 x
+// 8 points, their halo one direction a lane (1.3 evaluations a point), the
+// point's operands requested before the barrier, transposed closure rows
+// without branches.  Middle stage of 385 x 257 FP64: 25 us with 64 x 8 tiles
+// whose halo went eight lanes at a time, 12.7 with 64 x 4 tiles and the whole
+// region in both directions, 11.4 now; whole reverse step of 1025 x 513 268
+// -> 255, of 2049 x 1025 1087 -> 1051 against the second form.
+// One reversed RK stage on a tile: kappa and the flux fields on the tile and
+// its 2-point halo go to LDS, then the transposed stencils, the point-local
+// transposed terms and the accumulations of the running adjoints.
 // Blocks with holes (HOLES): the forward stage writes 0 at BLANKED points
 // whatever its inputs, so the adjoints arriving there (lacc, lin) count as 0
 // and kappa vanishes there; the transposed rows take the per-point codes.
 template <typename T, bool MEANF, int KIND, bool HOLES>
 __global__ void __launch_bounds__(TPB) k_adj_stage(AdjArgs<T> a) {
-  constexpr int TY = ADJ_TY, NR = TY + 2 * ST_H, RS = ST_TX + 2 * ST_H;
-  __shared__ T F[8][NR][RS];  // F[v] xi-flux, F[4 + v] eta-flux
+  constexpr int H = ST_H;
+  __shared__ T FX[4][ADJ_TY][ADJ_TX + 2 * H];  // xi fluxes with their halo columns
+  __shared__ T FE[4][ADJ_TY + 2 * H][ADJ_TX];  // eta fluxes with their halo rows
   const int tile = xcd_tile(blockIdx.x, a.chunk);
   if (tile >= a.ntiles) return;
-  const int tx = threadIdx.x, ty = __builtin_amdgcn_readfirstlane((int)threadIdx.y);  // a wave is one row
-  const int i0 = (tile % a.ntx) * ST_TX, j0 = (tile / a.ntx) * TY;
+  const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * ADJ_TX + tx;
+  const int i0 = (tile % a.ntx) * ADJ_TX, j0 = (tile / a.ntx) * ADJ_TY;
   const int ni = a.ni, nj = a.nj, n = ni * nj;
   const int VOFF[4] = {IS * n, IUX * n, IUY * n, IP * n};
-  const bool inner = HOLES ? box_clean(a.clean, ni, nj, i0 - ST_H, i0 + ST_TX + ST_H, j0 - ST_H, j0 + TY + ST_H)
-                           : (i0 >= 2 * ST_H && i0 + ST_TX + 2 * ST_H <= ni && j0 >= 2 * ST_H &&
-                              j0 + TY + 2 * ST_H <= nj);
+  const bool inner = HOLES ? box_clean(a.clean, ni, nj, i0 - H, i0 + ADJ_TX + H, j0 - H, j0 + ADJ_TY + H)
+                           : (i0 >= 2 * H && i0 + ADJ_TX + 2 * H <= ni && j0 >= 2 * H && j0 + ADJ_TY + 2 * H <= nj);
   const T hb = (T)a.hb, ha = (T)a.ha;
   // sponge zones of the tile: the boxes are kernel arguments at fixed places,
   // read all at once
   unsigned zmask = 0;
 #pragma unroll
   for (int z = 0; z < MAX_ZONES; z++)
-    zmask |= z < a.nz && a.z[z].i0 < i0 + ST_TX && a.z[z].i1 >= i0 && a.z[z].j0 < j0 + TY && a.z[z].j1 >= j0
+    zmask |= z < a.nz && a.z[z].i0 < i0 + ADJ_TX && a.z[z].i1 >= i0 && a.z[z].j0 < j0 + ADJ_TY && a.z[z].j1 >= j0
                  ? 1u << z : 0;
 
-  // (1) kappa and fluxes over the tile plus halo, in line order over the
-  // threads; points outside the block evaluate the nearest one inside and
-  // store 0
-  auto ring = [&](int idx) {
-    const int r = idx / RS, c = idx - r * RS;
-    const int rj = j0 - ST_H + r, ri = i0 - ST_H + c;
-    const int p = min(max(rj, 0), nj - 1) * ni + min(max(ri, 0), ni - 1);
-    const bool ok = rj >= 0 && rj < nj && ri >= 0 && ri < ni && !(HOLES && a.iblank[p] == BLANKED);
-    T kap[4];
+  // (1) kappa and fluxes: every thread's own point in both directions, then
+  // a point of the halo, in the direction that reads it, by 160 lanes (four
+  // rows by waves 0 and 1, four columns by half of wave 2); points outside
+  // the block evaluate the nearest one inside and store 0
+  struct Point {
+    double k[4], u0, v0, c, irb, J;  // c = gamma p kappa_p; J the negative Jacobian
+    bool ok;
+  };
+  auto point = [&](int ri, int rj, int p) {
+    Point q;
+    q.ok = rj >= 0 && rj < nj && ri >= 0 && ri < ni && !(HOLES && a.iblank[p] == BLANKED);
 #pragma unroll
     for (int v = 0; v < 4; v++) {
       T kv = hb * a.lacc[VOFF[v] + p];
       if (KIND != STAGE_LAST && a.lin) kv += ha * a.lin[VOFF[v] + p];
-      kap[v] = kv;
+      q.k[v] = kv;
     }
-    double u0 = a.u0, v0 = a.v0, gp = a.gp0, irb = 1.0 / a.rhob0;
+    double gp = a.gp0;
+    q.u0 = a.u0;
+    q.v0 = a.v0;
+    q.irb = 1.0 / a.rhob0;
     if (MEANF) {
-      u0 = a.mean[IUX * n + p];
-      v0 = a.mean[IUY * n + p];
+      q.u0 = a.mean[IUX * n + p];
+      q.v0 = a.mean[IUY * n + p];
       gp = a.gamma * a.mean[IP * n + p];
-      irb = 1.0 / a.rhob[p];
+      q.irb = 1.0 / a.rhob[p];
     }
-    const double ks = kap[0], ku = kap[1], kv = kap[2], kp = kap[3], c0 = gp * kp;
-    const double m[2][2] = {{a.met[p], a.met[(size_t)n + p]}, {a.met[(size_t)2 * n + p], a.met[(size_t)3 * n + p]}};
-    const double J = -a.jac[p];
-    // F_l = -J (U_l kappa + ...) with the contravariant velocity U_l
-#pragma unroll
-    for (int l = 0; l < 2; l++) {
-      const double U = m[l][0] * u0 + m[l][1] * v0;
-      const double f[4] = {U * ks * J, (U * ku + m[l][0] * c0) * J, (U * kv + m[l][1] * c0) * J,
-                           (U * kp + (m[l][0] * ku + m[l][1] * kv) * irb) * J};
-#pragma unroll
-      for (int v = 0; v < 4; v++) F[4 * l + v][r][c] = ok ? (T)f[v] : (T)0;
-    }
+    q.c = gp * q.k[3];
+    q.J = -a.jac[p];
+    return q;
   };
-  const int tid = ty * 64 + tx;
-#pragma unroll
-  for (int q = 0; q < NR * RS / TPB; q++) ring(tid + q * TPB);
-  if (tid + NR * RS / TPB * TPB < NR * RS) ring(tid + NR * RS / TPB * TPB);
-
-  // (2) the operands of the thread's point, requested before the barrier
+  // F_l = -J (U_l kappa + ...) with the contravariant velocity U_l
+  auto flux = [&](const Point &q, double mx, double my, T (&f)[4]) {
+    const double U = mx * q.u0 + my * q.v0;
+    f[0] = (T)(U * q.k[0] * q.J);
+    f[1] = (T)((U * q.k[1] + mx * q.c) * q.J);
+    f[2] = (T)((U * q.k[2] + my * q.c) * q.J);
+    f[3] = (T)((U * q.k[3] + (mx * q.k[1] + my * q.k[2]) * q.irb) * q.J);
+  };
   const int gi = i0 + tx, gj = j0 + ty;
   const int p = min(gj, nj - 1) * ni + min(gi, ni - 1);
+  {
+    const Point q = point(gi, gj, p);
+    T f[2][4];
+#pragma unroll
+    for (int l = 0; l < 2; l++)
+      flux(q, a.met[(size_t)(2 * l) * n + p], a.met[(size_t)(2 * l + 1) * n + p], f[l]);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      FX[v][ty][tx + H] = q.ok ? f[0][v] : (T)0;
+      FE[v][ty + H][tx] = q.ok ? f[1][v] : (T)0;
+    }
+  }
+  static_assert(ADJ_TX == 32 && ADJ_TY == 8 && TPB == 256, "halo lanes");
+  if (tid < 160) {
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6), hq = wave < 2 ? tid >> 5 : tid & 3;
+    const int hr = wave < 2 ? (hq < 2 ? hq : hq + ADJ_TY) : (tid >> 2) & 7;  // row of FE or FX
+    const int hc = wave < 2 ? tx : (hq < 2 ? hq : hq + ADJ_TX);              // and column
+    const int hj = wave < 2 ? j0 - H + hr : j0 + hr, hi = wave < 2 ? i0 + hc : i0 - H + hc;
+    const int hp = min(max(hj, 0), nj - 1) * ni + min(max(hi, 0), ni - 1);
+    const double *hm = a.met + (wave < 2 ? (size_t)2 * n : 0);
+    const Point q = point(hi, hj, hp);
+    T f[4];
+    flux(q, hm[hp], hm[(size_t)n + hp], f);
+#pragma unroll
+    for (int v = 0; v < 4; v++) {
+      T *to = wave < 2 ? &FE[v][hr][hc] : &FX[v][hr][hc];
+      *to = q.ok ? f[v] : (T)0;
+    }
+  }
+
+  // (2) the operands of the thread's point, requested before the barrier
   T lacc[4], lin[4], lyin[4], mg[8];
   double mb[4];
   const bool hole = HOLES && a.iblank[p] == BLANKED;
@@ -217,26 +246,25 @@ __global__ void __launch_bounds__(TPB) k_adj_stage(AdjArgs<T> a) {
 
   // (3) the point of the thread
   if (gi >= ni || gj >= nj) return;
-  const int lj = ty + ST_H, li = tx + ST_H;
   T lam[4];
   if (inner) {
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      lam[v] = fd_row_t_inner<T>(&F[v][lj][li], 1);
-      lam[v] += fd_row_t_inner<T>(&F[4 + v][lj][li], RS);
+      lam[v] = fd_row_t_inner<T>(&FX[v][ty][tx + H], 1);
+      lam[v] += fd_row_t_inner<T>(&FE[v][ty + H][tx], ADJ_TX);
     }
   } else if (HOLES) {
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      lam[v] = fd_row_t_codes<T>(&F[v][lj][li], 1, gi, ni, a.code, p, 1);
-      lam[v] += fd_row_t_codes<T>(&F[4 + v][lj][li], RS, gj, nj, a.code + n, p, ni);
+      lam[v] = fd_row_t_codes<T>(&FX[v][ty][tx + H], 1, gi, ni, a.code, p, 1);
+      lam[v] += fd_row_t_codes<T>(&FE[v][ty + H][tx], ADJ_TX, gj, nj, a.code + n, p, ni);
     }
   } else {
-    const RowT5<T> rx = row_t5<T>(gi, ni), ry = row_t5<T>(gj, nj);  // ry uniform
+    const RowT5<T> rx = row_t5<T>(gi, ni), ry = row_t5<T>(gj, nj);
 #pragma unroll
     for (int v = 0; v < 4; v++) {
-      lam[v] = row_t5_sum<T>(rx, &F[v][lj][li], 1);
-      lam[v] += row_t5_sum<T>(ry, &F[4 + v][lj][li], RS);
+      lam[v] = row_t5_sum<T>(rx, &FX[v][ty][tx + H], 1);
+      lam[v] += row_t5_sum<T>(ry, &FE[v][ty + H][tx], ADJ_TX);
     }
   }
   // kappa at the point (recomputed from the same operands)
@@ -624,7 +652,7 @@ static hipError_t adj_stage_t(hipStream_t s, lee_handle *h, Block &b, const AdjS
   AdjArgs<T> a{};
   a.ni = b.ni;
   a.nj = b.nj;
-  a.ntx = (b.ni + ST_TX - 1) / ST_TX;
+  a.ntx = (b.ni + ADJ_TX - 1) / ADJ_TX;
   a.nty = (b.nj + ADJ_TY - 1) / ADJ_TY;
   a.ntiles = a.ntx * a.nty;
   a.chunk = (a.ntiles + 7) / 8;
@@ -669,7 +697,7 @@ static hipError_t adj_stage_t(hipStream_t s, lee_handle *h, Block &b, const AdjS
     const T *mc = sizeof(T) == 8 ? (const T *)b.mc64 : (const T *)b.mc32;
     a.rad = mc + (size_t)MC_R * b.n;
   }
-  const dim3 grid(a.chunk * 8), block(64, 4);
+  const dim3 grid(a.chunk * 8), block(ADJ_TX, ADJ_TY);
   const bool mf = !b.uniform_mean, ho = b.has_holes;
 #define LEE_ADJ(MF, K, HO)                                                                     \
   do {                                                                                         \
