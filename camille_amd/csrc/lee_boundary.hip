@@ -274,26 +274,38 @@ struct BndArgs {
   double gi;
 };
 
-// Sum of receiver r, variable v (ov_sum5; the stencil lies in its block).
-// SHARED: some donors are points that other workgroups have written.
-template <typename T, bool SHARED>
-__device__ __forceinline__ double ov_sum(const BndArgs<T> &a, int r, int v) {
-#pragma clang fp contract(off)
+// Sum of receiver r, variable v (ov_sum5; the stencil lies in its block): its
+// coefficients and the first donor's place, then the sum.  SHARED: some
+// donors are points that other workgroups have written.
+template <typename T>
+struct OvSum {
+  double c[25];
+  const T *y;
+  int ni;
+};
+template <typename T>
+__device__ __forceinline__ OvSum<T> ov_stencil(const BndArgs<T> &a, int r, int v) {
+  OvSum<T> s;
   const int b = a.db[r];
-  double cc[25];
 #pragma unroll
-  for (int q = 0; q < 25; q++) cc[q] = a.coef5[(size_t)q * a.nrecv + r];
-  const int d0 = a.dl[r], ni = of_block(a.t.ni, b);
-  const T *y = of_block(a.t.y, b) + (size_t)v * of_block(a.t.nn, b) + d0;
+  for (int q = 0; q < 25; q++) s.c[q] = a.coef5[(size_t)q * a.nrecv + r];
+  const int d0 = a.dl[r];
+  s.ni = of_block(a.t.ni, b);
+  s.y = of_block(a.t.y, b) + (size_t)v * of_block(a.t.nn, b) + d0;
+  return s;
+}
+template <typename T, bool SHARED>
+__device__ __forceinline__ double ov_sum(const OvSum<T> &o) {
+#pragma clang fp contract(off)
   T yv[25];
 #pragma unroll
   for (int q = 0; q < 25; q++) {
-    const T *p = &y[(q % 5) + (q / 5) * ni];
+    const T *p = &o.y[(q % 5) + (q / 5) * o.ni];
     yv[q] = SHARED ? get(p) : *p;
   }
   double s = 0.0;
 #pragma unroll
-  for (int q = 0; q < 25; q++) s = s + cc[q] * (double)yv[q];
+  for (int q = 0; q < 25; q++) s = s + o.c[q] * (double)yv[q];
   return s;
 }
 
@@ -309,7 +321,7 @@ __device__ __forceinline__ void ov_rho(const BndArgs<T> &a, int b, int p, double
 }
 
 // All latency: three launches (faces, gather, scatter) took 4.6 + 8.0 + 4.1 us
-// on a cylinder's 3858 receivers and 257 face points, for 2 MB; this one 10.9.  Here every
+// on a cylinder's 3858 receivers and 257 face points, for 2 MB; this one 10.7.  Here every
 // workgroup takes face points or sums, and a sum is written at once where
 // nobody reads its receiver.  The others' order: workgroups with face points,
 // held sums or readers of held receivers count themselves when their part is
@@ -338,7 +350,7 @@ __global__ void __launch_bounds__(OV_T) k_boundary(BndArgs<T> a) {
     const bool on = v < nv && r < a.nearly;
     const int b = on ? a.rb[r] : 0, p = on ? a.rl[r] : 0;
     if (on) {
-      const double s = ov_sum<T, false>(a, r, v);
+      const double s = ov_sum<T, false>(ov_stencil(a, r, v));
       if (r < a.nheld) put(&a.buf[(size_t)v * a.nrecv + r], s);
       else of_block(a.t.y, b)[(size_t)v * of_block(a.t.nn, b) + p] = (T)s;
       sums[tid] = s;
@@ -351,6 +363,18 @@ __global__ void __launch_bounds__(OV_T) k_boundary(BndArgs<T> a) {
   if (a.nheld == 0 && a.nearly == a.nrecv) return;
   const int counted = nbc + max((a.nuse + a.rpw - 1) / a.rpw, 1);
   if ((int)blockIdx.x >= counted) return;
+  // what the last part needs of the tables, requested before the count: each
+  // read after it is one more latency on the launch
+  const int nlate = (a.nrecv - a.nearly) * nv, nw = a.nheld + a.nrecv - a.nearly;
+  auto late = [&](int q) { return ov_stencil(a, a.nearly + q / nv, q % nv); };
+  auto written = [&](int q) { return q < a.nheld ? q : a.nearly + q - a.nheld; };
+  OvSum<T> first{};
+  if (tid < nlate) first = late(tid);
+  int wb = 0, wp = 0;
+  if (tid < nw) {
+    wb = a.rb[written(tid)];
+    wp = a.rl[written(tid)];
+  }
   // this wave's loads have returned and its stores are complete
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_s_waitcnt(0);
@@ -359,26 +383,28 @@ __global__ void __launch_bounds__(OV_T) k_boundary(BndArgs<T> a) {
     last = __hip_atomic_fetch_add(a.done, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == (unsigned)counted - 1;
   __syncthreads();
   if (!last) return;
-  for (int q = tid; q < (a.nrecv - a.nearly) * nv; q += OV_T) {
-    const int v = q % nv, r = a.nearly + q / nv;
-    put(&a.buf[(size_t)v * a.nrecv + r], ov_sum<T, true>(a, r, v));
+  for (int q = tid; q < nlate; q += OV_T) {
+    if (q != tid) first = late(q);
+    put(&a.buf[(size_t)(q % nv) * a.nrecv + a.nearly + q / nv], ov_sum<T, true>(first));
   }
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup");
   __builtin_amdgcn_s_waitcnt(0);
   __syncthreads();
-  const int nw = a.nheld + a.nrecv - a.nearly;
   for (int q = tid; q < nw; q += OV_T) {
-    const int r = q < a.nheld ? q : a.nearly + q - a.nheld;
-    const int b = a.rb[r], p = a.rl[r];
-    T *y = of_block(a.t.y, b);
-    const int n = of_block(a.t.nn, b);
+    const int r = written(q);
+    if (q != tid) {
+      wb = a.rb[r];
+      wp = a.rl[r];
+    }
+    T *y = of_block(a.t.y, wb);
+    const int n = of_block(a.t.nn, wb);
     double s[MAXV];
 #pragma unroll
     for (int v = 0; v < MAXV; v++) s[v] = v < nv ? get(&a.buf[(size_t)v * a.nrecv + r]) : 0.0;
 #pragma unroll
     for (int v = 0; v < MAXV; v++)
-      if (v < nv) y[(size_t)v * n + p] = (T)s[v];
-    if (a.with_rho) ov_rho(a, b, p, s[IP], s[IS]);
+      if (v < nv) y[(size_t)v * n + wp] = (T)s[v];
+    if (a.with_rho) ov_rho(a, wb, wp, s[IP], s[IS]);
   }
   if (tid == 0) __hip_atomic_store(a.done, 0u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
