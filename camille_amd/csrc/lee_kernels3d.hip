@@ -8,7 +8,7 @@
 // and are checked against the 2-D path on z-invariant problems and by axis
 // permutations.
 //
-// Stage kernel: a 64 x 4 tile of (i, j) columns marches through a short
+// Stage kernel: a 32 x 8 tile of (i, j) columns marches through a short
 // chunk of z planes (z_chunk).  Each plane's tile plus its 2-point (i, j) halo is staged in
 // LDS for the xi and eta derivatives; the zeta derivative comes from a
 // 5-plane register window of the thread's own column.  Filter: one pass of
@@ -26,12 +26,12 @@ namespace lee {
 
 namespace {
 
-constexpr int S3_TY = 4;      // tile rows in j
+constexpr int S3_TX = 32, S3_TY = 8;  // columns of a stage tile
 // Planes per workgroup of the stage.  A workgroup's planes are one serial
 // chain (loads, barrier, arithmetic, stores: about 5 us a plane), and the
 // four window planes that the next chunk reads again are in its XCD's L2,
 // so short chunks win at every size, FP32 / FP64 middle stage as measured
-// before the mean fields' and closure rows' changes below: 48 x 40 x 32
+// before the changes to mean fields, rows and tile below: 48 x 40 x 32
 // 176 / 229 us with 32 planes, 25 / 33 with 4, 15 / 19 with 2, 10 / 14 with
 // 1; 144 x 120 x 112 218 / 376, 131 / 258, 128 / 247, 131 / 259;
 // 256 x 200 x 256 857 / 1599, 723 / 1338, 717 / 1329, 728 / 1386.
@@ -129,17 +129,23 @@ struct Stage3Args {
   T h, b, a;
 };
 
-// One RK stage on a 64 x 4 column tile through a chunk of zc planes.
+// One RK stage on a 32 x 8 column tile through a chunk of zc planes.
 // What bounds it: HBM at large blocks (256 x 200 x 256 FP32, a parallel jet:
 // 208 of the 268 bytes a point left once constant mean fields are read from
 // cache, 583 us, 4.7 TB/s of the 4.9 a large copy reaches; 717 us before).
 // Closure rows without branches (Row4) and zone boxes read once: middle stage
 // at 144 x 120 x 112 FP32 128 -> 104 us, FP64 247 -> 230.
+// Tiles of 32 x 8 read 160 halo points beside 256, one load a lane, where 64
+// x 4 read 288 in three loads, and leave the registers that the FP64 operands
+// need: first / middle / last stage of 144 x 120 x 112 FP32 98 / 104 / 96 ->
+// 86 / 95 / 83 us, FP64 174 / 230 / 171 -> 141 / 193 / 144; 256 x 200 x 256
+// FP64 897 / 1187 / 876 -> 826 / 1129 / 824, FP32 503 / 581 / 502 -> 492 / 578
+// / 486.
 // (FP64 is held to two waves per SIMD: left alone, the middle stage takes so
 // many registers that one fits.)
 template <typename T, bool MEANF, int KIND>
 __global__ void __launch_bounds__(TPB, sizeof(T) == 8 ? 2 : 3) k_stage3d(Stage3Args<T> a) {
-  constexpr int RS = ST_TX + 2 * ST_H, NR = S3_TY + 2 * ST_H;
+  constexpr int RS = S3_TX + 2 * ST_H, NR = S3_TY + 2 * ST_H;
   __shared__ T s[5][NR][RS];
   // within each z chunk, XCD x (workgroups x mod 8 of a grid row that is a
   // multiple of 8 wide) takes the x-th band of tiles, so that the halo a
@@ -147,8 +153,8 @@ __global__ void __launch_bounds__(TPB, sizeof(T) == 8 ? 2 : 3) k_stage3d(Stage3A
   const int ntl = a.ntx * a.nty;
   const int tile = xcd_tile(blockIdx.x, (ntl + 7) / 8);
   if (tile >= ntl) return;
-  const int tx = threadIdx.x, ty = __builtin_amdgcn_readfirstlane((int)threadIdx.y);  // a wave is one row
-  const int i0 = (tile % a.ntx) * ST_TX, j0 = (tile / a.ntx) * S3_TY;
+  const int tx = threadIdx.x, ty = threadIdx.y, tid = ty * S3_TX + tx;
+  const int i0 = (tile % a.ntx) * S3_TX, j0 = (tile / a.ntx) * S3_TY;
   const int k0 = blockIdx.y * a.zc, k1 = min(k0 + a.zc, a.nk);
   const int ni = a.ni, nj = a.nj, nk = a.nk;
   const size_t plane = (size_t)ni * nj, n = plane * nk;
@@ -156,7 +162,7 @@ __global__ void __launch_bounds__(TPB, sizeof(T) == 8 ? 2 : 3) k_stage3d(Stage3A
   const bool own = gi < ni && gj < nj;
   const size_t col = own ? (size_t)gj * ni + gi : 0;
   const Row4<T> rx = row4<T>(default_code(gi, ni, 2)), ry = row4<T>(default_code(gj, nj, 2));
-  const unsigned zmask = zones_meeting3(a.z, a.nz, i0, i0 + ST_TX - 1, j0, j0 + S3_TY - 1, k0, k1 - 1);
+  const unsigned zmask = zones_meeting3(a.z, a.nz, i0, i0 + S3_TX - 1, j0, j0 + S3_TY - 1, k0, k1 - 1);
   // register window of the own column: planes k - 2 .. k + 2
   T w[5][5];
 #pragma unroll
@@ -166,6 +172,14 @@ __global__ void __launch_bounds__(TPB, sizeof(T) == 8 ? 2 : 3) k_stage3d(Stage3A
 #pragma unroll
     for (int v = 0; v < 5; v++) w[v][q] = ok ? a.yin[v * n + (size_t)kk * plane + col] : (T)0;
   }
+  // the halo that the rows read: two rows beside the tile on either side
+  // (lanes 0 to 127) and two columns (128 to 159)
+  static_assert(S3_TX == 32 && S3_TY == 8 && TPB == 256, "halo lanes");
+  const int hq = tid < 128 ? tid >> 5 : tid & 3;
+  const int hr = tid < 128 ? (hq < 2 ? hq : hq + S3_TY) : ((tid >> 2) & 7) + ST_H;  // region row
+  const int hc = tid < 128 ? tx + ST_H : (hq < 2 ? hq : hq + S3_TX);                // and column
+  const bool hok = tid < 160 && j0 - ST_H + hr >= 0 && j0 - ST_H + hr < nj && i0 - ST_H + hc >= 0 && i0 - ST_H + hc < ni;
+  const size_t hp = hok ? (size_t)(j0 - ST_H + hr) * ni + (i0 - ST_H + hc) : 0;
   for (int k = k0; k < k1; k++) {
     // every global operand of plane k is requested before the barrier, so
     // one memory latency per plane is exposed instead of three
@@ -175,30 +189,11 @@ __global__ void __launch_bounds__(TPB, sizeof(T) == 8 ? 2 : 3) k_stage3d(Stage3A
 #pragma unroll
       for (int v = 0; v < 5; v++) w[v][4] = ok ? a.yin[v * n + (size_t)kk * plane + col] : (T)0;
     }
-    // plane k with its (i, j) halo.  The centre (region rows 2..5, columns
-    // 2..65) is the window's plane k, already in registers; only the ring
-    // is loaded: region row hr (rows 0, 1 for ty 0, 1; rows 6, 7 for ty 2,
-    // 3) at columns tx and 64 + tx, and for tx < 4 the side column sc (0,
-    // 1, 66, 67) of region row 2 + ty
-    const int hr = ty < 2 ? ty : ty + 4, sc = tx < 2 ? tx : ST_TX + tx;
-    T th[2][5], ts[5];
-    {
-      const int rj = j0 - ST_H + hr;
+    // plane k with its (i, j) halo.  The centre is the window's plane k,
+    // already in registers; only the halo is loaded, a point a lane
+    T th[5];
 #pragma unroll
-      for (int half = 0; half < 2; half++) {
-        const int c = half == 0 ? tx : ST_TX + tx;
-        const int ri = i0 - ST_H + c;
-        const bool ok = (half == 0 || tx < 2 * ST_H) && rj >= 0 && rj < nj && ri >= 0 && ri < ni;
-        const size_t q = (size_t)k * plane + (size_t)(ok ? rj : 0) * ni + (ok ? ri : 0);
-#pragma unroll
-        for (int v = 0; v < 5; v++) th[half][v] = ok ? a.yin[v * n + q] : (T)0;
-      }
-      const int sj = j0 + ty, si = i0 - ST_H + sc;
-      const bool ok = tx < 2 * ST_H && sj < nj && si >= 0 && si < ni;
-      const size_t q = (size_t)k * plane + (size_t)(ok ? sj : 0) * ni + (ok ? si : 0);
-#pragma unroll
-      for (int v = 0; v < 5; v++) ts[v] = ok ? a.yin[v * n + q] : (T)0;
-    }
+    for (int v = 0; v < 5; v++) th[v] = hok ? a.yin[v * n + (size_t)k * plane + hp] : (T)0;
     // per-point operands (a clamped column for threads outside the block)
     const size_t p = (size_t)k * plane + col;
     double m[3][3];
@@ -215,19 +210,24 @@ __global__ void __launch_bounds__(TPB, sizeof(T) == 8 ? 2 : 3) k_stage3d(Stage3A
     }
     const T rho_first = (MEANF && KIND == STAGE_FIRST) ? a.rho_in[p] : (T)0;
     T accp[5], ynp[5];
+    auto own_loads = [&]() {
 #pragma unroll
-    for (int v = 0; v < 5; v++) {
-      accp[v] = KIND != STAGE_FIRST ? a.acc[v * n + p] : (T)0;
-      ynp[v] = KIND == STAGE_MID ? a.yn[v * n + p] : (T)0;
-    }
-#pragma unroll
-    for (int v = 0; v < 5; v++) {
-      s[v][hr][tx] = th[0][v];
-      s[v][ty + ST_H][tx + ST_H] = w[v][2];
-      if (tx < 2 * ST_H) {
-        s[v][hr][ST_TX + tx] = th[1][v];
-        s[v][ty + ST_H][sc] = ts[v];
+      for (int v = 0; v < 5; v++) {
+        accp[v] = KIND != STAGE_FIRST ? a.acc[v * n + p] : (T)0;
+        ynp[v] = KIND == STAGE_MID ? a.yn[v * n + p] : (T)0;
       }
+    };
+    if constexpr (sizeof(T) == 4) own_loads();
+#pragma unroll
+    for (int v = 0; v < 5; v++) {
+      s[v][ty + ST_H][tx + ST_H] = w[v][2];
+      if (tid < 160) s[v][hr][hc] = th[v];
+    }
+    // in 64 bits only once the halo's registers are free: in flight together
+    // they spilled 92 bytes a lane (middle stage 214 instead of 193 us)
+    if constexpr (sizeof(T) == 8) {
+      __builtin_amdgcn_sched_barrier(0);
+      own_loads();
     }
     __syncthreads();
     if (own) {
@@ -649,7 +649,7 @@ static hipError_t stage3d_t(hipStream_t s, lee_handle *h, Block &b, int stage, c
   a.ni = b.ni;
   a.nj = b.nj;
   a.nk = b.nk;
-  a.ntx = (b.ni + ST_TX - 1) / ST_TX;
+  a.ntx = (b.ni + S3_TX - 1) / S3_TX;
   a.nty = (b.nj + S3_TY - 1) / S3_TY;
   a.zc = z_chunk((a.ntx * a.nty + 7) / 8 * 8, b.nk, STAGE_Z_CHUNK, b.cus);
   a.nzc = (b.nk + a.zc - 1) / a.zc;
@@ -703,7 +703,7 @@ static hipError_t stage3d_t(hipStream_t s, lee_handle *h, Block &b, int stage, c
   a.h = (T)sc.h;
   a.b = (T)sc.b;
   a.a = (T)sc.a;
-  const dim3 grid((a.ntx * a.nty + 7) / 8 * 8, a.nzc), block(ST_TX, S3_TY);
+  const dim3 grid((a.ntx * a.nty + 7) / 8 * 8, a.nzc), block(S3_TX, S3_TY);
   const bool mf = !b.uniform_mean;
 #define LEE_S3(MF)                                                                                    \
   do {                                                                                                \
