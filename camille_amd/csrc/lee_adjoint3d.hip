@@ -28,26 +28,14 @@ namespace {
 
 constexpr int A3_TX = 32, A3_TY = 8;  // points of a stage tile
 constexpr int A3_ZC = 16;      // most planes per chunk of the zeta^T filter pass (at least 4, z_chunk)
-// Planes per workgroup of the adjoint stage when `slots` workgroups are
-// resident: the fewest rounds of workgroups times planes each marches, with
-// two more for the start of its column; up to 10, past which little is
-// shared.  Whole reverse step with 4 planes whatever the block and with this
-// rule, FP32 / FP64: 112 x 96 x 80 640 / 960 -> 516 / 906 us (5 and 8
-// planes), 144 x 120 x 112 1389 / 2515 -> 1332 / 2376 (6 and 6), 256 x 200 x
-// 256 7770 / 13339 -> 7402 / 12877; 48 x 40 x 32 208 / 275 -> 147 / 185 (1).
-inline int adj_z_chunk(int tiles, int nk, int slots) {
-  int best = 1;
-  long long cost = -1;
-  for (int zc = 1; zc <= 10 && zc <= nk; zc++) {
-    const long long groups = (long long)tiles * ((nk + zc - 1) / zc);
-    const long long c = (groups + slots - 1) / slots * (zc + 2);
-    if (cost < 0 || c < cost) {
-      cost = c;
-      best = zc;
-    }
-  }
-  return best;
-}
+// Planes per workgroup of the adjoint stage (z_chunk_rounds): the start of a
+// column costs about two planes; up to 10, past which little is shared.
+// Whole reverse step with 4 planes whatever the block and with this rule,
+// FP32 / FP64: 112 x 96 x 80 640 / 960 -> 516 / 906 us (5 and 8 planes),
+// 144 x 120 x 112 1389 / 2515 -> 1332 / 2376 (6 and 6), 256 x 200 x 256 7770 /
+// 13339 -> 7402 / 12877; 48 x 40 x 32 208 / 275 -> 147 / 185 (1).
+constexpr int ADJ_Z_CHUNK = 10;
+constexpr double ADJ_Z_START = 2.0;
 
 inline unsigned nba(size_t n) { return (unsigned)((n + TPB - 1) / TPB); }
 
@@ -480,7 +468,8 @@ static hipError_t adj_stage3d_t(hipStream_t s, lee_handle *h, Block &b, const Ad
   a.nk = b.nk;
   a.ntx = (b.ni + A3_TX - 1) / A3_TX;
   a.nty = (b.nj + A3_TY - 1) / A3_TY;
-  a.zc = adj_z_chunk((a.ntx * a.nty + 7) / 8 * 8, b.nk, b.cus * (sizeof(T) == 8 ? 2 : b.uniform_mean ? 4 : 3));
+  a.zc = z_chunk_rounds((a.ntx * a.nty + 7) / 8 * 8, b.nk, b.cus * (sizeof(T) == 8 ? 2 : b.uniform_mean ? 4 : 3),
+                        ADJ_Z_START, ADJ_Z_CHUNK);
   a.nzc = (b.nk + a.zc - 1) / a.zc;
   T *const *L = sizeof(T) == 8 ? (T *const *)b.A64 : (T *const *)b.A32;
   auto buf = [&](int k) -> T * { return k < 0 ? nullptr : L[k]; };

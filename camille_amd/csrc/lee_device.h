@@ -297,6 +297,23 @@ inline int z_chunk(int tiles, int nk, int most, int cus) {
   return 1;
 }
 
+// The same for kernels of which `slots` workgroups are resident and whose
+// time goes with their rounds: the fewest rounds times planes, of which the
+// start of a column costs `start`.
+inline int z_chunk_rounds(int tiles, int nk, int slots, double start, int most) {
+  int best = 1;
+  double cost = -1.0;
+  for (int zc = 1; zc <= most && zc <= nk; zc++) {
+    const long long groups = (long long)tiles * ((nk + zc - 1) / zc);
+    const double c = (double)((groups + slots - 1) / slots) * (zc + start);
+    if (cost < 0.0 || c < cost) {
+      cost = c;
+      best = zc;
+    }
+  }
+  return best;
+}
+
 // Bit z set where zone z meets the box (uniform over the workgroup): the boxes
 // are read at fixed places, all at once, and the planes visit only zones that
 // can reach them.

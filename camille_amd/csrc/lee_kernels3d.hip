@@ -36,6 +36,13 @@ constexpr int S3_TX = 32, S3_TY = 8;  // columns of a stage tile
 // 1; 144 x 120 x 112 218 / 376, 131 / 258, 128 / 247, 131 / 259;
 // 256 x 200 x 256 857 / 1599, 723 / 1338, 717 / 1329, 728 / 1386.
 constexpr int STAGE_Z_CHUNK = 2;
+// In 64 bits, two workgroups a CU, the rounds of workgroups decide and the
+// window planes weigh more: middle stage with 2 planes and by z_chunk_rounds,
+// 112 x 96 x 80 81 -> 79 us (4 planes), 144 x 120 x 112 191 -> 183 (6),
+// 256 x 200 x 256 1128 -> 1051 (6).  (In 32 bits 3 to 6 planes change it by
+// -2 to 16 %.)
+constexpr int STAGE64_Z_CHUNK = 6;
+constexpr double STAGE64_Z_START = 0.3;
 // Most planes per chunk of the single-pass filter (4 halo planes a side) and
 // of the two-pass form's column pass; smaller blocks take fewer, at least 16
 // and 4 (z_chunk).  With 64 and 32 whatever the block, the filter of a
@@ -651,7 +658,9 @@ static hipError_t stage3d_t(hipStream_t s, lee_handle *h, Block &b, int stage, c
   a.nk = b.nk;
   a.ntx = (b.ni + S3_TX - 1) / S3_TX;
   a.nty = (b.nj + S3_TY - 1) / S3_TY;
-  a.zc = z_chunk((a.ntx * a.nty + 7) / 8 * 8, b.nk, STAGE_Z_CHUNK, b.cus);
+  const int tiles = (a.ntx * a.nty + 7) / 8 * 8;
+  a.zc = sizeof(T) == 8 ? z_chunk_rounds(tiles, b.nk, 2 * b.cus, STAGE64_Z_START, STAGE64_Z_CHUNK)
+                        : z_chunk(tiles, b.nk, STAGE_Z_CHUNK, b.cus);
   a.nzc = (b.nk + a.zc - 1) / a.zc;
   const int in_idx = stage == 0 ? 0 : (stage % 2 == 1 ? 2 : 3);
   const int out_idx = stage % 2 == 0 ? 2 : 3;

@@ -35,8 +35,8 @@ def _box3(ni, nj, nk, seed, flow="general"):
     return x, y, z, mean, rng.standard_normal((5, nk, nj, ni)), rng.standard_normal((5, nk, nj, ni))
 
 
-# (131, 61, 45) takes chunks of 2 planes forwards and 4 backwards, one plane
-# left over; (70, 13, 9) and (9, 9, 14) take single planes
+# (131, 61, 45) takes chunks of 2 or 4 planes forwards and 3 or 4 backwards,
+# with one plane left over; (70, 13, 9) and (9, 9, 14) take single planes
 @pytest.mark.parametrize("dims", [(131, 61, 45), (70, 13, 9), (9, 9, 14)])
 @pytest.mark.parametrize("flow", ["general", "jet", "rotor"])
 @pytest.mark.parametrize("prec,tol", [(FP64, 1e-12), (FP32, 2e-5)])
