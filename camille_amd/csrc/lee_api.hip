@@ -1567,8 +1567,12 @@ namespace {
 // still at work: a freshly allocated array is mapped page by page at its first
 // write, which made the copy into it run at 10 GB/s instead of 33 (144 x 120 x
 // 112 FP64 8.0 -> 2.6 ms).  Leaves the contents as they are, and ends when the
-// stream does.
+// stream does.  Memory that HIP knows (pinned, or not the host's) is left alone.
 void map_pages(hipStream_t s, void *dst, size_t bytes) {
+  hipPointerAttribute_t at{};
+  const hipError_t known = hipPointerGetAttributes(&at, dst);
+  if (known == hipSuccess && at.type != hipMemoryTypeUnregistered) return;
+  if (known != hipSuccess) (void)hipGetLastError();
   constexpr size_t PAGE = 4096, BATCH = 64 * PAGE;
   volatile char *p = (volatile char *)dst;
   for (size_t o = 0; o < bytes; o += BATCH) {
