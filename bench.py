@@ -133,7 +133,9 @@ def c5_leg(steps, warmup, single_steps):
                           persistent_graph_form=configured)
         if kt:
             res[label]["kernel_ms"] = {k: [round(t, 4), c] for k, (t, c) in kt.items()}
-            per_point = {"stage_first": 92, "stage_mid": 124, "stage_last": 92, "filter": 32}
+            # two RK stages a launch (no launch of the middle class): the second pair also reads y_n
+            per_point = {"stage_first": 92, "stage_mid": 124, "stage_last": 92 if kt["stage_mid"][1] else 108,
+                         "filter": 32}
             res[label]["kernel_hbm_frac"] = {
                 c: per_point[c] * npts / (kt[c][0] / kt[c][1] * 1e-3) / HBM_PEAK for c in per_point if kt[c][1]}
         b.close()
@@ -580,16 +582,17 @@ def main():
     avg_ms = kt[dom][0] / kt[dom][1]
     b = 4  # FP32 bulk
     V, D = 4, 2
+    paired = kt["stage_mid"][1] == 0  # two RK stages a launch: the first pair, then the second
     per_point = {  # algorithmic bytes per point per launch: state arrays, FP64 metrics + J, sigma
         "stage_first": 3 * V * b + 8 * (D * D + 1) + b,      # read y_n; write acc, next input
         "stage_mid": 5 * V * b + 8 * (D * D + 1) + b,        # read in, y_n, acc; write acc, next input
-        "stage_last": 3 * V * b + 8 * (D * D + 1) + b,       # read in, acc; write acc
+        "stage_last": (4 if paired else 3) * V * b + 8 * (D * D + 1) + b,  # read in, acc (pair: y_n too); write acc
         "filter": 2 * V * b,                                 # read y_{n+1}; write filtered
     }[dom]
     achieved = per_point * npts / (avg_ms * 1e-3)
     traffic = None
     tpath = os.path.join(ROOT, "profiles", "traffic_c2_fp32.json")
-    if os.path.exists(tpath):
+    if os.path.exists(tpath) and not paired:  # measured on one-stage launches
         try:
             traffic = json.load(open(tpath)).get(dom)
         except Exception:
@@ -618,7 +621,8 @@ def main():
 
     # algorithmic bytes per update of the whole step, FP32 bulk, uniform mean:
     # 5 V b state + 8 (D^2 + 1) metrics + b sigma + V b / 2 filter
-    algo_step_bytes = 5 * 4 * 4 + 8 * 5 + 4 + 8
+    # (two stages a launch: 3 V b + 4 V b state, metrics and sigma twice, 2 V b filter, over 4 stages)
+    algo_step_bytes = 7 * 4 + 2 * (8 * 5 + 4) / 4 + 8 if paired else 5 * 4 * 4 + 8 * 5 + 4 + 8
     v = res["fp32"]["ups"]
     out = {
         "metric": "grid-point RK-stage updates/s + % HBM peak; FP32 vs FP64 at <=1e-5 rel p-error",
@@ -651,7 +655,7 @@ def main():
         "tile_shape": {"stage_rows_per_thread": res["fp32"]["tiles"][0], "filter_tile_rows": res["fp32"]["tiles"][1]},
         "roofline": {"bound": "hbm", "kernel": dom, "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK, "traffic": traffic,
-                     "traffic_source": "profiles/traffic_c2_fp32.json: rocprofv3 FETCH_SIZE and WRITE_SIZE of "
+                     "traffic_source": "profiles/traffic_c2_fp32.json (launches of one RK stage): rocprofv3 FETCH_SIZE and WRITE_SIZE of "
                                        "this kernel in KiB per dispatch, scaled by a 256 MiB device copy "
                                        "(profiles/traffic_c2_fp32.md); not measured in this run",
                      "algorithmic_bytes_per_point": per_point, "avg_launch_ms": avg_ms,

@@ -228,16 +228,18 @@ int lee_last_solve_ms(lee_handle *h, float *ms);
  * counterpart): while enabled, HIP events bracket every launch on the
  * handle's stream.  lee_get_kernel_timing sums the recorded durations since
  * the last call into ms[5] / count[5] by class: 0 first RK stage, 1 middle
- * stages, 2 last stage, 3 filter, 4 boundary conditions + overset. */
+ * stages, 2 last stage, 3 filter, 4 boundary conditions + overset.  Where two
+ * stages share a launch, 0 is the first pair and 2 the second. */
 int lee_set_kernel_timing(lee_handle *h, int on);
 int lee_get_kernel_timing(lee_handle *h, double *ms, int *count);
 
 /* Tile shapes of the fused kernels (no reference counterpart).  The first
  * lee_solve of a handle times every stage tile height (4 * stage_rows, with
  * stage_rows 1, 2 or 4) and filter tile height (4, 8, 12 or 16) on each block
- * and keeps the fastest, cached per (ni, nj, precision, mean kind, holes).
- * lee_autotune re-runs the search; lee_set_tile_shape pins a shape (every
- * shape gives bit-identical results). */
+ * and keeps the fastest, cached per (ni, nj, precision, mean kind, holes); it
+ * also times two stages a launch where the block allows it.  lee_autotune
+ * re-runs the search; lee_set_tile_shape pins a shape of the launches of one
+ * stage and selects them (every shape and form gives bit-identical results). */
 int lee_autotune(lee_handle *h);
 int lee_set_tile_shape(lee_handle *h, int iblock, int stage_rows, int filter_rows);
 int lee_get_tile_shape(lee_handle *h, int iblock, int *stage_rows, int *filter_rows);
@@ -264,8 +266,8 @@ int lee_get_filter_march(lee_handle *h, int iblock, int *waves, int *rows);
 
 /* Batched ensemble (no reference counterpart: the reference runs one
  * problem per process).  nsolve independent single-block problems, block k
- * with its own lee_config cfgs[k], advanced together: per RK stage one
- * persistent launch covers the tiles of every solve, and one step is
+ * with its own lee_config cfgs[k], advanced together: one launch per RK stage
+ * or pair of stages covers the tiles of every solve, and one step is
  * captured once in a HIP graph and replayed.  The scheme settings (num_dim,
  * gamma, orders, blend, stages, sponge law, precision, path) must agree;
  * source, CFL or dt, grid, sponges and mean flow may differ (the means must
@@ -278,7 +280,8 @@ int lee_get_solve_time(const lee_handle *h, int isolve, int *time_step, double *
 /* Launch settings of a batch: graph replay on/off, persistent grid sizes of
  * the stage and filter launches (0 = one workgroup per tile;
  * LEE_GRID_RESIDENT = as many workgroups as the device holds at once for
- * that kernel, its occupancy per CU times the CUs).  Chosen by the
+ * that kernel, its occupancy per CU times the CUs).  A stage grid other than
+ * 0 launches one stage at a time.  Chosen by the
  * autotuner at the first lee_solve unless set here; every setting gives
  * bit-identical results. */
 #define LEE_GRID_RESIDENT (-1)
