@@ -939,14 +939,17 @@ static hipError_t batch_prepare_t(hipStream_t s, lee_handle *h) {
   // the host vectors die here: wait for the copies
   if ((e = hipStreamSynchronize(s)) != hipSuccess) return e;
   batch_resident_t<T>(h);
-  p.ready = true;
   return hipSuccess;
 }
 
 hipError_t batch_prepare(hipStream_t s, lee_handle *h) {
   batch_release(h);
-  const hipError_t e = h->cfg.precision == LEE_FP32 ? batch_prepare_t<float>(s, h) : batch_prepare_t<double>(s, h);
-  return e == hipSuccess && h->bp.pair ? batch_pair_prepare(s, h) : e;
+  hipError_t e = h->cfg.precision == LEE_FP32 ? batch_prepare_t<float>(s, h) : batch_prepare_t<double>(s, h);
+  if (e == hipSuccess && h->bp.pair) e = batch_pair_prepare(s, h);
+  // ready once every table that a launch reads is there: all of them or none
+  if (e == hipSuccess) h->bp.ready = true;
+  else batch_release(h);
+  return e;
 }
 
 // Grid of a batch launch over `total` list entries: one workgroup per entry

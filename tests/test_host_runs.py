@@ -1,0 +1,93 @@
+"""Host code of the library on a HIP runtime without a device
+(tests/hip_host.cpp): what it launches, and what it leaves behind when an
+allocation fails.  Every run is a process of its own, in which that runtime
+is loaded before the library."""
+import os
+import subprocess
+import sys
+import textwrap
+
+import pytest
+
+HERE = os.path.dirname(os.path.abspath(__file__))
+
+PRELUDE = """
+import ctypes, sys
+host = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
+host.host_launch_name.restype = ctypes.c_char_p
+host.host_launch_ptr.restype = ctypes.c_void_p
+host.host_mallocs.restype = host.host_live.restype = host.host_launches.restype = ctypes.c_long
+host.host_fail_malloc.argtypes = [ctypes.c_long]
+host.host_launch_name.argtypes = [ctypes.c_long]
+host.host_launch_ptr.argtypes = [ctypes.c_long, ctypes.c_int]
+sys.path.insert(0, sys.argv[2])
+import numpy as np
+from camille_amd import *
+
+def launches():
+    return [host.host_launch_name(k).decode() for k in range(host.host_launches())]
+
+def tables():  # the operand table and tile list of every batch launch
+    return [(host.host_launch_ptr(k, 0), host.host_launch_ptr(k, 1)) for k, n in enumerate(launches()) if "k_batch_" in n]
+
+def block(ni, nj):
+    x, y = np.meshgrid(0.5 * np.arange(ni), 0.5 * np.arange(nj))
+    mean = np.zeros((5, nj, ni))
+    mean[4] = 1 / 1.4
+    return dict(x=x, y=y, mean=mean)
+"""
+
+
+@pytest.fixture(scope="module")
+def runtime(tmp_path_factory):
+    so = str(tmp_path_factory.mktemp("hip_host") / "libhip_host.so")
+    subprocess.run(["g++", "-O1", "-shared", "-fPIC", "-w", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    os.path.join(HERE, "hip_host.cpp"), "-o", so], check=True)
+
+    def run(code):
+        p = subprocess.run([sys.executable, "-c", PRELUDE + textwrap.dedent(code), so, os.path.dirname(HERE)],
+                           capture_output=True, text=True, timeout=300)
+        assert p.returncode == 0, p.stdout[-2000:] + p.stderr[-2000:]
+        return p.stdout
+    return run
+
+
+BATCH = """
+def batch():
+    b = Batch([dict(block(70, 40), mode="FIX_DT", value=0.01) for _ in range(2)], precision=FP32)
+    for k in range(2):
+        b.set_solution(np.zeros((5, 40, 70)), k)
+    host.host_forget()
+    return b
+
+def solved(b, fail=0):
+    host.host_fail_malloc(fail)
+    try:
+        b.solve(3)
+        return True
+    except LeeError:
+        return False
+    finally:
+        host.host_fail_malloc(0)
+
+b = batch()
+host.host_fail_malloc(0)
+b.solve(3)
+total = host.host_mallocs()
+assert total > 10 and any("k_batch_pair" in n for n in launches())
+b.close()
+"""
+
+
+def test_batch_after_a_failed_allocation(runtime):
+    """Whichever allocation of a batch's first solve fails, the solve says so
+    and the next one runs on whole tables."""
+    runtime(BATCH + """
+for k in range(1, total + 1):
+    b = batch()
+    assert not solved(b, fail=k), k
+    host.host_forget()
+    assert solved(b), k
+    assert launches() and all(p and q for p, q in tables()), k
+    b.close()
+""")
