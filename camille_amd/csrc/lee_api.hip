@@ -418,10 +418,11 @@ int batch_capture(lee_handle *h) {
 }
 
 // Tile shape and persistent grid of the batched kernels, timed with HIP
-// events on scratch tables (the state in Y0 is untouched).
-int batch_autotune(lee_handle *h) {
+// events on scratch tables (the state in Y0 is untouched).  batch_autotune
+// makes the events and, however the timing ends, takes the scratch tables
+// back and leaves settings that a solve can run with.
+int batch_tune(lee_handle *h, hipEvent_t &e0, hipEvent_t &e1) {
   BatchPlan &p = h->bp;
-  if (p.tuned) return LEE_OK;
   int rc = batch_reserve(h, 1);
   if (rc) return rc;
   std::vector<BatchSched> zero(h->nblk * h->cfg.rk_stages, BatchSched{0.0, 0.0, 0.0});
@@ -433,7 +434,6 @@ int batch_autotune(lee_handle *h) {
     if (hipDeviceGetAttribute(&v, hipDeviceAttributeMultiprocessorCount, h->device) == hipSuccess && v > 0) dev_cu = v;
   }
   const int grids[5] = {0, LEE_GRID_RESIDENT, 4 * dev_cu, 8 * dev_cu, 16 * dev_cu};
-  hipEvent_t e0, e1;
   HIPCHK(hipEventCreate(&e0));
   HIPCHK(hipEventCreate(&e1));
   const int reps = 5;
@@ -539,11 +539,6 @@ int batch_autotune(lee_handle *h) {
       }
     }
   }
-  p.stack = 0;
-  p.tuning = false;
-  (void)hipEventDestroy(e0);
-  (void)hipEventDestroy(e1);
-  batch_release(h);
   if (rc) return rc;
   p.R = bR;
   p.pair = bP;
@@ -553,6 +548,27 @@ int batch_autotune(lee_handle *h) {
   p.grid_filter = bF;
   p.tuned = true;
   return LEE_OK;
+}
+
+int batch_autotune(lee_handle *h) {
+  BatchPlan &p = h->bp;
+  if (p.tuned) return LEE_OK;
+  const int R = p.R, TY = p.TY, stack = p.stack, pair = p.pair, gs = p.grid_stage, gf = p.grid_filter;
+  hipEvent_t e0 = nullptr, e1 = nullptr;
+  const int rc = batch_tune(h, e0, e1);
+  for (hipEvent_t e : {e0, e1})
+    if (e) (void)hipEventDestroy(e);
+  p.tuning = false;
+  batch_release(h);
+  if (rc) {
+    p.R = R;
+    p.TY = TY;
+    p.stack = stack;
+    p.pair = pair;
+    p.grid_stage = gs;
+    p.grid_filter = gf;
+  }
+  return rc;
 }
 
 // lee_solve for a batch: per chunk of steps, the host schedule goes to the

@@ -91,3 +91,25 @@ for k in range(1, total + 1):
     assert launches() and all(p and q for p, q in tables()), k
     b.close()
 """)
+
+
+def test_batch_whose_tuner_failed(runtime):
+    """A tuner that stops at a failed allocation leaves neither events nor the
+    tables it times on: a pinned shape then runs on the state.  Stage 1 reads
+    Y2 and Y0; on the scratch tables it would read Y2 twice (the pointers
+    after the six integers of StageArgs)."""
+    runtime(BATCH + """
+clean = host.host_live()
+for k in range(1, total + 1):
+    b = batch()
+    assert not solved(b, fail=k), k
+    b.set_tile_shape(1, 4)
+    host.host_forget()
+    assert solved(b), k
+    mid = [p for (p, _), n in zip(tables(), launches()) if "k_batch_stageIfLb0ELi1ELi1E" in n]
+    assert mid and len(tables()) == len(launches()), k
+    yin, yn = (ctypes.c_void_p * 2).from_address(mid[0] + 24)
+    assert yin != yn, k
+    b.close()
+    assert host.host_live() == clean, (k, host.host_live())
+""")
