@@ -393,6 +393,7 @@ int batch_reserve(lee_handle *h, size_t nsteps) {
   if (p.exec) HIPCHK(hipGraphExecDestroy(p.exec));
   p.exec = nullptr;
   dfree(p.sched);
+  p.sched_steps = 0;
   HIPCHK(dalloc(&p.sched, nsteps * h->nblk * h->cfg.rk_stages));
   p.sched_steps = nsteps;
   return LEE_OK;

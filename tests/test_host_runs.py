@@ -113,3 +113,21 @@ for k in range(1, total + 1):
     b.close()
     assert host.host_live() == clean, (k, host.host_live())
 """)
+
+
+def test_batch_after_a_failed_schedule(runtime):
+    """A schedule that could not grow is not taken for the shorter one before."""
+    runtime(BATCH + """
+b = batch()
+assert solved(b)
+host.host_fail_malloc(1)
+try:
+    b.solve(50)
+    assert False
+except LeeError:
+    pass
+host.host_fail_malloc(0)
+b.solve(2)
+b.solve(60)
+b.close()
+""")
