@@ -28,6 +28,7 @@ std::string g_create_err;
     hipError_t _e = (expr);                                                            \
     if (_e != hipSuccess) {                                                            \
       h->err = std::string("HIP error ") + hipGetErrorString(_e) + " at " #expr;       \
+      (void)hipGetLastError(); /* reported here, not by the next call's launches */    \
       return LEE_EHIP;                                                                 \
     }                                                                                  \
   } while (0)

@@ -21,7 +21,7 @@ std::vector<Launch> g_launches;
 std::map<void *, size_t> g_live;
 long g_mallocs = 0, g_fail_at = 0;
 float g_elapsed = 1e6f;
-bool g_capturing = false;
+hipError_t g_last = hipSuccess;
 char g_symbol[1 << 20];
 
 hipError_t take(void **p, size_t bytes) {
@@ -84,7 +84,7 @@ hipError_t hipLaunchKernel(const void *f, dim3, dim3, void **args, size_t, hipSt
 hipError_t hipMalloc(void **p, size_t bytes) {
   if (++g_mallocs == g_fail_at) {
     *p = nullptr;
-    return hipErrorOutOfMemory;
+    return g_last = hipErrorOutOfMemory;
   }
   return take(p, bytes);
 }
@@ -126,7 +126,11 @@ hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *) {
   return hipSuccess;
 }
 const char *hipGetErrorString(hipError_t e) { return e == hipErrorOutOfMemory ? "out of memory" : "error"; }
-hipError_t hipGetLastError() { return hipSuccess; }
+hipError_t hipGetLastError() {
+  const hipError_t e = g_last;
+  g_last = hipSuccess;
+  return e;
+}
 hipError_t hipEventCreate(hipEvent_t *e) { return take((void **)e, 8); }
 hipError_t hipEventCreateWithFlags(hipEvent_t *e, unsigned) { return hipEventCreate(e); }
 hipError_t hipEventDestroy(hipEvent_t e) { return hipFree(e); }
@@ -142,11 +146,9 @@ hipError_t hipStreamDestroy(hipStream_t s) { return hipFree(s); }
 hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) {
-  g_capturing = true;
   return hipSuccess;
 }
 hipError_t hipStreamEndCapture(hipStream_t, hipGraph_t *g) {
-  g_capturing = false;
   return take((void **)g, 8);
 }
 hipError_t hipGraphInstantiate(hipGraphExec_t *e, hipGraph_t, hipGraphNode_t *, char *, size_t) {
