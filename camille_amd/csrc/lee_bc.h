@@ -49,7 +49,8 @@ __device__ __forceinline__ double bc_neumann_value(const BcArgs &a, int c, int l
 // and the centerline conditions.  Arithmetic in FP64 for both precisions.
 // Face point q of the face box (i fastest), block point p; get(v, s) is the
 // value of variable v at s points inward (s = 0: the face point; clamped to
-// the face point where that leaves the block).
+// the face point where that leaves the block).  Only s < a.sb is asked for:
+// the points that bc_reach counts.
 template <typename T, int NS, typename Get>
 __device__ __forceinline__ void bc_face_data(const BcArgs &a, int q, int p, int c, int len, const double *met,
                                              const double *jac, Get get, double (&data)[NV]) {
@@ -70,7 +71,7 @@ __device__ __forceinline__ void bc_face_data(const BcArgs &a, int q, int p, int 
 #pragma unroll
     for (int s = 1; s <= NS; s++)
 #pragma unroll
-      for (int v = 0; v < NV; v++) nb[v][s - 1] = get(v, s);
+      for (int v = 0; v < NV; v++) nb[v][s - 1] = get(v, s < a.sb ? s : 0);
     for (int v = 0; v < NV; v++) {
       if (a.type == LEE_BC_WALL_SLIP_KINEMATIC && v >= IUX && v <= IUZ) continue;
       data[v] = bc_neumann_value<T, NS>(a, c, len, nb[v]);

@@ -59,7 +59,7 @@ __device__ __forceinline__ void bc_face_point(T *__restrict__ y, const double *_
     if (bc_is_neumann(a)) {
       T nbz[8];
 #pragma unroll
-      for (int s = 1; s <= 8; s++) nbz[s - 1] = y[vo + at(s)];
+      for (int s = 1; s <= 8; s++) nbz[s - 1] = y[vo + at(s < a.sb ? s : 0)];
       d = bc_neumann_value<T, 8>(a, c, len, nbz);
     }
     set(&y[vo + p], d);

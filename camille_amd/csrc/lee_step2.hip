@@ -83,8 +83,7 @@ __device__ __forceinline__ void faces_lds(T (&s)[4][NR][RS], const PairScalars<T
           a, q, j * a.ni + i, c, len, ps.met, ps.jac,
           [&](int v, int d) -> T {
             if (v == IUZ) return (T)0;  // blocks that carry w' run one stage a launch
-            // entries past the row's own (masked by the sum) repeat the face point
-            const int o = d < a.sb && c + sg * d >= 0 && c + sg * d < len ? sg * d : 0;
+            const int o = c + sg * d >= 0 && c + sg * d < len ? sg * d : 0;
             return s[v == IP ? 3 : v][j - gj0 + (a.dir == 1 ? o : 0)][i - gi0 + (a.dir == 0 ? o : 0)];
           },
           data);

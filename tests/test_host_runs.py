@@ -131,3 +131,14 @@ b.solve(2)
 b.solve(60)
 b.close()
 """)
+
+
+def test_boundary_faces_read_within_their_reach(tmp_path):
+    """What a face's conditions read lies in bc_reach, by which faces and
+    early receivers share the boundary launch."""
+    exe, root = str(tmp_path / "bc_reads"), os.path.dirname(HERE)
+    subprocess.run(["g++", "-std=c++17", "-O1", "-w", "-fpermissive", "-D__HIP_PLATFORM_AMD__", "-I/opt/rocm/include",
+                    "-I" + os.path.join(root, "include"), "-I" + os.path.join(root, "camille_amd", "csrc"),
+                    os.path.join(HERE, "bc_reads.cpp"), "-o", exe], check=True)
+    p = subprocess.run([exe], capture_output=True, text=True, timeout=60)
+    assert p.returncode == 0, p.stdout
