@@ -301,7 +301,8 @@ int enqueue_batch_step(lee_handle *h) {
 // sums are formed; up to nuse those whose stencils read a receiver; up to
 // nearly the others; then those whose stencils read what a face writes,
 // summed after that.  No order (the two-phase form runs) for tables that
-// name a point twice or none of their block's.
+// name a point twice or none of their block's, or that leave too much to the
+// launch's last workgroup.
 int plan_overset(lee_handle *h, const std::vector<double> &coef5) {
   Overset &o = h->ov;
   enum { FACE = 1, REACH = 2, READ = 4, RECV = 8 };
@@ -331,6 +332,7 @@ int plan_overset(lee_handle *h, const std::vector<double> &coef5) {
     const bool held = (mark[o.h_rb[r]][o.h_rl[r]] & (REACH | READ)) != 0;
     order[seen & FACE ? 3 : held ? 0 : seen & RECV ? 1 : 2].push_back(r);
   }
+  if (!boundary_in_one_launch(nvars(h), (int)order[0].size(), (int)order[3].size())) return LEE_OK;
   o.nheld = (int)order[0].size();
   o.nuse = o.nheld + (int)order[1].size();
   o.nearly = o.nuse + (int)order[2].size();

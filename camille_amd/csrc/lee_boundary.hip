@@ -333,6 +333,16 @@ __device__ __forceinline__ void ov_rho(const BndArgs<T> &a, int b, int p, double
 // spread over as many CUs as there are.
 constexpr int OV_T = 128;
 
+// What one workgroup may be left with: the receivers it writes at the end, in
+// passes of OV_T.  A pass costs it 1 to 2 us (a float run that refreshes rho':
+// 7.9 us for the launch with 2 held receivers, 10.3 with 256, 14.3 with 512,
+// 21.7 with 1024, 52 with 3072), where the launches per face, gather and
+// scatter take 12 to 18 whatever the receivers' kind.  The sums it forms first
+// cost 2.5 to 3.5 us for one pass and as much for the next (14.1 us with 51
+// receivers that read face points, 15.8 with 60, 363 with 4000; 12 to 18 us in
+// launches of their own), so they have to fit one.
+constexpr int OV_LAST_PASSES = 3;
+
 template <typename T>
 __global__ void __launch_bounds__(OV_T) k_boundary(BndArgs<T> a) {
   __shared__ double sums[OV_T];
@@ -414,6 +424,10 @@ inline unsigned nblocks(size_t n) { return (unsigned)((n + TPB - 1) / TPB); }
 }  // namespace
 
 // ------------------------------------------------------------- launchers
+
+bool boundary_in_one_launch(int nv, int nheld, int nlate) {
+  return nlate * nv <= OV_T && nheld + nlate <= OV_LAST_PASSES * OV_T;
+}
 
 hipError_t apply_bcs(hipStream_t s, lee_handle *h, const Block &b, double *y64, float *y32, bool fp32,
                      double *rho64, float *rho32, double he) {

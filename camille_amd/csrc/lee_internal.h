@@ -322,6 +322,9 @@ double harmonic_entropy(const lee_config &c, double t);
 double harmonic_gaussian(const lee_config &c, double x, double y, double z);
 hipError_t apply_bcs(hipStream_t s, lee_handle *h, const Block &b, double *y64, float *y32, bool fp32,
                      double *rho64, float *rho32, double he = 0.0);
+// Whether the boundary phase of an overset run pays as one launch: nheld
+// receivers held back and nlate that read face points, nv variables.
+bool boundary_in_one_launch(int nv, int nheld, int nlate);
 hipError_t boundary_phase(hipStream_t s, lee_handle *h, bool fp32, int buf_index, bool with_rho, double he);
 // Overset interpolation of caller-owned FP64 block arrays ys[b] (device,
 // 5n each), receiver values staged in buf (nrecv * NV doubles, device).

@@ -142,3 +142,32 @@ def test_boundary_faces_read_within_their_reach(tmp_path):
                     os.path.join(HERE, "bc_reads.cpp"), "-o", exe], check=True)
     p = subprocess.run([exe], capture_output=True, text=True, timeout=60)
     assert p.returncode == 0, p.stdout
+
+
+OVERSET = """
+sys.path.insert(0, sys.argv[2] + "/tests")
+from boundary_tables import DIMS, WALL, tables
+
+def phase(*kinds, **kw):
+    blocks = [block(*d) for d in DIMS]
+    s = Solver(blocks, overset=tables(*kinds, **kw), mode="FIX_DT", value=0.01, boundaries=[WALL])
+    host.host_forget()
+    s.update_boundary([np.zeros((5,) + b["x"].shape) for b in blocks])
+    s.close()
+    names = [n for n in launches() if "k_b" in n or "k_ov" in n]
+    assert names and any("k_boundary" in n for n in names) != any("k_ov_scatter" in n for n in names), names
+    return any("k_boundary" in n for n in names)
+"""
+
+
+def test_boundary_phase_is_one_launch_where_its_tail_is_short(runtime):
+    """One launch for few held receivers and few that read what faces write;
+    with more, one workgroup would work through them, pass by pass (41 times
+    the time of the separate launches for 16000 receivers along a wall)."""
+    runtime(OVERSET + """
+assert phase(0, 0, 1) and phase(2, 0, 5000) and phase(150, 12, 3000) and phase(384 - 25, 25, 10)
+assert phase(20, 10, 200, 30, 8)
+assert not phase(385, 0, 10) and not phase(3000, 0, 0)
+assert not phase(0, 26, 1000) and not phase(0, 4000, 0)
+assert not phase(2, 2, 100, twice=True) and not phase(20, 10, 200, 30, 8, twice=True)
+""")

@@ -3,6 +3,7 @@ rules: against plain formulas, the CPU oracle, or the form they replace."""
 import numpy as np
 import pytest
 
+import boundary_tables
 from camille_amd import FP32, FP64, PATH_PLAIN, Solver
 from test_zz_no_alloc import _noalloc
 
@@ -209,3 +210,41 @@ def test_boundary_phase_in_one_launch(nrecv, faces, twice):
         for got, ref in zip(ys, want):
             assert np.all(np.isfinite(got)) and np.array_equal(got, ref)
     s.close()
+
+
+@pytest.mark.parametrize("shear", [False, True])
+@pytest.mark.parametrize("prec", [FP64, FP32])
+@pytest.mark.parametrize("nscalar", [0, 2])
+def test_boundary_phase_forms_agree_over_a_run(shear, prec, nscalar):
+    """Steps of an overset run whose boundary phase is one launch against the
+    same run with a receiver named twice, which takes a launch per face, gather
+    and scatter (test_host_runs pins both for these tables), bit for bit: with
+    the aux density refreshed (sheared mean), in both precisions and with
+    scalars, of which fewer receivers fit a workgroup."""
+    rng = np.random.default_rng(5)
+    blocks, ics = [], []
+    for ni, nj in boundary_tables.DIMS:
+        i, j = np.meshgrid(np.arange(ni), np.arange(nj))
+        x, y = i + 0.1 * np.sin(0.5 * j), j + 0.1 * np.sin(0.4 * i)
+        mean = np.zeros((5 + nscalar, nj, ni))
+        mean[1], mean[4] = 0.2, 1.0 / GAMMA
+        if shear:
+            mean[1] = 0.2 * np.tanh(0.1 * (y - y.mean()))
+            mean[4] = (1.0 + 0.05 * np.sin(0.1 * x)) / GAMMA
+        for z in range(nscalar):
+            mean[5 + z] = 0.1 * np.cos(0.05 * x + z)
+        ic = 1e-3 * rng.standard_normal(mean.shape)
+        ic[3] = 0.0
+        blocks.append(dict(x=x, y=y, mean=mean))
+        ics.append(ic)
+    out = []
+    for twice in (False, True):
+        s = Solver(blocks, overset=boundary_tables.tables(20, 10, 200, 30, 8, twice=twice), precision=prec,
+                   boundaries=[boundary_tables.WALL], mode="FIX_DT", value=0.05, num_scalar=nscalar)
+        for ib, ic in enumerate(ics):
+            s.set_solution(ic, ib)
+        s.solve(6)
+        out.append([s.solution(ib) for ib in range(2)])
+        s.close()
+    for a, b in zip(*out):
+        assert np.all(np.isfinite(a)) and np.array_equal(a, b)
