@@ -51,15 +51,16 @@ __device__ __forceinline__ T fd_wt(int code, int d) {
   }
 }
 
-// Transposed FD row where every neighbour's row is interior: D^T = -D there.
+// Transposed FD row where every neighbour's row is interior: D^T = -D there
+// (fusions as in row_t5_sum).
 template <typename T>
 __device__ __forceinline__ T fd_row_t_inner(const T *f, int st) {
+#pragma clang fp contract(off)
   const T c1 = (T)(8.0 / 12.0), c2 = (T)(-1.0 / 12.0);
   T acc = c2 * f[-2 * st];
-  acc += c1 * f[-st];
-  acc += -c1 * f[st];
-  acc += -c2 * f[2 * st];
-  return acc;
+  acc = fmx(c1, f[-st], acc);
+  acc = fmx(-c1, f[st], acc);
+  return fmx(-c2, f[2 * st], acc);
 }
 
 // Transposed FD row at block point p (coordinate c of a line of length

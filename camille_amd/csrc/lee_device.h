@@ -156,7 +156,10 @@ __device__ __forceinline__ T row4_sum(const Row4<T> &r, const T *s, int st) {
 // Weights of the transposed OA4 rows at coordinate c of a line of length len
 // without holes: (D^T f)_c = sum_o w[o + 2] f_{c+o}, 0 for neighbours off the
 // line.  Formed once per lane and line, so that tiles at a block's edge run
-// the sums of its inside.
+// the sums of its inside.  The smallest product is the one that is rounded,
+// the others are fused onto it: left to the compiler, the first fusion took the
+// small product instead, and the float gradients of 112 x 96 x 80 runs were 4 %
+// (state) and 12 % (source) further from their values in 64 bits.
 template <typename T>
 struct RowT5 {
   T w[5];
@@ -178,12 +181,12 @@ __device__ __forceinline__ RowT5<T> row_t5(int c, int len) {
 }
 template <typename T>
 __device__ __forceinline__ T row_t5_sum(const RowT5<T> &r, const T *f, int st) {
+#pragma clang fp contract(off)
   T acc = r.w[0] * f[-2 * st];
-  acc += r.w[1] * f[-st];
-  acc += r.w[2] * f[0];
-  acc += r.w[3] * f[st];
-  acc += r.w[4] * f[2 * st];
-  return acc;
+  acc = fmx(r.w[1], f[-st], acc);
+  acc = fmx(r.w[2], f[0], acc);
+  acc = fmx(r.w[3], f[st], acc);
+  return fmx(r.w[4], f[2 * st], acc);
 }
 
 // Weight of the filter row with code `code` on offset d (rows are centred
@@ -241,10 +244,11 @@ __device__ __forceinline__ FltRowT<T, ORDER> flt_row_t(int c, int len) {
 }
 template <typename T, int ORDER>
 __device__ __forceinline__ T flt_row_t_sum(const FltRowT<T, ORDER> &r, const T *f, int st) {
+#pragma clang fp contract(off)
   constexpr int H = ORDER / 2;
   T acc = r.w[0] * f[-H * st];
 #pragma unroll
-  for (int o = 1 - H; o <= H; o++) acc += r.w[o + H] * f[o * st];
+  for (int o = 1 - H; o <= H; o++) acc = fmx(r.w[o + H], f[o * st], acc);
   return acc;
 }
 
