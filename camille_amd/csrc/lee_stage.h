@@ -8,24 +8,14 @@ namespace lee {
 
 namespace {
 
-// Mean-flow coefficient fields of block point p (MC_* order; the radius only
-// in axisymmetric runs, rho gi / p and rho not where the carried density
-// stands in for them).
-template <typename T, bool STALE, typename AT>
-__device__ __forceinline__ void stage_mean(const AT &a, int p, int n, T (&mc)[MC_COUNT]) {
-#pragma unroll
-  for (int f = 0; f < MC_COUNT; f++)
-    mc[f] = f == MC_R || (STALE && (f == MC_RP || f == MC_RB)) ? (T)0 : a.mc[f * n + p];
-  if (a.axi) mc[MC_R] = a.mc[MC_R * n + p];
-}
-
 // Chain rule and LEE right-hand side of a point from its values yc and
 // index-space derivatives dx, dy (s', u', v', p'), its FP64 metrics m and J
-// and, for a non-uniform mean, its coefficients mc (STALE: with the carried
-// aux density instead of that of yc).  Every fusion is written out (fmx), so
-// all callers round alike.
-template <typename T, bool MEANF, bool STALE, typename AT>
-__device__ __forceinline__ void stage_terms(const AT &a, const double (&m)[4], double J, const T *mc, T stale_rho,
+// and, for a non-uniform mean, its coefficients mc(f), f an MC_* index (STALE:
+// with the carried aux density rho() instead of that of yc).  They are asked
+// for after the chain rule, where a caller may read them from memory (see
+// stage_rhs).  Every fusion is written out (fmx), so all callers round alike.
+template <typename T, bool MEANF, bool STALE, typename AT, typename Mean, typename Rho>
+__device__ __forceinline__ void stage_terms(const AT &a, const double (&m)[4], double J, Mean mc, Rho stale_rho,
                                             const T (&yc)[4], const T (&dx)[4], const T (&dy)[4], T (&r)[4]) {
 #pragma clang fp contract(off)
   // chain rule with FP64 metrics (spatial:1810-1820)
@@ -62,10 +52,10 @@ __device__ __forceinline__ void stage_terms(const AT &a, const double (&m)[4], d
   } else {
     // per-point mean coefficients (MC_* order): u, v, gamma p, 1/rho,
     // the eight mean gradients, rho gi / p and rho (all at the point)
-    const T u0 = mc[MC_U], v0 = mc[MC_V], gp = mc[MC_GP], irb = mc[MC_IRB];
-    const T gsx = mc[MC_GSX], gsy = mc[MC_GSY], gux = mc[MC_GUX], guy = mc[MC_GUY];
-    const T gvx = mc[MC_GVX], gvy = mc[MC_GVY], gpx = mc[MC_GPX], gpy = mc[MC_GPY];
-    const T rho = STALE ? stale_rho : fmx(pv, mc[MC_RP], -(sv * mc[MC_RB]));
+    const T u0 = mc(MC_U), v0 = mc(MC_V), gp = mc(MC_GP), irb = mc(MC_IRB);
+    const T gsx = mc(MC_GSX), gsy = mc(MC_GSY), gux = mc(MC_GUX), guy = mc(MC_GUY);
+    const T gvx = mc(MC_GVX), gvy = mc(MC_GVY), gpx = mc(MC_GPX), gpy = mc(MC_GPY);
+    const T rho = STALE ? stale_rho() : fmx(pv, mc(MC_RP), -(sv * mc(MC_RB)));
     const T g = (T)a.gamma;
     const T ru_fac = rho * irb;
     const T uf = fmx(ru_fac, u0, uv), vf = fmx(ru_fac, v0, vv), gpv = g * pv;
@@ -92,7 +82,7 @@ __device__ __forceinline__ void stage_terms(const AT &a, const double (&m)[4], d
     rp = fmx(-gp, fy[2], rp);
     rp = fmx(-gpv, gvy, rp);
     // axisymmetry (spatial:2119-2126): -gamma (pbar v' + p' vbar) / (r + 1e-99)
-    if (a.axi) rp -= fmx(gp, vv, g * v0 * pv) / mc[MC_R];
+    if (a.axi) rp -= fmx(gp, vv, g * v0 * pv) / mc(MC_R);
   }
   r[0] = rs;
   r[1] = ru;
@@ -117,9 +107,11 @@ __device__ __forceinline__ void stage_rhs(const AT &a, double s1, double s2, dou
                                           const double (&m)[4], double J, const T (&yc)[4], const T (&dx)[4],
                                           const T (&dy)[4], T (&r)[4]) {
 #pragma clang fp contract(off)
-  T mc[MC_COUNT];
-  if (MEANF) stage_mean<T, STALE>(a, p, n, mc);
-  stage_terms<T, MEANF, STALE>(a, m, J, mc, MEANF && STALE ? a.rho_in[p] : (T)0, yc, dx, dy, r);
+  // the mean coefficients straight from memory: gathered before the chain rule
+  // they take the middle 11-point stage in FP64 from 152 to 238 registers, and
+  // 11-point steps were 5 to 11 % slower (1025 x 769 FP64 249 -> 275 us)
+  stage_terms<T, MEANF, STALE>(a, m, J, [&](int f) { return a.mc[f * n + p]; }, [&]() { return a.rho_in[p]; }, yc, dx, dy,
+                               r);
   // physical source (source.cpp:22-107), pressure equation
   if (gi >= a.si0 && gi <= a.si1 && gj >= a.sj0 && gj <= a.sj1) {
     const double gval = a.g[(gj - a.sj0) * (a.si1 - a.si0 + 1) + (gi - a.si0)];

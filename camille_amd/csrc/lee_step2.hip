@@ -273,7 +273,8 @@ __device__ __forceinline__ void pair_tile_k(const AT &a, const PairScalars<T> &p
         dy[v] = row4_sum<T>(ry, sp, RS);
       }
     }
-    stage_terms<T, MEANF, stale.value>(a, m[k], J[k], mck, rho0[k], yc, dx, dy, r);
+    stage_terms<T, MEANF, stale.value>(a, m[k], J[k], [&](int f) { return mck[f]; }, [&]() { return rho0[k]; }, yc, dx,
+                                       dy, r);
     if (sourced && gi >= a.si0 && gi <= a.si1 && gj >= a.sj0 && gj <= a.sj1) {
       const double gval = a.g[(gj - a.sj0) * (a.si1 - a.si0 + 1) + (gi - a.si0)];
       r[3] += (T)(ps.s[st].s1 * gval * ps.s[st].s2);
