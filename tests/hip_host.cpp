@@ -19,7 +19,7 @@ struct Launch {
 std::map<const void *, std::string> g_kernels;
 std::vector<Launch> g_launches;
 std::map<void *, size_t> g_live;
-long g_mallocs = 0, g_fail_at = 0;
+long g_mallocs = 0, g_fail_at = 0, g_pointer_queries = 0, g_busy = 0;
 float g_elapsed = 1e6f;
 hipError_t g_last = hipSuccess;
 char g_symbol[1 << 20];
@@ -40,6 +40,8 @@ void host_fail_malloc(long nth) {  // the nth allocation from now on fails; 0: n
   g_mallocs = 0;
   g_fail_at = nth;
 }
+long host_pointer_queries() { return g_pointer_queries; }
+void host_busy(long n) { g_busy = n; }  // the stream is at work for the next n queries
 long host_live() { return (long)g_live.size(); }
 void host_forget() { g_launches.clear(); }
 long host_launches() { return (long)g_launches.size(); }
@@ -121,6 +123,7 @@ hipError_t hipOccupancyMaxActiveBlocksPerMultiprocessor(int *n, const void *, in
   return hipSuccess;
 }
 hipError_t hipPointerGetAttributes(hipPointerAttribute_t *a, const void *) {
+  g_pointer_queries++;
   std::memset(a, 0, sizeof(*a));
   a->type = hipMemoryTypeUnregistered;
   return hipSuccess;
@@ -143,7 +146,11 @@ hipError_t hipEventElapsedTime(float *ms, hipEvent_t, hipEvent_t) {
 }
 hipError_t hipStreamCreate(hipStream_t *s) { return take((void **)s, 8); }
 hipError_t hipStreamDestroy(hipStream_t s) { return hipFree(s); }
-hipError_t hipStreamQuery(hipStream_t) { return hipSuccess; }
+hipError_t hipStreamQuery(hipStream_t) {
+  if (g_busy <= 0) return hipSuccess;
+  g_busy--;
+  return g_last = hipErrorNotReady;
+}
 hipError_t hipStreamSynchronize(hipStream_t) { return hipSuccess; }
 hipError_t hipStreamBeginCapture(hipStream_t, hipStreamCaptureMode) {
   return hipSuccess;

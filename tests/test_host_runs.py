@@ -17,6 +17,8 @@ host = ctypes.CDLL(sys.argv[1], mode=ctypes.RTLD_GLOBAL)
 host.host_launch_name.restype = ctypes.c_char_p
 host.host_launch_ptr.restype = ctypes.c_void_p
 host.host_mallocs.restype = host.host_live.restype = host.host_launches.restype = ctypes.c_long
+host.host_pointer_queries.restype = ctypes.c_long
+host.host_busy.argtypes = [ctypes.c_long]
 host.host_fail_malloc.argtypes = [ctypes.c_long]
 host.host_launch_name.argtypes = [ctypes.c_long]
 host.host_launch_ptr.argtypes = [ctypes.c_long, ctypes.c_int]
@@ -170,4 +172,26 @@ assert phase(20, 10, 200, 30, 8)
 assert not phase(385, 0, 10) and not phase(3000, 0, 0)
 assert not phase(0, 26, 1000) and not phase(0, 4000, 0)
 assert not phase(2, 2, 100, twice=True) and not phase(20, 10, 200, 30, 8, twice=True)
+""")
+
+
+def test_result_pages_are_mapped_while_there_is_work_only(runtime):
+    """A fetch with nothing to wait for goes straight to the copy; beside work
+    in flight the result's pages are written as they are."""
+    runtime("""
+y = np.random.default_rng(0).standard_normal((5, 40, 70))
+y[3] = 0
+for prec in (FP64, FP32):
+    s = Solver([block(70, 40)], precision=prec, mode="FIX_DT", value=0.01)
+    s.set_solution(y)
+    before = host.host_pointer_queries()
+    out = s.solution()
+    assert host.host_pointer_queries() == before
+    host.host_busy(2)  # ends while the pages are mapped
+    out = s.solution()
+    assert host.host_pointer_queries() == before + 1
+    if prec == FP64:
+        assert np.array_equal(out, y)
+    s.solve(1)  # the stream's "not ready" is no failure of what follows
+    s.close()
 """)
