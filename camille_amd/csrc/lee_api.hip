@@ -1799,6 +1799,36 @@ int lee_set_tile_shape(lee_handle *h, int ib, int stage_rows, int filter_rows) {
   return LEE_OK;
 }
 
+int lee_set_stage_pairs(lee_handle *h, int ib, int rows) {
+  if (!h || ib < 0 || ib >= h->nblk) return fail(h, LEE_EINVAL, "bad argument");
+  if (rows < 0 || rows > 2) return fail(h, LEE_EINVAL, "paired stages take 1 or 2 rows per wave, 0 turns them off");
+  for (int k = 0; k < h->nblk && rows; k++)
+    if ((h->batch || k == ib) && !paired_stages_ok(h, h->b[k]))
+      return fail(h, LEE_EINVAL,
+                  "two RK stages a launch: 2-D blocks of the fused path with the 4th-order scheme and four stages, "
+                  "without holes, receivers, scalars or w', at most 4 faces (none in a batch) and 4 sponges, no three of which "
+                  "meet");
+  if (h->batch) {  // one launch covers every solve
+    HIPCHK(hipStreamSynchronize(h->stream));
+    h->bp.pair = rows;
+    if (rows) h->bp.grid_stage = 0;  // a stage grid launches one stage at a time
+    h->bp.tuned = true;
+    batch_release(h);
+    return LEE_OK;
+  }
+  h->b[ib].tune_pair = rows;
+  h->b[ib].tuned = true;
+  return LEE_OK;
+}
+
+int lee_get_stage_pairs(lee_handle *h, int ib, int *rows) {
+  if (!h || ib < 0 || ib >= h->nblk || !rows) return fail(h, LEE_EINVAL, "bad argument");
+  const Block &b = h->b[ib];
+  if (h->batch) *rows = h->bp.grid_stage == 0 ? h->bp.pair : 0;
+  else *rows = b.tune_pair > 0 && paired_stages_ok(h, b) ? b.tune_pair : 0;
+  return LEE_OK;
+}
+
 int lee_set_filter_grid(lee_handle *h, int ib, int workgroups) {
   if (!h || ib < 0 || ib >= h->nblk || workgroups < 0) return fail(h, LEE_EINVAL, "bad argument");
   if (h->batch) return fail(h, LEE_EINVAL, "a batch launches its filter through the batch launch settings");

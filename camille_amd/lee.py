@@ -112,6 +112,7 @@ EXPORTS = [
     "lee_set_source_field", "lee_set_observer", "lee_objective_forward", "lee_objective_backward",
     "lee_get_source_gradient", "lee_get_state_gradient", "lee_compute_rhs_adjoint", "lee_apply_filter_adjoint",
     "lee_sample_observers", "lee_update_boundary_noalloc", "lee_update_boundary_adjoint",
+    "lee_set_stage_pairs", "lee_get_stage_pairs",
 ]
 
 _lib = None
@@ -158,6 +159,8 @@ def library():
     L.lee_autotune.argtypes = [vp]
     L.lee_set_tile_shape.argtypes = [vp, i, i, i]
     L.lee_get_tile_shape.argtypes = [vp, i, ip, ip]
+    L.lee_set_stage_pairs.argtypes = [vp, i, i]
+    L.lee_get_stage_pairs.argtypes = [vp, i, ip]
     L.lee_set_filter_grid.argtypes = [vp, i, i]
     L.lee_get_filter_grid.argtypes = [vp, i, ip]
     L.lee_set_filter_march.argtypes = [vp, i, i, i]
@@ -445,6 +448,15 @@ class Solver:
 
     def set_tile_shape(self, stage_rows, filter_rows, ib=0):
         self._check(self.L.lee_set_tile_shape(self.h, ib, int(stage_rows), int(filter_rows)))
+
+    def set_stage_pairs(self, rows, ib=0):
+        """Two RK stages a launch with 1 or 2 rows per wave; 0: one stage."""
+        self._check(self.L.lee_set_stage_pairs(self.h, ib, int(rows)))
+
+    def stage_pairs(self, ib=0):
+        r = ctypes.c_int()
+        self._check(self.L.lee_get_stage_pairs(self.h, ib, ctypes.byref(r)))
+        return r.value
 
     def set_filter_grid(self, workgroups, ib=0):
         """0: one filter workgroup per tile; >0: that many persistent

@@ -243,6 +243,17 @@ int lee_get_kernel_timing(lee_handle *h, double *ms, int *count);
 int lee_autotune(lee_handle *h);
 int lee_set_tile_shape(lee_handle *h, int iblock, int stage_rows, int filter_rows);
 int lee_get_tile_shape(lee_handle *h, int iblock, int *stage_rows, int *filter_rows);
+/* Two RK stages a launch (no reference counterpart): rows per wave, 1 or 2;
+ * 0 launches one stage at a time.  2-D blocks of the fused path with the
+ * 4th-order scheme and four stages, without holes, receivers, scalars or w',
+ * with at most 4 faces (none in a batch) and 4 sponges, no three of which meet,
+ * can run so; 1 and 2 are refused for others.  A handle of several blocks pairs its stages where all
+ * of them do; in a batch the setting is that of every solve and takes the
+ * stage grid back to 0.  Pins the form until lee_autotune; bit-identical
+ * results in every form.  The getter gives the form in use, so that a pinned
+ * tile shape can be followed by the form that was chosen before. */
+int lee_set_stage_pairs(lee_handle *h, int iblock, int rows);
+int lee_get_stage_pairs(lee_handle *h, int iblock, int *rows);
 /* Launch form of the fused filter (no reference counterpart): workgroups 0
  * launches one workgroup per tile; a positive count (rounded up to a
  * multiple of 8) launches that many persistent workgroups, each loading its

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 import boundary_tables
-from camille_amd import FP32, FP64, PATH_PLAIN, Solver
+from camille_amd import FP32, FP64, PATH_PLAIN, Batch, LeeError, Solver
 from test_zz_no_alloc import _noalloc
 
 pytestmark = pytest.mark.gpu
@@ -164,6 +164,83 @@ def test_paired_stages_bit_identical(shape, kind, prec):
         s.close()
     assert np.all(np.isfinite(out[0][0]))
     assert np.array_equal(out[0][0], out[1][0]) and out[0][1] == out[1][1]
+
+
+def _launched(s, steps):
+    """Stage launches of `steps` steps: (first, middle, last class)."""
+    s.set_kernel_timing(True)
+    s.solve(steps)
+    n = {k: v[1] for k, v in s.kernel_timing().items()}
+    s.set_kernel_timing(False)
+    return tuple(n["stage_" + k] for k in ("first", "mid", "last"))
+
+
+@pytest.mark.parametrize("shape", [(61, 13), (60, 12), (59, 25), (9, 9), (9, 12), (9, 131), (181, 121)])
+@pytest.mark.parametrize("kind", ["sponges", "sheared", "faces", "wave"])
+@pytest.mark.parametrize("prec", [FP64, FP32])
+def test_both_paired_forms_bit_identical(shape, kind, prec):
+    """Two RK stages a launch, with tiles of one and of two rows per wave,
+    against one stage a launch, bit for bit after 5 steps; the launches of
+    every run are counted."""
+    block, ic, kw = _pair_case(*shape, kind, seed=11)
+    s = Solver([block], precision=prec, **kw)
+    if shape == (9, 9) and kind in ("sponges", "sheared"):  # its three sponges meet
+        with pytest.raises(LeeError, match="no three"):
+            s.set_stage_pairs(1)
+        return
+    out = []
+    for rows in (0, 1, 2):
+        s.set_stage_pairs(rows)
+        assert s.stage_pairs() == rows
+        s.set_solution(ic)
+        s.set_time(0, 0.0, 1e-6)
+        assert _launched(s, 5) == ((5, 10, 5) if rows == 0 else (5, 0, 5))
+        out.append((s.solution(), s.clock()))
+    s.set_tile_shape(*s.tile_shape())
+    assert s.stage_pairs() == 0
+    s.close()
+    assert np.all(np.isfinite(out[0][0]))
+    for o in out[1:]:
+        assert np.array_equal(o[0], out[0][0]) and o[1] == out[0][1]
+
+
+@pytest.mark.parametrize("kind", ["sponges", "sheared"])
+@pytest.mark.parametrize("prec", [FP64, FP32])
+def test_both_paired_forms_of_a_batch(kind, prec):
+    """The same for a batch of uneven solves, against one stage a launch."""
+    cases = [_pair_case(*shape, kind, seed=3 + k) for k, shape in
+             enumerate([(61, 13), (9, 12), (120, 24), (59, 131), (181, 121)])]
+    b = Batch([dict(block, **{k: v for k, v in kw.items() if k != "harmonic"}) for block, _, kw in cases], precision=prec)
+    out = []
+    for rows in (0, 1, 2):
+        b.set_tile_shape(1, 4)
+        b.set_stage_pairs(rows)
+        assert b.stage_pairs() == rows
+        for k, (_, ic, _) in enumerate(cases):
+            b.set_solution(ic, k)
+        b.set_time(0, 0.0, 1e-6)
+        b.solve(3)  # replays of the captured step
+        assert _launched(b, 2) == ((2, 4, 2) if rows == 0 else (2, 0, 2))
+        out.append([b.solution(k) for k in range(len(cases))])
+    b.close()
+    for o in out[1:]:
+        assert all(np.all(np.isfinite(q)) and np.array_equal(p, q) for p, q in zip(o, out[0]))
+
+
+def test_stage_pairs_are_refused_where_they_cannot_run():
+    block, _, kw = _pair_case(61, 33, "sponges", seed=1)
+    for bad in (dict(kw, rk=2), dict(kw, fd_order=11), dict(kw, path=PATH_PLAIN),
+                dict(kw, boundaries=[(0, "sponge_freund_ambient", "+xi", "0", "4", str(5 * q), str(5 * q + 3), "0", "0")
+                                     for q in range(5)])):
+        s = Solver([block], precision=FP64, **bad)
+        for rows in (1, 2):
+            with pytest.raises(LeeError, match="two RK stages"):
+                s.set_stage_pairs(rows)
+        s.set_stage_pairs(0)
+        assert s.stage_pairs() == 0
+        with pytest.raises(LeeError, match="1 or 2 rows"):
+            s.set_stage_pairs(3)
+        s.close()
 
 
 _FACES = {
