@@ -27,7 +27,7 @@ __device__ __forceinline__ bool bc_is_neumann(const BcArgs &a) {
 // bc_neumann (boundary_condition.cpp:348-444): the face value whose closure
 // row vanishes, from the values nb[s - 1] at s points inward; c is the face
 // coordinate on a line of length len.  NS: the most entries past the first
-// that a row of the operator has (2 for OA4, 8 for FDO11P).
+// that a row of the operator has (2 for OA4 alone, 8 with FDO11P).
 template <typename T, int NS>
 __device__ __forceinline__ double bc_neumann_value(const BcArgs &a, int c, int len, const T (&nb)[NS]) {
 #pragma clang fp contract(off)
@@ -36,7 +36,7 @@ __device__ __forceinline__ double bc_neumann_value(const BcArgs &a, int c, int l
 #pragma unroll
   for (int s = 1; s <= NS; s++) {
     const int cs = c + sg * s;
-    const bool use = s < a.sb && cs >= 0 && cs < len;
+    const bool use = (NS == 2 || s < a.sb) && cs >= 0 && cs < len;
     const double t1 = a.end == 0 ? d - a.neu[s] * (double)nb[s - 1] : d + a.neu[s] * (double)nb[s - 1];
     d = use ? t1 : d;
   }
@@ -71,7 +71,7 @@ __device__ __forceinline__ void bc_face_data(const BcArgs &a, int q, int p, int 
 #pragma unroll
     for (int s = 1; s <= NS; s++)
 #pragma unroll
-      for (int v = 0; v < NV; v++) nb[v][s - 1] = get(v, s < a.sb ? s : 0);
+      for (int v = 0; v < NV; v++) nb[v][s - 1] = get(v, NS == 2 || s < a.sb ? s : 0);
     for (int v = 0; v < NV; v++) {
       if (a.type == LEE_BC_WALL_SLIP_KINEMATIC && v >= IUX && v <= IUZ) continue;
       data[v] = bc_neumann_value<T, NS>(a, c, len, nb[v]);

@@ -125,23 +125,24 @@ __device__ __forceinline__ T fd_row(const T *s, int st, int code) {
 }
 
 // An OA4 row as four products in fd_row's order: the neighbours' offsets and
-// their weights, the last one or two 0 (on a neighbour already in the sum) in
-// a closure row.  A lane near an end of its line runs the same instructions as
-// its neighbours instead of a branch per row kind, each waiting for LDS: the
-// rows of a tile on the block's edge took 5800 cycles, this way ROW_CYC.
+// their weights, the last one or two 0 in a closure row, on the neighbour
+// `none`, which has to hold a 0 (an infinite one would make a NaN of the sum;
+// leaving the products out instead cost a 1025 x 1025 run 2.4 %).  A lane near
+// an end of its line runs the same instructions as its neighbours instead of a
+// branch per row kind, each waiting for LDS.
 template <typename T>
 struct Row4 {
   int o[4];
   T w[4];
 };
 template <typename T>
-__device__ __forceinline__ Row4<T> row4(int code) {
+__device__ __forceinline__ Row4<T> row4(int code, int none) {
   const T c1 = (T)(8.0 / 12.0), c2 = (T)(-1.0 / 12.0);
   Row4<T> r{{-2, -1, 1, 2}, {-c2, -c1, c1, c2}};
-  if (code == CODE_LEFT + 0) r = {{0, 1, 2, 2}, {(T)-1.5, (T)2.0, (T)-0.5, (T)0}};
-  if (code == CODE_LEFT + 1) r = {{-1, 1, 1, 1}, {(T)-0.5, (T)0.5, (T)0, (T)0}};
-  if (code == CODE_LEFT + 2) r = {{0, -1, -2, -2}, {(T)1.5, (T)-2.0, (T)0.5, (T)0}};
-  if (code == CODE_LEFT + 3) r = {{1, -1, -1, -1}, {(T)0.5, (T)-0.5, (T)0, (T)0}};
+  if (code == CODE_LEFT + 0) r = {{0, 1, 2, none}, {(T)-1.5, (T)2.0, (T)-0.5, (T)0}};
+  if (code == CODE_LEFT + 1) r = {{-1, 1, none, none}, {(T)-0.5, (T)0.5, (T)0, (T)0}};
+  if (code == CODE_LEFT + 2) r = {{0, -1, -2, none}, {(T)1.5, (T)-2.0, (T)0.5, (T)0}};
+  if (code == CODE_LEFT + 3) r = {{1, -1, none, none}, {(T)0.5, (T)-0.5, (T)0, (T)0}};
   return r;
 }
 template <typename T>
@@ -171,7 +172,7 @@ __device__ __forceinline__ RowT5<T> row_t5(int c, int len) {
   for (int o = -2; o <= 2; o++) {
     const int j = c + o;
     // the row at j puts weight row4 of its code on offset -o
-    const Row4<T> q = row4<T>(default_code(j, len, 2));
+    const Row4<T> q = row4<T>(default_code(j, len, 2), 9);
     T w = (T)0;
 #pragma unroll
     for (int e = 0; e < 4; e++) w += q.o[e] == -o ? q.w[e] : (T)0;

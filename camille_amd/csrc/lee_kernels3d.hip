@@ -153,7 +153,7 @@ struct Stage3Args {
 template <typename T, bool MEANF, int KIND>
 __global__ void __launch_bounds__(TPB, sizeof(T) == 8 ? 2 : 3) k_stage3d(Stage3Args<T> a) {
   constexpr int RS = S3_TX + 2 * ST_H, NR = S3_TY + 2 * ST_H;
-  __shared__ T s[5][NR][RS];
+  __shared__ T s[5][NR + 1][RS];  // and a row of zeros (Row4)
   // within each z chunk, XCD x (workgroups x mod 8 of a grid row that is a
   // multiple of 8 wide) takes the x-th band of tiles, so that the halo a
   // tile reads of its neighbours is mostly in the same XCD's L2
@@ -168,7 +168,8 @@ __global__ void __launch_bounds__(TPB, sizeof(T) == 8 ? 2 : 3) k_stage3d(Stage3A
   const int gi = i0 + tx, gj = j0 + ty;
   const bool own = gi < ni && gj < nj;
   const size_t col = own ? (size_t)gj * ni + gi : 0;
-  const Row4<T> rx = row4<T>(default_code(gi, ni, 2)), ry = row4<T>(default_code(gj, nj, 2));
+  const int zeros = NR - ST_H - ty;  // rows down to them
+  const Row4<T> rx = row4<T>(default_code(gi, ni, 2), zeros * RS), ry = row4<T>(default_code(gj, nj, 2), zeros);
   const unsigned zmask = zones_meeting3(a.z, a.nz, i0, i0 + S3_TX - 1, j0, j0 + S3_TY - 1, k0, k1 - 1);
   // register window of the own column: planes k - 2 .. k + 2
   T w[5][5];
@@ -187,6 +188,9 @@ __global__ void __launch_bounds__(TPB, sizeof(T) == 8 ? 2 : 3) k_stage3d(Stage3A
   const int hc = tid < 128 ? tx + ST_H : (hq < 2 ? hq : hq + S3_TX);                // and column
   const bool hok = tid < 160 && j0 - ST_H + hr >= 0 && j0 - ST_H + hr < nj && i0 - ST_H + hc >= 0 && i0 - ST_H + hc < ni;
   const size_t hp = hok ? (size_t)(j0 - ST_H + hr) * ni + (i0 - ST_H + hc) : 0;
+  if (tid < RS)
+#pragma unroll
+    for (int v = 0; v < 5; v++) s[v][NR][tid] = (T)0;
   for (int k = k0; k < k1; k++) {
     // every global operand of plane k is requested before the barrier, so
     // one memory latency per plane is exposed instead of three

@@ -113,8 +113,9 @@ __device__ __forceinline__ void st_off(U *base, unsigned off, U v) {
   *(U *)((char *)base + off) = v;
 }
 
+// The input tile with its halo of 4, and a row of zeros (Row4).
 template <typename T, int RA>
-using PairLds = T[4][P2_WAVES * RA + 4][68];
+using PairLds = T[4][P2_WAVES * RA + 5][68];
 
 // Stages A and B of a pair on a tile of 60 x (4 RA - 4) points.  Lane l of
 // wave w holds block column 60 tile_x - 2 + l and the RA rows from
@@ -136,7 +137,7 @@ __device__ __forceinline__ void pair_tile_k(const AT &a, const PairScalars<T> &p
   const int i0 = tx0 * 60 - 4, j0 = ty0 * TYO - 4;  // block point of LDS (0, 0)
   const int gi = i0 + 2 + lane;
   const bool col = INNER || (gi >= 0 && gi < ni);
-  const Row4<T> rx = row4<T>(INNER ? CODE_INTERIOR : default_code(gi, ni, 2));
+  const Row4<T> rx = row4<T>(INNER ? CODE_INTERIOR : default_code(gi, ni, 2), 0);
   auto row_of = [&](int k) { return w * RA + k + 2; };  // LDS row
   auto in_block = [&](int k) {
     const int gj = j0 + row_of(k);
@@ -243,6 +244,8 @@ __device__ __forceinline__ void pair_tile_k(const AT &a, const PairScalars<T> &p
     c[MC_R] = a.axi ? ld_off(a.mc + MC_R * n + r, oT) : (T)0;
   };
   if (MEANF) mean_of(std::integral_constant<bool, FIRST>{}, 0, mc[0]);
+  if constexpr (!INNER)  // the zeros
+    for (int q = w * 64 + lane; q < 4 * RS; q += 64 * NW) s[q / RS][NR + 4][q % RS] = (T)0;
 #pragma unroll
   for (int k = 0; k <= RA; k++)
 #pragma unroll
@@ -265,11 +268,15 @@ __device__ __forceinline__ void pair_tile_k(const AT &a, const PairScalars<T> &p
         dy[v] = fd_row<T>(sp, RS, CODE_INTERIOR);
       }
     } else {
-      const Row4<T> ry = row4<T>(default_code(gj, nj, 2));  // uniform
+      const int zeros = NR + 4 - row;  // rows down to them
+      const Row4<T> ry = row4<T>(default_code(gj, nj, 2), zeros);  // uniform
+      Row4<T> rk = rx;
+#pragma unroll
+      for (int e = 2; e < 4; e++) rk.o[e] = rx.w[e] == (T)0 ? zeros * RS : rx.o[e];
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         const T *sp = &s[v][row][lane + 2];
-        dx[v] = row4_sum<T>(rx, sp, 1);
+        dx[v] = row4_sum<T>(rk, sp, 1);
         dy[v] = row4_sum<T>(ry, sp, RS);
       }
     }
@@ -368,13 +375,16 @@ __device__ __forceinline__ void pair_tile(const AT &a, const PairScalars<T> &ps,
 // 117 us against 67).
 constexpr int pair_waves(bool meanf, int ra) { return meanf ? (ra == 2 ? 2 : 3) : 4; }
 
-template <typename T, bool MEANF, bool FIRST, int RA>
+// FACES: the block has faces.  Instances without them keep 30 to 100 scalar
+// registers fewer in vector lanes: 1025 x 1025 FP32 / FP64 61.1 / 87.3 us a step
+// -> 59.0 / 86.0, 701 x 467 FP32 sheared, without walls, 39.1 -> 37.4.
+template <typename T, bool MEANF, bool FIRST, int RA, bool FACES>
 __global__ void __launch_bounds__(64 * P2_WAVES, pair_waves(MEANF, RA)) k_fused_pair(StageArgs<T> a,
                                                                                      PairScalars<T> ps) {
   __shared__ PairLds<T, RA> s;
   const int tile = xcd_tile(blockIdx.x, a.chunk);
   if (tile >= a.ntiles) return;
-  pair_tile<T, MEANF, FIRST, RA, true>(a, ps, tile, s);
+  pair_tile<T, MEANF, FIRST, RA, FACES>(a, ps, tile, s);
 }
 
 // The same for a batched ensemble: one workgroup per (solve, tile) entry of
@@ -433,10 +443,12 @@ hipError_t fused_pair_t(hipStream_t s, lee_handle *h, Block &b, int first, const
   ps.jac = b.jac;
   const dim3 grid(a.chunk * 8), block(64, P2_WAVES);
   const bool mf = !b.uniform_mean;
-#define LEE_P2(MF, FF)                                                                                \
-  do {                                                                                                \
-    if (RA == 1) hipLaunchKernelGGL((k_fused_pair<T, MF, FF, 1>), grid, block, 0, s, a, ps);          \
-    else hipLaunchKernelGGL((k_fused_pair<T, MF, FF, 2>), grid, block, 0, s, a, ps);                  \
+#define LEE_P2(MF, FF)                                                                                           \
+  do {                                                                                                           \
+    if (RA == 1 && ps.nf == 0) hipLaunchKernelGGL((k_fused_pair<T, MF, FF, 1, false>), grid, block, 0, s, a, ps); \
+    else if (RA == 1) hipLaunchKernelGGL((k_fused_pair<T, MF, FF, 1, true>), grid, block, 0, s, a, ps);          \
+    else if (ps.nf == 0) hipLaunchKernelGGL((k_fused_pair<T, MF, FF, 2, false>), grid, block, 0, s, a, ps);      \
+    else hipLaunchKernelGGL((k_fused_pair<T, MF, FF, 2, true>), grid, block, 0, s, a, ps);                       \
   } while (0)
   if (mf && F) LEE_P2(true, true);
   else if (mf) LEE_P2(true, false);

@@ -375,3 +375,49 @@ def test_transposed_rows_round_their_smallest_product(dims):
     for v in [0, 1, 2, 4] + ([3] if d3 else []):
         off = np.mean(got[v][inner] != lam[v][inner].astype(np.float64))
         assert off <= 1e-3, (v, off)
+
+
+@pytest.mark.parametrize("prec", [FP64, FP32])
+@pytest.mark.parametrize("end", [0, 1])
+def test_closure_rows_keep_infinities(prec, end):
+    """An infinite value two points from a face, which the first two closure
+    rows read once, gives the infinities and NaNs that the rows' definition
+    gives: two RK stages a launch as one a launch, and the 3-D right-hand side
+    as its formula from the derivative entry point."""
+    ni, nj = 90, 41
+    i, j = np.meshgrid(np.arange(ni), np.arange(nj))
+    mean = np.zeros((5, nj, ni))
+    mean[1], mean[2], mean[4] = 0.3, 0.2, 1.0 / GAMMA
+    ic = 1e-3 * np.random.default_rng(4).standard_normal((5, nj, ni))
+    ic[3] = 0.0
+    ic[4, 20, 2 if end == 0 else ni - 3] = np.inf
+    s = Solver([dict(x=0.5 * i + 0.1 * j, y=0.4 * j - 0.1 * i, mean=mean)], precision=prec, filter_order=0, mode="FIX_DT",
+               value=0.01)
+    out = []
+    for rows in (0, 1, 2):
+        s.set_stage_pairs(rows)
+        s.set_solution(ic)
+        s.solve(1)
+        out.append(s.solution())
+    s.close()
+    assert np.isinf(out[0]).any()
+    for o in out[1:]:
+        assert np.array_equal(o, out[0], equal_nan=True)
+
+    dims = (40, 19, 11)
+    k, j, i = np.meshgrid(*[np.arange(n) for n in dims[::-1]], indexing="ij")
+    xyz = dict(x=0.5 * i - 0.1 * j - 0.05 * k, y=0.5 * j - 0.1 * k - 0.1 * i, z=0.4 * k - 0.1 * i - 0.05 * j)
+    mean = np.zeros((5,) + i.shape)
+    ub = (0.3, 0.2, 0.1)
+    for d in range(3):
+        mean[1 + d] = ub[d]
+    mean[4] = 1.0 / GAMMA
+    y = 1e-3 * np.random.default_rng(5).standard_normal(mean.shape)
+    y[0, 5, 9, 2 if end == 0 else dims[0] - 3] = np.inf
+    y[0, 5, 2 if end == 0 else dims[1] - 3, 20] = np.inf
+    s = Solver([dict(mean=mean, **xyz)], precision=prec, mode="FIX_DT", value=0.01, num_dim=3)
+    ref = -sum(ub[d] * s.take_derivative_xyz(y[0], d) for d in range(3))
+    r = s.compute_rhs(y, 0.0)[0]
+    s.close()
+    assert np.isinf(ref).sum() >= 4
+    assert np.array_equal(np.isnan(r), np.isnan(ref)) and np.array_equal(np.isinf(r), np.isinf(ref))
