@@ -185,7 +185,10 @@ __device__ __forceinline__ T row_t5_sum(const RowT5<T> &r, const T *f, int st) {
 #pragma clang fp contract(off)
   T acc = r.w[0] * f[-2 * st];
   acc = fmx(r.w[1], f[-st], acc);
-  acc = fmx(r.w[2], f[0], acc);
+  // only the ends of a line weigh their own point: elsewhere it is left out,
+  // so that its infinite flux stays its neighbours'
+  const T a2 = fmx(r.w[2], f[0], acc);
+  acc = r.w[2] != (T)0 ? a2 : acc;
   acc = fmx(r.w[3], f[st], acc);
   return fmx(r.w[4], f[2 * st], acc);
 }

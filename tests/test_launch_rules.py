@@ -421,3 +421,27 @@ def test_closure_rows_keep_infinities(prec, end):
     s.close()
     assert np.isinf(ref).sum() >= 4
     assert np.array_equal(np.isnan(r), np.isnan(ref)) and np.array_equal(np.isinf(r), np.isinf(ref))
+
+
+@pytest.mark.parametrize("prec", [FP64, FP32])
+@pytest.mark.parametrize("dims,at", [((70, 40), (33, 20)), ((70, 40), (6, 9)), ((40, 19, 15), (20, 9, 7)),
+                                     ((40, 19, 15), (5, 5, 5))])
+def test_transposed_rows_leave_out_their_own_point(prec, dims, at):
+    """An infinite adjoint value inside the block reaches the neighbours whose
+    rows read it and not its own point, which no row but a line's first and
+    last reads, under a uniform mean without sponges."""
+    d3 = len(dims) == 3
+    axes = np.meshgrid(*[np.arange(n) for n in dims[::-1]], indexing="ij")[::-1]
+    xyz = dict(zip("xyz", [0.5 * axes[0] - 0.1 * axes[1], 0.4 * axes[1] + 0.1 * axes[0]]
+                   + ([0.3 * axes[2] - 0.05 * axes[0]] if d3 else [])))
+    mean = np.zeros((5,) + axes[0].shape)
+    mean[1], mean[2], mean[4] = 0.3, 0.2, 1.0 / GAMMA
+    s = Solver([dict(mean=mean, **xyz)], precision=prec, mode="FIX_DT", value=0.01, num_dim=len(dims))
+    kap = np.random.default_rng(6).standard_normal(mean.shape)
+    if not d3:
+        kap[3] = 0
+    kap[(0,) + at[::-1]] = np.inf
+    lam = s.compute_rhs_adjoint(kap)
+    s.close()
+    assert np.isfinite(lam[(0,) + at[::-1]])
+    assert np.isinf(lam[0]).sum() == 4 * len(dims) and not np.isnan(lam).any()
