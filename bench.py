@@ -592,9 +592,10 @@ def main():
     achieved = per_point * npts / (avg_ms * 1e-3)
     traffic = None
     tpath = os.path.join(ROOT, "profiles", "traffic_c2_fp32.json")
-    if os.path.exists(tpath) and not paired:  # measured on one-stage launches
+    if os.path.exists(tpath):
+        key = {"stage_first": "pair_first", "stage_last": "pair_second"}.get(dom, dom) if paired else dom
         try:
-            traffic = json.load(open(tpath)).get(dom)
+            traffic = json.load(open(tpath)).get(key)
         except Exception:
             traffic = None
 
@@ -655,7 +656,7 @@ def main():
         "tile_shape": {"stage_rows_per_thread": res["fp32"]["tiles"][0], "filter_tile_rows": res["fp32"]["tiles"][1]},
         "roofline": {"bound": "hbm", "kernel": dom, "achieved": achieved / 1e9, "peak": HBM_PEAK / 1e9,
                      "unit": "GB/s", "frac": achieved / HBM_PEAK, "traffic": traffic,
-                     "traffic_source": "profiles/traffic_c2_fp32.json (launches of one RK stage): rocprofv3 FETCH_SIZE and WRITE_SIZE of "
+                     "traffic_source": "profiles/traffic_c2_fp32.json: rocprofv3 FETCH_SIZE and WRITE_SIZE of "
                                        "this kernel in KiB per dispatch, scaled by a 256 MiB device copy "
                                        "(profiles/traffic_c2_fp32.md); not measured in this run",
                      "algorithmic_bytes_per_point": per_point, "avg_launch_ms": avg_ms,

@@ -327,8 +327,13 @@ __device__ __forceinline__ void ov_rho(const BndArgs<T> &a, int b, int p, double
 // held sums or readers of held receivers count themselves when their part is
 // done, and the one that counts last (none waits) forms the sums that read
 // face points and writes what was held.  What it reads of the others' goes
-// through put and get, complete before the count (a release fence instead
-// writes a whole L2 back per workgroup: 19 us).
+// through put and get (a release fence at agent scope instead writes a whole
+// L2 back per workgroup: 19 us).  Their order rests on the instruction set, not
+// on the memory model, to which all of it is relaxed: gfx950 stores of agent
+// scope are written through to where every XCD's loads of agent scope read, and
+// s_waitcnt 0 ends only when they have been; the barrier after it puts the
+// stores of every wave before the count, and the branch on the count puts the
+// loads behind it.
 // 128 threads: the lanes of a sum scatter over 25 rows, so the sums are
 // spread over as many CUs as there are.
 constexpr int OV_T = 128;

@@ -39,8 +39,8 @@ constexpr int STAGE_Z_CHUNK = 2;
 // In 64 bits, two workgroups a CU, the rounds of workgroups decide and the
 // window planes weigh more: middle stage with 2 planes and by z_chunk_rounds,
 // 112 x 96 x 80 81 -> 79 us (4 planes), 144 x 120 x 112 191 -> 183 (6),
-// 256 x 200 x 256 1128 -> 1051 (6).  (In 32 bits 3 to 6 planes change it by
-// -2 to 16 %.)
+// 256 x 200 x 256 1128 -> 1051 (6).  (In 32 bits 3 to 6 planes take from 2 %
+// less to 16 % more time than 2.)
 constexpr int STAGE64_Z_CHUNK = 6;
 constexpr double STAGE64_Z_START = 0.3;
 // Most planes per chunk of the single-pass filter (4 halo planes a side) and
