@@ -104,7 +104,7 @@ __device__ __forceinline__ void adj_dir3(const AdjPoint3 &q, double m0, double m
   F[IP] = (T)((U * q.kap[IP] + (m0 * q.kap[IUX] + m1 * q.kap[IUY] + m2 * q.kap[IUZ]) * q.irb) * q.J);
 }
 
-// What bounds it: the wait for its operands (four fifths of a wave's time);
+// What bounds it: the wait for its operands (three quarters of a wave's time);
 // a flux evaluation is some 75 FP64 operations.  Tiles of 32 x 8 points hold
 // their own fluxes in registers from the plane that first needs them, so a
 // point is evaluated once and its halo lanes (160 beside 256 points, one

@@ -2,26 +2,27 @@
 //
 // A stage reads its input, y_n, the accumulator and the FP64 geometry and
 // writes the accumulator and the next input; the next launch reads all of it
-// back.  Run in pairs, the stages of RK4 move 88 + 104 bytes a point in FP32
+// back.  Run in pairs, the stages of RK4 move 92 + 108 bytes a point in FP32
 // (uniform mean) instead of 92 + 124 + 124 + 92, and two launches replace
 // four; the price is the first stage of each pair on a halo of 2 points.
 // Every point takes the operations of the one-stage kernels in the same
 // order, so the results are bit-identical to theirs.
 //
 // Steps of RK4 with the 8th-order filter, one stage a launch -> paired (us):
-//   97 x 81      FP32 30.0 -> 16.1   FP64 31.8 -> 17.6   (1 row a wave)
-//   257 x 257    FP32 30.3 -> 17.1   FP64 35.5 -> 21.1   (1 row)
-//   513 x 513    FP32 40.8 -> 28.6   FP64 54.0 -> 40.1   (2 rows)
-//   1025 x 1025  FP32 90.5 -> 61.1   FP64 134  -> 90.5   (2 rows)
-//   2311 x 1507  FP32 299  -> 181    FP64 562  -> 318    (2 rows)
-//   701 x 467, sheared mean and two walls: FP32 67.3 -> 46.1, FP64 96.9 -> 67.2
+//   97 x 81      FP32 30.1 -> 15.9   FP64 31.8 -> 17.1   (1 row a wave)
+//   257 x 257    FP32 30.4 -> 17.1   FP64 35.7 -> 21.2   (1 row)
+//   513 x 513    FP32 41.3 -> 27.8   FP64 54.2 -> 39.7   (2 rows, FP64 1)
+//   1025 x 1025  FP32 89.7 -> 59.1   FP64 132  -> 85.3   (2 rows)
+//   2311 x 1507  FP32 299  -> 179    FP64 549  -> 306    (2 rows)
+//   701 x 467, sheared mean and two walls: FP32 67.0 -> 45.5, FP64 96.0 -> 67.2
 // What bounds it: at small blocks one workgroup's chain of latencies (launch,
-// operands, two stages), at large ones HBM (2311 x 1507 FP32: 192 bytes a
-// point in 157 us, 4.3 TB/s where a large copy reaches 4.9).
+// operands, two stages), at large ones HBM (2311 x 1507 FP32: 200 bytes a
+// point in 155 us, 4.5 TB/s where a large copy reaches 4.9; the counters of
+// 1025 x 1025 give 97 + 105 MB for the 97 + 113 that the data take).
 //
 // A workgroup is 8 waves of RA rows: RA = 2 costs 16 / 12 rows of the first
 // stage, RA = 1 8 / 4, but has the shortest chain.  Measured and not kept, at
-// 1025 x 1025 FP32 against 61 us: 4 waves of 3 rows 63 (2311 x 1507 the same,
+// 1025 x 1025 FP32 against 61 us then: 4 waves of 3 rows 63 (2311 x 1507 the same,
 // FP64 1.6 times slower for its registers), 16 of 1 row 74, 4 of 2 rows 68, 16
 // of 2 and 8 of 3 rows slower still.
 #include <hip/hip_runtime.h>
@@ -362,8 +363,12 @@ __device__ __forceinline__ void pair_tile(const AT &a, const PairScalars<T> &ps,
   constexpr int NR = P2_WAVES * RA;
   const int tx0 = tile % a.ntx, ty0 = tile / a.ntx;
   const int i0 = tx0 * 60 - 4, j0 = ty0 * (NR - 4) - 4;
-  if (i0 >= 0 && i0 + 68 <= a.ni && j0 >= 0 && j0 + NR + 4 <= a.nj)
-    pair_tile_k<T, MEANF, FIRST, RA, true, FACES>(a, ps, tx0, ty0, s);
+  // a tile whose input lies inside the block, and off its faces: those that
+  // touch one take the other instance, so that this one has no faces in it
+  // (701 x 467 FP32 between walls 46.5 -> 45.5 us a step)
+  constexpr int OFF = FACES ? 1 : 0;
+  if (i0 >= OFF && i0 + 68 <= a.ni - OFF && j0 >= OFF && j0 + NR + 4 <= a.nj - OFF)
+    pair_tile_k<T, MEANF, FIRST, RA, true, false>(a, ps, tx0, ty0, s);
   else
     pair_tile_k<T, MEANF, FIRST, RA, false, FACES>(a, ps, tx0, ty0, s);
 }
