@@ -114,9 +114,11 @@ __device__ __forceinline__ void st_off(U *base, unsigned off, U v) {
   *(U *)((char *)base + off) = v;
 }
 
-// The input tile with its halo of 4, and a row of zeros (Row4).
+// The input tile with its halo of 4, and a row of zeros (Row4) per row of a
+// wave: the zeros then lie as far from every one of its rows, and the rows'
+// addresses differ by constants.
 template <typename T, int RA>
-using PairLds = T[4][P2_WAVES * RA + 5][68];
+using PairLds = T[4][P2_WAVES * RA + 4 + RA][68];
 
 // Stages A and B of a pair on a tile of 60 x (4 RA - 4) points.  Lane l of
 // wave w holds block column 60 tile_x - 2 + l and the RA rows from
@@ -138,8 +140,9 @@ __device__ __forceinline__ void pair_tile_k(const AT &a, const PairScalars<T> &p
   const int i0 = tx0 * 60 - 4, j0 = ty0 * TYO - 4;  // block point of LDS (0, 0)
   const int gi = i0 + 2 + lane;
   const bool col = INNER || (gi >= 0 && gi < ni);
-  const Row4<T> rx = row4<T>(INNER ? CODE_INTERIOR : default_code(gi, ni, 2), 0);
   auto row_of = [&](int k) { return w * RA + k + 2; };  // LDS row
+  const int zeros = NR + 4 - row_of(0);                 // rows down to the zeros
+  const Row4<T> rx = row4<T>(INNER ? CODE_INTERIOR : default_code(gi, ni, 2), zeros * RS);
   auto in_block = [&](int k) {
     const int gj = j0 + row_of(k);
     return INNER || (col && gj >= 0 && gj < nj);
@@ -245,8 +248,11 @@ __device__ __forceinline__ void pair_tile_k(const AT &a, const PairScalars<T> &p
     c[MC_R] = a.axi ? ld_off(a.mc + MC_R * n + r, oT) : (T)0;
   };
   if (MEANF) mean_of(std::integral_constant<bool, FIRST>{}, 0, mc[0]);
-  if constexpr (!INNER)  // the zeros
-    for (int q = w * 64 + lane; q < 4 * RS; q += 64 * NW) s[q / RS][NR + 4][q % RS] = (T)0;
+  static_assert(P2_WAVES == 8 && RA <= 2, "a wave sets a variable's row of zeros");
+  if (!INNER && w < 4 * RA) {
+    s[w & 3][NR + 4 + (w >> 2)][lane] = (T)0;
+    if (xtra) s[w & 3][NR + 4 + (w >> 2)][64 + lane] = (T)0;
+  }
 #pragma unroll
   for (int k = 0; k <= RA; k++)
 #pragma unroll
@@ -269,15 +275,11 @@ __device__ __forceinline__ void pair_tile_k(const AT &a, const PairScalars<T> &p
         dy[v] = fd_row<T>(sp, RS, CODE_INTERIOR);
       }
     } else {
-      const int zeros = NR + 4 - row;  // rows down to them
       const Row4<T> ry = row4<T>(default_code(gj, nj, 2), zeros);  // uniform
-      Row4<T> rk = rx;
-#pragma unroll
-      for (int e = 2; e < 4; e++) rk.o[e] = rx.w[e] == (T)0 ? zeros * RS : rx.o[e];
 #pragma unroll
       for (int v = 0; v < 4; v++) {
         const T *sp = &s[v][row][lane + 2];
-        dx[v] = row4_sum<T>(rk, sp, 1);
+        dx[v] = row4_sum<T>(rx, sp, 1);
         dy[v] = row4_sum<T>(ry, sp, RS);
       }
     }
