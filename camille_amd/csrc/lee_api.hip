@@ -481,6 +481,7 @@ int batch_tune(lee_handle *h, hipEvent_t &e0, hipEvent_t &e1) {
       };
       ms = 1e30f;
       for (int trial = 0; trial < 3; trial++) {
+        HIPCHK(hold_stream(h->stream));  // as in autotune_block
         HIPCHK(hipEventRecord(e0, h->stream));
         for (int k = 0; k < 2; k++)
           if (int e = step()) return e;
@@ -788,8 +789,13 @@ int autotune_block(lee_handle *h, Block &b) {
         }
         return LEE_OK;
       };
+      // the timed launches queue up behind a pause, so that a small block's
+      // time is the device's: the host's, which is longer, is the same for every
+      // form (97 x 81 FP32: without the pause a quarter of the searches took 2
+      // rows, 20.5 us a step instead of 16)
       float ms = 1e30f;
       for (int trial = 0; trial < 4; trial++) {  // the first one untimed
+        HIPCHK(hold_stream(h->stream));
         HIPCHK(hipEventRecord(e0, h->stream));
         for (int k = 0; k < 4; k++)
           if (int rc = step()) return rc;

@@ -356,6 +356,7 @@ struct PairStep {
   double he_in = 0.0, he_mid = 0.0;
 };
 bool paired_stages_ok(const lee_handle *h, const Block &b);
+hipError_t hold_stream(hipStream_t s);  // some 100 us of nothing, behind which launches queue up
 hipError_t fused_pair(hipStream_t s, lee_handle *h, Block &b, int first, const PairStep &st);
 hipError_t batch_pair(hipStream_t s, lee_handle *h, int first);
 hipError_t batch_pair_prepare(hipStream_t s, lee_handle *h);  // called by batch_prepare

@@ -502,6 +502,18 @@ bool paired_stages_ok(const lee_handle *h, const Block &b) {
   return true;
 }
 
+// Keeps the stream at a fixed number of short sleeps, some 100 us, on one wave.
+namespace {
+__global__ void k_hold(int naps) {
+  for (int k = 0; k < naps; k++) __builtin_amdgcn_s_sleep(127);  // 127 x 64 cycles
+}
+}  // namespace
+
+hipError_t hold_stream(hipStream_t s) {
+  hipLaunchKernelGGL(k_hold, dim3(1), dim3(64), 0, s, 30);
+  return hipGetLastError();
+}
+
 hipError_t fused_pair(hipStream_t s, lee_handle *h, Block &b, int first, const PairStep &st) {
   if (h->cfg.precision == LEE_FP32) return fused_pair_t<float>(s, h, b, first, st, b.Y32, b.rho32);
   return fused_pair_t<double>(s, h, b, first, st, b.Y64, b.rho64);

@@ -227,6 +227,21 @@ def test_both_paired_forms_of_a_batch(kind, prec):
         assert all(np.all(np.isfinite(q)) and np.array_equal(p, q) for p, q in zip(o, out[0]))
 
 
+def test_paired_form_is_searched_for_on_the_device():
+    """On a small block a launch takes the host longer than the device, and the
+    paired forms as long as each other there: the search has to see that one
+    row per wave takes the device a third less than two, every time."""
+    block, ic, kw = _pair_case(97, 81, "sponges", seed=2)
+    s = Solver([block], precision=FP32, **kw)
+    s.set_solution(ic)
+    picks = []
+    for _ in range(16):
+        s.autotune()
+        picks.append(s.stage_pairs())
+    s.close()
+    assert picks == [1] * 16
+
+
 def test_stage_pairs_are_refused_where_they_cannot_run():
     block, _, kw = _pair_case(61, 33, "sponges", seed=1)
     for bad in (dict(kw, rk=2), dict(kw, fd_order=11), dict(kw, path=PATH_PLAIN),
