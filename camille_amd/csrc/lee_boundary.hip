@@ -25,8 +25,9 @@ __device__ __forceinline__ T get(const T *p) {
 }
 
 // One point of a BC face in global memory.  SHARED: other workgroups of the
-// launch read or overwrite it.
-template <typename T, bool SHARED>
+// launch read or overwrite it.  NS: as bc_neumann_value's (OA4 faces read two
+// points inward, not eight).
+template <typename T, int NS, bool SHARED>
 __device__ __forceinline__ void bc_face_point(T *__restrict__ y, const double *__restrict__ met,
                                               const double *__restrict__ jac, const int8_t *__restrict__ iblank,
                                               const BcArgs &a, T *__restrict__ rho, const double *__restrict__ mean,
@@ -49,7 +50,7 @@ __device__ __forceinline__ void bc_face_point(T *__restrict__ y, const double *_
     else *to = (T)x;
   };
   double data[NV];
-  bc_face_data<T, 8>(a, q, p, c, len, met, jac, [&](int v, int s) { return y[(size_t)v * n + at(s)]; }, data);
+  bc_face_data<T, NS>(a, q, p, c, len, met, jac, [&](int v, int s) { return y[(size_t)v * n + at(s)]; }, data);
   // passive scalars: Neumann data at Neumann, wall-slip (its non-velocity
   // variables, boundary_condition.cpp:122-136) and centerline faces; 0 at
   // dirichlet_allzero and harmonic-wave faces, whose data start at 0
@@ -57,10 +58,10 @@ __device__ __forceinline__ void bc_face_point(T *__restrict__ y, const double *_
     const size_t vo = (size_t)(NV + z) * n;
     double d = 0.0;
     if (bc_is_neumann(a)) {
-      T nbz[8];
+      T nbz[NS];
 #pragma unroll
-      for (int s = 1; s <= 8; s++) nbz[s - 1] = y[vo + at(s < a.sb ? s : 0)];
-      d = bc_neumann_value<T, 8>(a, c, len, nbz);
+      for (int s = 1; s <= NS; s++) nbz[s - 1] = y[vo + at(NS == 2 || s < a.sb ? s : 0)];
+      d = bc_neumann_value<T, NS>(a, c, len, nbz);
     }
     set(&y[vo + p], d);
   }
@@ -84,7 +85,7 @@ struct BcBatch {
   BcArgs f[BC_BATCH];
 };
 
-template <typename T>
+template <typename T, int NS>
 __global__ void __launch_bounds__(TPB) k_bc_faces(T *__restrict__ y, const double *__restrict__ met,
                                                   const double *__restrict__ jac,
                                                   const int8_t *__restrict__ iblank, BcBatch b,
@@ -95,7 +96,7 @@ __global__ void __launch_bounds__(TPB) k_bc_faces(T *__restrict__ y, const doubl
   const BcArgs &a = b.f[k];
   const int q = ((int)blockIdx.x - b.start[k]) * TPB + threadIdx.x;
   if (q >= (a.i1 - a.i0 + 1) * (a.j1 - a.j0 + 1)) return;
-  bc_face_point<T, false>(y, met, jac, iblank, a, rho, mean, rhob, gi, q);
+  bc_face_point<T, NS, false>(y, met, jac, iblank, a, rho, mean, rhob, gi, q);
 }
 
 // ---------------------------------------------------------------- overset
@@ -348,7 +349,7 @@ constexpr int OV_T = 128;
 // launches of their own), so they have to fit one.
 constexpr int OV_LAST_PASSES = 3;
 
-template <typename T>
+template <typename T, int NS>
 __global__ void __launch_bounds__(OV_T) k_boundary(BndArgs<T> a) {
   __shared__ double sums[OV_T];
   __shared__ bool last;
@@ -359,7 +360,7 @@ __global__ void __launch_bounds__(OV_T) k_boundary(BndArgs<T> a) {
     const BndFace<T> &f = a.f[k];
     const int q = ((int)blockIdx.x - a.start[k]) * OV_T + tid;
     if (q < (f.a.i1 - f.a.i0 + 1) * (f.a.j1 - f.a.j0 + 1))
-      bc_face_point<T, true>(f.y, f.met, f.jac, f.iblank, f.a, f.rho, f.mean, f.rhob, a.gi, q);
+      bc_face_point<T, NS, true>(f.y, f.met, f.jac, f.iblank, f.a, f.rho, f.mean, f.rhob, a.gi, q);
   } else {
     const int v = tid / a.rpw, lr = tid - v * a.rpw, r = ((int)blockIdx.x - nbc) * a.rpw + lr;
     const bool on = v < nv && r < a.nearly;
@@ -441,12 +442,13 @@ hipError_t apply_bcs(hipStream_t s, lee_handle *h, const Block &b, double *y64, 
   auto flush = [&]() {
     if (t.nf == 0) return;
     const dim3 grid(t.start[t.nf]);
-    if (fp32)
-      hipLaunchKernelGGL(k_bc_faces<float>, grid, dim3(TPB), 0, s, y32, b.met, b.jac, ib, t, rho32, b.mean, b.rhobar,
+    const bool oa4 = h->fd.sb == 3;
+    auto launch = [&](auto kernel, auto *y, auto *rho) {
+      hipLaunchKernelGGL(kernel, grid, dim3(TPB), 0, s, y, b.met, b.jac, ib, t, rho, b.mean, b.rhobar,
                          1.0 / h->cfg.gamma);
-    else
-      hipLaunchKernelGGL(k_bc_faces<double>, grid, dim3(TPB), 0, s, y64, b.met, b.jac, ib, t, rho64, b.mean, b.rhobar,
-                         1.0 / h->cfg.gamma);
+    };
+    if (fp32) launch(oa4 ? k_bc_faces<float, 2> : k_bc_faces<float, 8>, y32, rho32);
+    else launch(oa4 ? k_bc_faces<double, 2> : k_bc_faces<double, 8>, y64, rho64);
     t.nf = 0;
   };
   // in the order of the BC file; a face joins the launch before it unless
@@ -554,7 +556,8 @@ static hipError_t boundary_phase_t(hipStream_t s, lee_handle *h, T *const *ys, T
   a.with_rho = any_rho ? 1 : 0;
   a.gi = 1.0 / h->cfg.gamma;
   const int wg = a.start[a.nf] + std::max((o.nearly + a.rpw - 1) / a.rpw, 1);
-  hipLaunchKernelGGL(k_boundary<T>, dim3(wg), dim3(OV_T), 0, s, a);
+  if (h->fd.sb == 3) hipLaunchKernelGGL((k_boundary<T, 2>), dim3(wg), dim3(OV_T), 0, s, a);
+  else hipLaunchKernelGGL((k_boundary<T, 8>), dim3(wg), dim3(OV_T), 0, s, a);
   return hipGetLastError();
 }
 
