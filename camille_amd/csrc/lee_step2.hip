@@ -12,9 +12,9 @@
 //   97 x 81      FP32 30.1 -> 15.9   FP64 31.8 -> 17.1   (1 row a wave)
 //   257 x 257    FP32 30.4 -> 17.1   FP64 35.7 -> 21.2   (1 row)
 //   513 x 513    FP32 41.3 -> 27.8   FP64 54.2 -> 39.7   (2 rows, FP64 1)
-//   1025 x 1025  FP32 89.7 -> 59.1   FP64 132  -> 85.3   (2 rows)
+//   1025 x 1025  FP32 89.7 -> 59.1   FP64 132  -> 83.5   (2 rows)
 //   2311 x 1507  FP32 299  -> 179    FP64 549  -> 306    (2 rows)
-//   701 x 467, sheared mean and two walls: FP32 67.0 -> 45.5, FP64 96.0 -> 67.2
+//   701 x 467, sheared mean and two walls: FP32 67.0 -> 45.2, FP64 96.0 -> 67.2
 // What bounds it: at small blocks one workgroup's chain of latencies (launch,
 // operands, two stages), at large ones HBM (2311 x 1507 FP32: 200 bytes a
 // point in 155 us, 4.5 TB/s where a large copy reaches 4.9; the counters of
